@@ -179,8 +179,7 @@ extern "C" const char *mlg_error_string(int code) {
 extern "C" int mlg_init(const mlg_params *p, mlg_ctx **out) {
   if (!p || !out) return MLG_E_ARG;
   *out = nullptr;
-  // supported: even NR, NTH and NX from 2 to 4096 (powers of two take the
-  // FFT kernels, other lengths direct DFTs), the reference's chop limits
+  // supported: even NR, NTH and NX from 2 to 4096, the reference's chop limits
   // (mod_fft.f90:238-244, mod_scalar3.f90:183-190)
   if (p->nr < 4 || p->nr % 2 || p->nth < 2 || p->nx < 2) return MLG_E_ARG;
   if (2 * p->nxchop > p->nx || p->nxchop < 1 || p->ntchop < 1 || p->nrchop < 1) return MLG_E_ARG;
@@ -248,10 +247,9 @@ extern "C" int mlg_init(const mlg_params *p, mlg_ctx **out) {
     std::vector<double2> v(G.nth + 1);
     for (int j = 0; j <= G.nth; j++) v[j] = make_double2(re[j], im[j]);
     RET(upload(&d.tw_h, v));
-    std::vector<double2> v2(2 * (size_t)G.nth);
-    for (int j = 0; j < 2 * G.nth; j++) v2[j] = make_double2(re[j], im[j]);
-    RET(upload(&d.tw_h2, v2));
   }
+  if (!fft4_length(G.nx)) RET(fft_any_setup(G.nx, &c->fz));
+  if (!fft4_length(G.nth)) RET(fft_any_setup(G.nth, &c->ft));
   if (!G.hv_r.empty()) {
     std::vector<double> hv;
     hv.insert(hv.end(), G.hv_r.begin(), G.hv_r.end());
@@ -297,7 +295,7 @@ extern "C" int mlg_finalize(mlg_ctx *c) {
   c->timer.spare.clear();
   DevTables &d = c->d;
   void *ptrs[] = {d.pf, d.vdt, d.w, d.ones, d.r, d.x, d.lnx, d.at1, d.ak, d.norm, d.lognorm, d.bxm, d.bxxdx, d.bdel2h,
-                  d.tw_z, d.tw_t, d.tw_h, d.tw_h2, d.hv, d.red, d.vproj, d.cvdt, d.err,
+                  d.tw_z, d.tw_t, d.tw_h, c->fz.freq, c->ft.freq, d.hv, d.red, d.vproj, d.cvdt, d.err,
                   d.pf_sb, d.pf_eb, d.pf_sf, d.pf_ef, d.vdt_s, d.vdt_e, d.cvdt_s, d.cvdt_e};
   for (auto &f : c->fcache) (void)hipFree(f.f);
   c->fcache.clear();

@@ -7,6 +7,7 @@
 #include <unordered_set>
 #include <vector>
 
+#include "fft_plan.h"
 #include "mlegs_hip.h"
 
 namespace mlg {
@@ -35,6 +36,14 @@ void band_xm(int ni, int m, const double *ln, double *b);
 void band_xxdx(int ni, int m, const double *ln, double *b);
 void band_del2h(int ni, int m, double ell, const double *ln, double *b);
 
+// A mixed-radix transform of length n (k_fft_any.hip); n = 0: none.
+struct FftAny {
+  int n = 0, ns = 0, direct = 0;
+  int rad[FFT_MAX_STAGES] = {0};
+  int *freq = nullptr;  // device: fft_order's freq, then its pos (one allocation)
+  int *pos = nullptr;
+};
+
 // Device copies of the tables and scratch.
 struct DevTables {
   double *pf = nullptr;       // [mm][n][i]  (i fastest), npf rows
@@ -46,7 +55,6 @@ struct DevTables {
   double2 *tw_z = nullptr;    // e^{-2 pi i j / NX}, j < NX
   double2 *tw_t = nullptr;    // e^{-2 pi i j / NTH}, j < NTH
   double2 *tw_h = nullptr;    // e^{-2 pi i j / (2 NTH)}, j <= NTH
-  double2 *tw_h2 = nullptr;   // e^{-2 pi i j / (2 NTH)}, j < 2 NTH (theta DFTs of other lengths)
   double *hv = nullptr;       // [hv_r | hv_t | hv_x | hd_r | hd_t | hd_x]
   double *red = nullptr;      // reduction scratch
   double *vproj = nullptr;    // VEL2PLN projections [NRCHOPDIM]
@@ -112,6 +120,7 @@ struct mlg_ctx {
   mlg::Grid g;
   mlg::KTimer timer;
   mlg::DevTables d;
+  mlg::FftAny fz, ft;  // z and theta lengths that the four-step kernels do not take
   hipStream_t stream = nullptr;
   hipStream_t own_stream = nullptr;
   long n_fff = 0, n_pff = 0, n_ppp = 0, n_max = 0;
@@ -254,8 +263,7 @@ int etd_sponge(mlg_ctx *c, mlg_field *uz, mlg_field *b, double dt);
 // the filter tables of the context's current coefficients to the device
 int upload_hyperv(mlg_ctx *c);
 // dz, dm: bit j set = job j transforms d/dz (i k times) or d/dtheta (i m
-// times) of its input (four-step lengths, NX <= 256, only); zl[0..nzl-1]:
-// LN coefficients the launch sets to zero (nzl <= MAX_TRANSFORM_JOBS)
+// times) of its input; zl[0..nzl-1]: LN coefficients the launch sets to zero (nzl <= MAX_TRANSFORM_JOBS)
 int launch_verfft_bwd_n(mlg_ctx *c, int n, const double2 *const *in, double2 *const *out, unsigned dz = 0,
                         unsigned dm = 0, double *const *zl = nullptr, int nzl = 0);
 int launch_verfft_fwd_n(mlg_ctx *c, int n, const double2 *const *in, double2 *const *out);
@@ -287,11 +295,18 @@ int launch_horfft_bwd(mlg_ctx *c, double2 *a);
 constexpr int MAX_HOR_JOBS = 10;
 struct HorJobs {
   double2 *a[MAX_HOR_JOBS];
+  int n;
   double s0, s1;
   const double *wr;
 };
 int launch_horfft_fwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double s1);
 int launch_horfft_bwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double s1, const double *wr);
+// ---- transforms of any length (k_fft_any.hip)
+// lengths of the four-step register kernels
+static inline bool fft4_length(int n) { return n >= 2 && n <= 256 && (n & (n - 1)) == 0; }
+int fft_any_setup(int n, FftAny *f);  // allocates f's device tables
+int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd);
+int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd);
 // ---- physical-space products (k_physical.hip)
 int launch_vprod(mlg_ctx *c, const double2 *rur, const double2 *rup, const double2 *uz, double2 *ror, double2 *rop, double2 *oz);
 int launch_vdot(mlg_ctx *c, const double2 *rar, const double2 *rap, const double2 *az, const double2 *rbr,
