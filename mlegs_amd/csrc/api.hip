@@ -148,8 +148,6 @@ static int upload(T **dst, const std::vector<T> &src) {
   return 0;
 }
 
-static bool pow2(int n) { return n >= 1 && (n & (n - 1)) == 0; }
-
 extern "C" const char *mlg_error_string(int code) {
   switch (code) {
     case 0: return "ok";
@@ -802,10 +800,10 @@ static int to_pff_n(mlg_ctx *c, int n, mlg_field *const *fs, mlg_field *const *k
 
 // keep (optional, FFF velocities only): receives the FFF elements of the
 // velocities, see to_pff_n
-// fix false (non-FFF velocities only): psi's value-at-infinity fix-up is
-// left to the caller
+// inner (non-FFF velocities only): inside a right-hand side, where VEL2PLN
+// runs in one launch and psi's value-at-infinity fix-up is left to the caller
 static int project_impl(mlg_field *rur, mlg_field *rup, mlg_field *uz, mlg_field *psi, mlg_field *chi, int ln_mode, double ln,
-                        mlg_field *const *keep = nullptr, bool fix = true) {
+                        mlg_field *const *keep = nullptr, bool inner = false) {
   if (!(rur->space == rup->space && rup->space == uz->space)) return 2;
   mlg_ctx *c = rur->ctx;
   mlg_field *const vel[3] = {rur, rup, uz};
@@ -846,9 +844,15 @@ static int project_impl(mlg_field *rur, mlg_field *rup, mlg_field *uz, mlg_field
     chi->space = MLG_FFF;
     RET(launch_set_ln(c, chi->ln, nullptr, 0.0, 0.0));
   }
-  if (ln_mode) RET(launch_vel2pln(c, rup->e, psi->ln, ln_mode, ln));
+  if (ln_mode && inner) {
+    const double *vec = nullptr;
+    RET(m0_vectors(c, &vec));
+    RET(launch_vel2pln_vec(c, rup->e, psi->ln, ln_mode, ln, vec));
+  } else if (ln_mode) {
+    RET(launch_vel2pln(c, rup->e, psi->ln, ln_mode, ln));
+  }
   RET(launch_project(c, rur->e, rup->e, uz->e, psi->e, chi->e));  // CHOPDO of psi, chi included
-  return fix ? launch_fix_at_infinity(c, psi->e) : 0;
+  return inner ? 0 : launch_fix_at_infinity(c, psi->e);
 }
 
 extern "C" int mlg_project(mlg_field *rur, mlg_field *rup, mlg_field *uz, mlg_field *psi, mlg_field *chi, int has_ln, double ln) {
@@ -857,68 +861,9 @@ extern "C" int mlg_project(mlg_field *rur, mlg_field *rup, mlg_field *uz, mlg_fi
 }
 
 // ------------------------------------------------------------------ Boussinesq terms
-// FFF -> PFF -> PFP (TOFP without the theta transform, done by the fused
-// product kernel)
-static int to_pfp(mlg_field *a) {
-  if (a->space == MLG_FFF) RET(mlg_rtran(a, 1));
-  if (a->space == MLG_PFF) RET(mlg_verfft(a, 1));
-  return a->space == MLG_PFP ? 0 : 2;
-}
-
-// to_pfp of n independent FFF fields: one RTRAN backward launch and one
-// VERFFT backward launch for all of them (each field as mlg_rtran then
-// mlg_verfft treat it)
-// keep[i] (i < nkeep, optional) receives the FFF contents of fs[i] (E and LN)
-// instead of discarding them; it must be a temporary of the caller.
-static int to_pfp_n(mlg_ctx *c, int n, mlg_field *const *fs, mlg_field *const *keep = nullptr, int nkeep = 0) {
-  bool all_fff = n <= MAX_TRANSFORM_JOBS;
-  for (int i = 0; i < n; i++) all_fff = all_fff && fs[i]->space == MLG_FFF;
-  if (!all_fff) {
-    for (int i = 0; i < nkeep; i++) {  // unchopped copies
-      if (fs[i]->space != MLG_FFF) return 2;
-      RET(launch_copy(c, keep[i]->e, fs[i]->e, space_count(c, MLG_FFF)));
-      RET(launch_set_ln(c, keep[i]->ln, fs[i]->ln, 1.0, 0.0));
-      keep[i]->space = MLG_FFF;
-    }
-    for (int i = 0; i < n; i++) RET(to_pfp(fs[i]));
-    return 0;
-  }
-  Temps T(c);
-  mlg_field *t[MAX_TRANSFORM_JOBS];
-  for (int i = 0; i < n; i++) t[i] = T.buffer();
-  RET(T.ready());
-  const double2 *in[MAX_TRANSFORM_JOBS];
-  const double *ln[MAX_TRANSFORM_JOBS];
-  double2 *out[MAX_TRANSFORM_JOBS];
-  for (int i = 0; i < n; i++) {
-    in[i] = fs[i]->e;
-    ln[i] = fs[i]->ln;
-    out[i] = t[i]->e;
-  }
-  RET(launch_rtran_bwd_n(c, n, in, ln, out));  // padding rows included
-  double *lns[MAX_TRANSFORM_JOBS];
-  for (int i = 0; i < n; i++) {
-    swap_storage(fs[i], t[i]);
-    if (i < nkeep) {  // the FFF storage and its LN move to keep[i]
-      std::swap(keep[i]->e, t[i]->e);
-      std::swap(keep[i]->ln, fs[i]->ln);
-      keep[i]->space = MLG_FFF;
-    }
-    fs[i]->space = MLG_PFF;
-    lns[i] = fs[i]->ln;
-    in[i] = fs[i]->e;
-    out[i] = t[i]->e;  // the FFF storage (or keep[i]'s), free again
-  }
-  RET(launch_verfft_bwd_n(c, n, in, out, 0, 0, lns, n));  // the PFF fields' LN = 0
-  for (int i = 0; i < n; i++) {
-    swap_storage(fs[i], t[i]);
-    fs[i]->space = MLG_PFP;
-  }
-  return 0;
-}
-
-// The seven FFF fields fs to PFP (as to_pfp_n, with keep for the first
-// three), together with GRAD's i m b and i k b in PFP (rbp, bz), which come
+// The seven FFF fields fs to PFP (TOFP without the theta transform) with one
+// RTRAN backward launch and one VERFFT backward launch, the FFF storage and
+// LN of the first three moving to keep[], together with GRAD's i m b and i k b in PFP (rbp, bz), which come
 // from one backward Legendre transform of b (b stays in FFF): the
 // z-transform multiplies by i m or i k as it loads.  The same linear maps as
 // GRAD then RTRAN, VERFFT, in another order.
@@ -969,11 +914,71 @@ static int to_pfp_b(mlg_ctx *c, mlg_field *const *fs, const mlg_field *b, mlg_fi
   return 0;
 }
 
+// CALC_BOUSSI_FORCE where the products are fused with the theta transforms.
+// W = TOFP(B) at NRCHOP and GRAD's i m b and i k b at NRCHOP+3 are Legendre
+// jobs of the one batch (the z-transform multiplies by i m or i k as it
+// loads), GRAD's r d/dr b comes with PC2VEL and PC2VOR, N_b's z-transform
+// runs with PROJECT's, and psi's fix-up at infinity with chi's: eleven
+// launches, where the routines called one by one are twenty-two.  A launch
+// is about 4.4 us of a captured step whatever it does.  With the AB2 step and
+// VISC2's right-hand sides in one launch (visc_cn) a step is thirteen launches
+// instead of twenty-seven: 178 -> 115 us at 64x32x32, 225 -> 160 at 128x64x64.
+static int force_fused(const mlg_field *psi, const mlg_field *chi, const mlg_field *b, mlg_field *psin, mlg_field *chin,
+                       mlg_field *bn) {
+  mlg_ctx *c = psi->ctx;
+  if (psi->space != MLG_FFF || chi->space != MLG_FFF || b->space != MLG_FFF) return 3;
+  Temps T(c);
+  constexpr int NL = 9, NZ = 10;
+  mlg_field *f[NZ], *t[NL];  // rur rup uz ror rop oz rbr rbp bz w
+  for (auto &q : f) q = T.buffer();
+  for (auto &q : t) q = T.buffer();
+  mlg_field *w2 = T.buffer();
+  RET(T.ready());
+  VelVorOut vo;
+  for (int i = 0; i < 7; i++) vo.e[i] = f[i]->e, vo.ln[i] = f[i]->ln;
+  vo.b = b->e;
+  vo.ln_b = b->ln;
+  RET(mlg_chopset(c, 3));
+  int rc = launch_pc2velvor(c, psi->e, psi->ln, chi->e, chi->ln, vo);  // with PC2VOR's DEL2 check
+  const double2 *in[NZ];
+  const double *ln[NL];
+  double2 *out[NZ];
+  const int dn[NL] = {0, 0, 0, 0, 0, 0, 0, 0, -3};
+  for (int i = 0; i < NL; i++) {
+    in[i] = i < 7 ? f[i]->e : b->e;
+    ln[i] = i < 7 ? f[i]->ln : b->ln;
+    out[i] = t[i]->e;
+  }
+  if (!rc) rc = launch_rtran_bwd_n(c, NL, in, ln, out, dn);
+  mlg_chopset(c, -3);
+  RET(rc);
+  for (int i = 0; i < NZ; i++) {  // b's transform is read twice
+    in[i] = t[i < 8 ? i : i - 1]->e;
+    out[i] = f[i]->e;
+  }
+  RET(launch_verfft_bwd_n(c, NZ, in, out, 1u << 8, 1u << 7));
+  {
+    const double2 *pi[10];
+    for (int i = 0; i < 10; i++) pi[i] = f[i]->e;
+    double2 *po[4] = {f[3]->e, f[4]->e, f[5]->e, bn->e};
+    RET(launch_fused_products(c, pi, po, 2 * c->g.p.omega, std::pow(c->g.p.bv0, 2.0), 1, bn->ln));  // and N_b's LN = 0
+  }
+  bn->space = f[3]->space = f[4]->space = f[5]->space = MLG_PFP;
+  mlg_field *const pf4[4] = {f[3], f[4], f[5], bn};
+  RET(to_pff_n(c, 4, pf4));
+  RET(project_impl(f[3], f[4], f[5], psin, w2, 1, 0.0, nullptr, true));
+  RET(solve_op(w2, chin, 1, 0.0, 0, 0.0, false));  // IDEL2LN
+  double2 *const fix[2] = {psin->e, chin->e};
+  RET(launch_chopdo_fff_n(c, 2, fix, true));  // CHOPDO, and the fixes at infinity of PROJECT and IDEL2LN
+  return mlg_toff(bn);
+}
+
 // CALC_BOUSSI_FORCE (src/mod_boussinesq.f90:317-410)
 extern "C" int mlg_force(const mlg_field *psi, const mlg_field *chi, const mlg_field *b, mlg_field *psin, mlg_field *chin,
                          mlg_field *bn) {
   if (!psi || !chi || !b || !psin || !chin || !bn) return MLG_E_ARG;
   mlg_ctx *c = psi->ctx;
+  if (fused_products_supported(c)) return force_fused(psi, chi, b, psin, chin, bn);
   Temps T(c);
   mlg_field *rur = T.get(), *rup = T.get(), *uz = T.get(), *ror = T.get(), *rop = T.get(), *oz = T.get();
   mlg_field *rbr = T.get(), *rbp = T.get(), *bz = T.get(), *w = T.get(), *w2 = T.get();
@@ -983,29 +988,19 @@ extern "C" int mlg_force(const mlg_field *psi, const mlg_field *chi, const mlg_f
   if (!rc) rc = mlg_pc2vel(psi, chi, rur, rup, uz);
   if (!rc) rc = mlg_pc2vor(psi, chi, ror, rop, oz);
   mlg_field *fs[9] = {rur, rup, uz, ror, rop, oz, rbr, rbp, bz};
-  const bool fused = fused_products_supported(c);
-  if (!rc && fused) rc = to_pfp_n(c, 9, fs);
-  for (int i = 0; i < 9 && !rc && !fused; i++) rc = mlg_tofp(fs[i]);
+  for (int i = 0; i < 9 && !rc; i++) rc = mlg_tofp(fs[i]);
   mlg_chopset(c, -3);
   RET(rc);
   // W = TOFP(B) at NRCHOP (its value does not depend on the products, so it
   // is formed first and fed to the product kernel)
   RET(copy0(w, b));
-  if (fused) {
-    RET(to_pfp(w));
-    const double2 *in[10] = {rur->e, rup->e, uz->e, ror->e, rop->e, oz->e, rbr->e, rbp->e, bz->e, w->e};
-    double2 *out[4] = {ror->e, rop->e, oz->e, bn->e};
-    RET(launch_fused_products(c, in, out, 2 * c->g.p.omega, std::pow(c->g.p.bv0, 2.0), 1, bn->ln));  // and N_b's LN = 0
-    bn->space = ror->space = rop->space = oz->space = MLG_PFP;
-  } else {
-    RET(mlg_tofp(w));
-    bn->space = MLG_PPP;
-    RET(launch_force_products(c, rur->e, rup->e, uz->e, ror->e, rop->e, oz->e, rbr->e, rbp->e, bz->e, w->e, bn->e,
-                              2 * c->g.p.omega, std::pow(c->g.p.bv0, 2.0), 1));
-    RET(launch_set_ln(c, bn->ln, nullptr, 0.0, 0.0));
-    RET(launch_chopdo(c, bn->e, MLG_PPP));
-    ror->space = rop->space = oz->space = MLG_PPP;
-  }
+  RET(mlg_tofp(w));
+  bn->space = MLG_PPP;
+  RET(launch_force_products(c, rur->e, rup->e, uz->e, ror->e, rop->e, oz->e, rbr->e, rbp->e, bz->e, w->e, bn->e,
+                            2 * c->g.p.omega, std::pow(c->g.p.bv0, 2.0), 1));
+  RET(launch_set_ln(c, bn->ln, nullptr, 0.0, 0.0));
+  RET(launch_chopdo(c, bn->e, MLG_PPP));
+  ror->space = rop->space = oz->space = MLG_PPP;
   RET(mlg_project(ror, rop, oz, psin, w2, 1, 0.0));
   RET(mlg_idel2ln(w2, chin));
   return mlg_toff(bn);
@@ -1035,7 +1030,7 @@ static int nonlin_impl(const mlg_field *b, mlg_field *rur, mlg_field *rup, mlg_f
   mlg_field *rbr = T.buffer(), *rbp = T.buffer(), *bz = T.buffer(), *psi = T.buffer(), *chi = T.buffer(), *w = T.buffer();
   RET(T.ready());
   int rc;
-  if (fused_products_supported(c) && c->g.nx <= 256 && pow2(c->g.nx)) {
+  if (fused_products_supported(c)) {
     // GRAD's r d/dr b is formed in FFF; its i m b and i k b components come
     // from b's own transform (to_pfp_b)
     RET(mlg_chopset(c, 1));
@@ -1062,7 +1057,7 @@ static int nonlin_impl(const mlg_field *b, mlg_field *rur, mlg_field *rup, mlg_f
     // psi, and IDEL2's CHOPDO and fix-up of chi, are made there, on the
     // columns it stages
     const int nrchop0 = c->g.nrchop;
-    RET(project_impl(ror, rop, oz, psi, w, 1, 0.0, nullptr, false));
+    RET(project_impl(ror, rop, oz, psi, w, 1, 0.0, nullptr, true));
     RET(solve_op(w, chi, 0, 0.0, 0, 0.0, false));  // IDEL2
     RET(mlg_chopset(c, 3));
     rc = pc2vel_impl(psi, chi, ror, rop, oz, nrchop0);
@@ -1079,31 +1074,18 @@ static int nonlin_impl(const mlg_field *b, mlg_field *rur, mlg_field *rup, mlg_f
   mlg_chopset(c, -1);
   RET(rc);
   mlg_field *fs[9] = {rur, rup, uz, ror, rop, oz, rbr, rbp, bz};
-  if (fused_products_supported(c)) {
-    RET(to_pfp_n(c, 9, fs, vel_fff, vel_fff ? 3 : 0));
-    const double2 *in[10] = {rur->e, rup->e, uz->e, ror->e, rop->e, oz->e, rbr->e, rbp->e, bz->e, nullptr};
-    double2 *out[4] = {ror->e, rop->e, oz->e, bn->e};
-    RET(launch_fused_products(c, in, out, 0.0, 0.0, 0, bn->ln));  // and N_b's LN = 0
-    bn->space = ror->space = rop->space = oz->space = MLG_PFP;
-    if (!keep_velocity) {
-      RET(mlg_horfft(rur, 1));
-      RET(mlg_horfft(rup, 1));
-      RET(mlg_horfft(uz, 1));
+  if (vel_fff)  // unchopped copies: the velocities carry NRCHOP+3 rows
+    for (int i = 0; i < 3; i++) {
+      RET(launch_copy(c, vel_fff[i]->e, fs[i]->e, space_count(c, MLG_FFF)));
+      RET(launch_set_ln(c, vel_fff[i]->ln, fs[i]->ln, 1.0, 0.0));
+      vel_fff[i]->space = MLG_FFF;
     }
-  } else {
-    if (vel_fff)  // unchopped copies: the velocities carry NRCHOP+3 rows
-      for (int i = 0; i < 3; i++) {
-        RET(launch_copy(c, vel_fff[i]->e, fs[i]->e, space_count(c, MLG_FFF)));
-        RET(launch_set_ln(c, vel_fff[i]->ln, fs[i]->ln, 1.0, 0.0));
-        vel_fff[i]->space = MLG_FFF;
-      }
-    for (int i = 0; i < 9; i++) RET(mlg_tofp(fs[i]));
-    bn->space = MLG_PPP;
-    RET(launch_force_products(c, rur->e, rup->e, uz->e, ror->e, rop->e, oz->e, rbr->e, rbp->e, bz->e, nullptr, bn->e, 0.0,
-                              0.0, 0));
-    RET(launch_set_ln(c, bn->ln, nullptr, 0.0, 0.0));
-    RET(launch_chopdo(c, bn->e, MLG_PPP));
-  }
+  for (int i = 0; i < 9; i++) RET(mlg_tofp(fs[i]));
+  bn->space = MLG_PPP;
+  RET(launch_force_products(c, rur->e, rup->e, uz->e, ror->e, rop->e, oz->e, rbr->e, rbp->e, bz->e, nullptr, bn->e, 0.0,
+                            0.0, 0));
+  RET(launch_set_ln(c, bn->ln, nullptr, 0.0, 0.0));
+  RET(launch_chopdo(c, bn->e, MLG_PPP));
   RET(mlg_project(ror, rop, oz, psi, w, 1, 0.0));
   RET(mlg_idel2(w, chi, 0, 0.0));
   RET(mlg_chopset(c, 3));
@@ -1269,8 +1251,9 @@ static int richardson(mlg_field *y, const mlg_field *x1, bool ln) {
 
 // IHELM of n independent fields, A_i = IHELM(B_i, ALP_i), with one band-solve
 // launch for all of them (each field as solve_op does it for op 2).
-// bil: the right-hand sides b are row-interleaved (launch_visc2_rhs_il)
-static int ihelm_n(int n, mlg_field *const *b, mlg_field *const *a, const double *alp, int bil = 0) {
+// bil: the right-hand sides b are row-interleaved (launch_visc2_rhs_il);
+// chop false: the rows past the truncation of a are zero already
+static int ihelm_n(int n, mlg_field *const *b, mlg_field *const *a, const double *alp, int bil = 0, bool chop = true) {
   mlg_ctx *c = b[0]->ctx;
   const double2 *be[3];
   double2 *ae[3];
@@ -1292,7 +1275,7 @@ static int ihelm_n(int n, mlg_field *const *b, mlg_field *const *a, const double
   double2 *te[3] = {nullptr, nullptr, nullptr};
   for (int i = 0; i < n; i++) te[i] = tf[i]->e;
   RET(launch_band_solve_n(c, 2, n, be, ae, aln, bln, alp, 0, 0.0, te, bil));
-  return launch_chopdo_fff_n(c, n, ae, false);
+  return chop ? launch_chopdo_fff_n(c, n, ae, false) : 0;
 }
 
 // VISC1 (mod_march.f90:1529-1576): backward Euler diffusion; the right-hand
@@ -1326,7 +1309,11 @@ static int visc_be(mlg_ctx *c, mlg_field *psi, mlg_field *chi, mlg_field *b, dou
 // VISC2 on (psi, chi, b): the current values are read from fa[] (which may
 // be the outputs f[] themselves), the previous ones from fo[]; all three
 // right-hand sides are formed before the batched solves write f[].
-static int visc_cn(mlg_ctx *c, mlg_field *const *f, const mlg_field *const *fa, const mlg_field *const *fo) {
+// With x, h (the AB2 march): the current values are the AB2 step of fo[]
+// with N = x[] and the history h[], formed with the right-hand sides; h[]
+// takes N (launch_visc2_rhs_il); fo[] are the outputs.
+static int visc_cn(mlg_ctx *c, mlg_field *const *f, const mlg_field *const *fa, const mlg_field *const *fo,
+                   mlg_field *const *x = nullptr, mlg_field *const *h = nullptr) {
   if (c->g.p.visc_sw != 1) return 0;
   Temps T(c);
   mlg_field *wk[3] = {T.buffer(), T.buffer(), T.buffer()};  // the right-hand-side kernel writes E and LN
@@ -1344,12 +1331,19 @@ static int visc_cn(mlg_ctx *c, mlg_field *const *f, const mlg_field *const *fa, 
     alp[i] = 2 / nu[i] / c->g.p.dt;
     wk[i]->space = MLG_FFF;
     jobs.j[i] = Visc2Job{fo[i]->e, fo[i]->ln, fa[i]->e, fa[i]->ln, alp[i], wk[i]->e, wk[i]->ln};
+    if (x) {
+      Visc2Job &J = jobs.j[i];
+      J.x = x[i]->e, J.ln_x = x[i]->ln, J.h = h[i]->e, J.ln_h = h[i]->ln, J.y = f[i]->e;
+      J.ab2_ln = i < 2;
+      h[i]->space = MLG_FFF;
+    }
   }
+  jobs.dt = c->g.p.dt;
   // WK row-interleaved for the one-thread-per-system solve, in columns for the partitioned one
   const int il = band_lanes(kgrid(c)) == 0;
   RET(launch_visc2_rhs_il(c, n, jobs, il));
   mlg_field *out[3] = {f[0], f[1], f[2]};
-  return ihelm_n(n, wk, out, alp, il);
+  return ihelm_n(n, wk, out, alp, il, x == nullptr);  // with x the outputs are chopped with the right-hand sides
 }
 static int visc_cn(mlg_ctx *c, mlg_field *psi, mlg_field *chi, mlg_field *b, const mlg_field *psio, const mlg_field *chio,
                    const mlg_field *bo) {
@@ -1431,14 +1425,23 @@ static int step_ab_cn(mlg_solver *s, mlg_field *psi, mlg_field *chi, mlg_field *
   s->t += dt;
   s->n += 1;
   Temps T(c);
-  mlg_field *psin = T.get(), *chin = T.get(), *bn = T.get(), *psi0 = T.get(), *chi0 = T.get(), *b0 = T.get();
+  // no LN is cleared: the right-hand side writes those of psin, chin and bn
+  mlg_field *psin = T.buffer(), *chin = T.buffer(), *bn = T.buffer();
   RET(T.ready());
   RET(mlg_force(psi, chi, b, psin, chin, bn));
-  // PSI0 = PSI ; AB2 ; N history = the new N, for the three fields in one launch
-  mlg_field *y[3] = {psi, chi, b}, *y0[3] = {psi0, chi0, b0}, *h[3] = {s->n_psi, s->n_chi, s->n_b};
-  const mlg_field *x[3] = {psin, chin, bn};
+  mlg_field *y[3] = {psi, chi, b}, *h[3] = {s->n_psi, s->n_chi, s->n_b}, *x[3] = {psin, chin, bn};
   bool fff = true;
   for (int i = 0; i < 3; i++) fff = fff && y[i]->space == MLG_FFF && x[i]->space == MLG_FFF;
+  if (fff && c->g.p.visc_sw == 1 && c->g.p.kappa != 0.0 && band_lanes(kgrid(c)) != 0) {
+    // the AB2 step, the history copies and VISC2's right-hand sides of the
+    // three fields in one launch (right-hand sides in columns)
+    RET(visc_cn(c, y, y, y, x, h));
+    return hyperv_state(c, psi, chi, b, dt);
+  }
+  // PSI0 = PSI ; AB2 ; N history = the new N, for the three fields in one launch
+  mlg_field *psi0 = T.buffer(), *chi0 = T.buffer(), *b0 = T.buffer();
+  RET(T.ready());
+  mlg_field *y0[3] = {psi0, chi0, b0};
   if (fff) {
     Ab2Jobs jobs;
     for (int i = 0; i < 3; i++) {

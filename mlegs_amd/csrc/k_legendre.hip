@@ -244,7 +244,7 @@ __device__ __forceinline__ void rtran_bwd_tile(const KGrid &g, const typename Le
   const double *__restrict__ ln_in = jobs.ln[fj];
   double2 *__restrict__ out = jobs.out[fj];
   const int mv = mm * g.minc;
-  const int nn = d_nrchops(g.nrchop, mv);
+  const int nn = d_nrchops(g.nrchop + jobs.dn[fj], mv);
   const int i0 = ti * TI, c0 = tc * TC;
   // the thread id through an empty asm: in the grouped kernel's tile loop
   // the compiler then keeps no thread-dependent offsets of every tile shape
@@ -472,7 +472,8 @@ k_rtran_bwd_grouped(const BwdJob *__restrict__ jb, const int *__restrict__ b0, i
   }
 }
 
-int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double *const *ln_in, double2 *const *out) {
+int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double *const *ln_in, double2 *const *out,
+                       const int *dn) {
   if (n < 1 || n > MAX_TRANSFORM_JOBS) return MLG_E_ARG;
   KGrid g = kgrid(c);
   TransformJobs jobs;
@@ -480,6 +481,7 @@ int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double
     jobs.in[i] = in[i];
     jobs.ln[i] = ln_in[i];
     jobs.out[i] = out[i];
+    jobs.dn[i] = dn ? dn[i] : 0;
   }
   // 2 NR sum_m NRCHOPS(m) NXCHOPDIM flops per field (real table x complex data, folded)
   const double per_k = n * 2.0 * g.nr * g.nxchopdim;
@@ -1421,9 +1423,10 @@ __global__ void __launch_bounds__(256) k_project_fff_m0(KGrid g, const double *_
   }
 }
 
-// The composed tables (once) and the m = 0 vectors (once per truncation: a
-// buffer per NRCHOP value, kept until the context ends, so that a captured
-// step that reads one set is never handed another truncation's vectors).
+// The composed tables (once).  m0_vectors: the m = 0 vectors, once per
+// truncation: a buffer per NRCHOP value, kept until the context ends, so that
+// a captured step that reads one set is never handed another truncation's
+// vectors.
 static int ensure_cvdt(mlg_ctx *c, const double **m0vec) {
   if (c->g.nrh < 1) return MLG_E_ARG;
   KGrid g = kgrid(c);
@@ -1443,6 +1446,11 @@ static int ensure_cvdt(mlg_ctx *c, const double **m0vec) {
                               (long)nh * nh, 1, nh, nh, SPLIT_KC);
     if (rc) return rc;
   }
+  return m0_vectors(c, m0vec);
+}
+
+int m0_vectors(mlg_ctx *c, const double **m0vec) {
+  KGrid g = kgrid(c);
   for (auto &v : c->m0vecs)
     if (v.first == g.nrchop) {
       *m0vec = v.second;

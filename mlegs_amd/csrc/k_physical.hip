@@ -162,6 +162,39 @@ __global__ void __launch_bounds__(256) k_vel2pln_apply(KGrid g, const double *__
   if (threadIdx.x == 0 && ln_mode != 2) psi_ln[0] = ln_mode == 1 ? ln : pln;
 }
 
+// VEL2PLN in one block, with the Gauss sums and the sum over n folded into
+// one vector over the nodes beforehand (vec: G_e, G_o of k_m0_gauss, per
+// truncation): LN = -(sum_i (p + q) G_e + (p - q) G_o) / 2, then pass 2's
+// removal.  Two launches became one inside the steps (9 us each way at any
+// size: they are launches, not work).
+__global__ void __launch_bounds__(256) k_vel2pln_vec(KGrid g, const double *__restrict__ pf, const double *__restrict__ vec,
+                                                     double2 *__restrict__ rup, double *__restrict__ psi_ln, int ln_mode,
+                                                     double ln) {
+  __shared__ double part[4];
+  const double *ge = vec + 4 * (size_t)g.nrchopdim, *go = ge + g.nrh;
+  double v = 0.0;
+  for (int i = threadIdx.x; i < g.nrh; i += 256) {
+    const double p = rup[i].x, q = rup[g.nr - 1 - i].x;
+    v += (p + q) * ge[i] + (p - q) * go[i];
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  const double pln = -(((part[0] + part[1]) + part[2]) + part[3]) / 2.0;
+  for (int i = threadIdx.x; i < g.nrh; i += 256) {
+    const double e = -pf[i] * pln / g.norm0, o = -pf[(size_t)g.nrh + i] * pln / g.norm1;
+    rup[i].x = rup[i].x - (e + o);
+    rup[g.nr - 1 - i].x = rup[g.nr - 1 - i].x - (e - o);
+  }
+  if (threadIdx.x == 0 && ln_mode != 2) psi_ln[0] = ln_mode == 1 ? ln : pln;
+}
+int launch_vel2pln_vec(mlg_ctx *c, double2 *rup, double *psi_ln, int ln_mode, double ln, const double *vec) {
+  hipLaunchKernelGGL(k_vel2pln_vec, dim3(1), dim3(256), 0, c->stream, kgrid(c), c->d.pf, vec, rup, psi_ln, ln_mode, ln);
+  MLG_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+
 static int vel2pln_passes(mlg_ctx *c, double2 *rup, double *psi_ln, int ln_mode, double ln, double *proj) {
   KGrid g = kgrid(c);
   if (g.nrchop > 0)

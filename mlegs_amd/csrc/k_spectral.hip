@@ -383,8 +383,14 @@ int launch_del2(mlg_ctx *c, const double2 *a, const double *ln_a, double2 *b, do
 
 // WK%LN = -ALP*A%LN, and DEL2's top-mode check of AO at NRCHOP+2
 // (one thread of each job)
-__device__ __forceinline__ void visc2_ln_check(const KGrid &g, int nrchop2, const Visc2Job &J, double alp, int *err) {
-  J.ln_wk[0] = J.ln_a[0] * -alp + 0.0;
+__device__ __forceinline__ void visc2_ln_check(const KGrid &g, int nrchop2, const Visc2Job &J, double alp, double dt, int *err) {
+  double ln_a = J.x ? J.ln_ao[0] : J.ln_a[0];
+  if (J.x) {  // the AB2 step of LN (k_ab2_hist)
+    const double xl = J.ln_x[0];
+    if (J.ab2_ln) ln_a = ln_a + dt * (1.5 * xl - 0.5 * J.ln_h[0]);
+    J.ln_h[0] = xl * 1.0 + 0.0;
+  }
+  J.ln_wk[0] = ln_a * -alp + 0.0;
   if (g.ntchopdim >= 2) {
     const int nt = s_nrchops(nrchop2, g.minc);
     if (nt >= 1 && g.ntchop > 1 && nt - 1 < s_nrchops(g.nrchop, g.minc)) {
@@ -509,7 +515,7 @@ __global__ void __launch_bounds__(256) k_visc2_rhs_il(KGrid g, int nrchop2, cons
       }
     }
   }
-  if (s0 == 0 && blockIdx.y == 0 && t == 0) visc2_ln_check(g, nrchop2, J, alp, err);
+  if (s0 == 0 && blockIdx.y == 0 && t == 0) visc2_ln_check(g, nrchop2, J, alp, jobs.dt, err);
 }
 
 // The same right-hand sides written in the FFF columns, the layout that the
@@ -521,7 +527,9 @@ __global__ void __launch_bounds__(256) k_visc2_rhs_il(KGrid g, int nrchop2, cons
 // one column group consecutive, so a chunk's halo rows come from the L2
 // that its neighbours filled.  Four threads per column form VR/4
 // consecutive rows each by k_visc2_rhs_il's operations; each wave writes VR
-// consecutive rows of 64 / VR columns, adding -ALP*A on the way.
+// consecutive rows of 64 / VR columns, adding -ALP*A on the way.  With J.x
+// the AB2 step is formed there as well: one launch and the traffic of two
+// fields less than k_ab2_hist before it.
 template <int VR>
 __global__ void __launch_bounds__(256) k_visc2_rhs_col(KGrid g, int nrchop2, const double *__restrict__ bd,
                                                        const double *__restrict__ ak, Visc2Jobs jobs, int nrc, int *err) {
@@ -592,10 +600,23 @@ __global__ void __launch_bounds__(256) k_visc2_rhs_col(KGrid g, int nrchop2, con
     if (cc < nk && n < g.nrchopdim) {
       const size_t o = cb0 + kstride * cc + n;
       const double2 v = sx[cc * XP + rl];
-      J.wk[o] = sub2(make_double2(-v.x, -v.y), axc(alp, J.a[o]));
+      double2 a;
+      if (J.x) {
+        // AB2 on the way (k_ab2_hist's operations): only this thread reads
+        // and writes the row of X and H, and rows past the truncation, which
+        // every AO read above takes as zero, are chopped here
+        const bool in = n < nn;
+        const double2 x = in ? J.x[o] : zero2(), h = in ? J.h[o] : zero2();
+        a = in ? add2(J.ao[o], axc(jobs.dt, sub2(axc(1.5, x), axc(0.5, h)))) : zero2();
+        J.h[o] = x;
+        if (!in) J.y[o] = zero2();
+      } else {
+        a = J.a[o];
+      }
+      J.wk[o] = sub2(make_double2(-v.x, -v.y), axc(alp, a));
     }
   }
-  if (lid == 0 && t == 0) visc2_ln_check(g, nrchop2, J, alp, err);
+  if (lid == 0 && t == 0) visc2_ln_check(g, nrchop2, J, alp, jobs.dt, err);
 }
 int launch_visc2_rhs_il(mlg_ctx *c, int n, const Visc2Jobs &jobs, int il) {
   if (n < 1 || n > 3) return MLG_E_ARG;
@@ -823,7 +844,8 @@ int launch_pc2vor(mlg_ctx *c, const double2 *psi, const double *ln_psi, const do
 // ---------------------------------------------------------------- PC2VEL + PC2VOR
 // Both of one (PSI, CHI) pair in one pass, as the time steps call them
 // (CHOPSET(3); PC2VEL; PC2VOR): one block per (m, k) column, the column of
-// psi and chi, DEL2 chi and the two MULXM(DELSQH) stages in LDS.  Every
+// psi and chi, DEL2 chi and the two MULXM(DELSQH) stages in LDS (and b's
+// column for GRAD's XXDX b, in the right-hand side of the AB2 march).  Every
 // output row is formed by the same operations as in k_pc2vel and k_pc2vor.
 __global__ void __launch_bounds__(256) k_pc2velvor(KGrid g, const double *bxm, const double *bxxdx, const double *bd,
                                                    const double *ak, const double2 *psi, const double *ln_psi,
@@ -833,7 +855,8 @@ __global__ void __launch_bounds__(256) k_pc2velvor(KGrid g, const double *bxm, c
   const int mv = mm * g.minc, nn = mm < g.ntchop ? s_nrchops(g.nrchop, mv) : 0;
   const size_t cb = fcol(g, mm, k);
   double2 *P = csm, *X = P + g.nrchopdim, *Q = X + g.nrchopdim, *WP = Q + g.nrchopdim, *WX = WP + g.nrchopdim;
-  const double lp = ln_psi[0], lc = ln_chi[0];
+  double2 *B = WX + g.nrchopdim;  // with o.b
+  const double lp = ln_psi[0], lc = ln_chi[0], lb = o.b ? o.ln_b[0] : 0.0;
   const double *bdm = bd + (size_t)mm * g.nband * 5, *xm = bxm + (size_t)mm * g.nband * 3,
                *xx = bxxdx + (size_t)mm * g.nband * 3;
   RowTables<5> T5;
@@ -845,6 +868,7 @@ __global__ void __launch_bounds__(256) k_pc2velvor(KGrid g, const double *bxm, c
   for (int n = threadIdx.x; n < nn; n += blockDim.x) {
     P[n] = psi[cb + n];
     X[n] = chi[cb + n];
+    if (o.b) B[n] = o.b[cb + n];
   }
   __syncthreads();
   // DEL2's exactness check of PC2VOR (k_check_top_m1): the top mode of
@@ -895,14 +919,23 @@ __global__ void __launch_bounds__(256) k_pc2velvor(KGrid g, const double *bxm, c
     o.e[3][cb + n] = wr;
     o.e[4][cb + n] = wp;
     o.e[5][cb + n] = wz;
+    if (o.b) {  // GRAD's XXDX b (k_grad)
+      double2 vr = zero2();
+      if (n < nn) vr = band3_r(rx, B, n, nn);
+      if (mm == 0 && k == 0) {
+        if (n == 0) vr.x = vr.x + lb / g.norm0;
+        if (n == 1) vr.x = vr.x + lb / g.norm1;
+      }
+      o.e[6][cb + n] = vr;
+    }
   };
   FOR_MY_ROWS(g.nrchopdim, TX, xx, TM, xm, out);
-  if (mm == 0 && k == 0 && threadIdx.x < 6) o.ln[threadIdx.x][0] = 0.0;
+  if (mm == 0 && k == 0 && threadIdx.x < (o.b ? 7 : 6)) o.ln[threadIdx.x][0] = 0.0;
 }
 int launch_pc2velvor(mlg_ctx *c, const double2 *psi, const double *ln_psi, const double2 *chi, const double *ln_chi,
                      const VelVorOut &o) {
   KGrid g = kgrid(c);
-  hipLaunchKernelGGL(k_pc2velvor, column_grid(g), dim3(256), 5 * sizeof(double2) * (size_t)g.nrchopdim, c->stream, g,
+  hipLaunchKernelGGL(k_pc2velvor, column_grid(g), dim3(256), (o.b ? 6 : 5) * sizeof(double2) * (size_t)g.nrchopdim, c->stream, g,
                      c->d.bxm, c->d.bxxdx, c->d.bdel2h, c->d.ak, psi, ln_psi, chi, ln_chi, o, c->d.err);
   MLG_CHECK_HIP(hipGetLastError());
   return 0;
@@ -1583,8 +1616,8 @@ __device__ __forceinline__ double2 dpp_next2(double2 v) {
   return make_double2(dpp_next<DIR>(v.x), dpp_next<DIR>(v.y));
 }
 
-// The start states of the segments, passed along the P lanes of each system
-// in turn (lanes seg + 1 after seg forward, seg - 1 after seg back): every
+// The start states of the segments, passed along the P segments of each system
+// (those that hold rows: lanes past them carry zero states either way) in turn (lanes seg + 1 after seg forward, seg - 1 after seg back): every
 // lane forms its segment's end state E = p + G s from its current start
 // state (G[u]: the end state of the run from unit state u), and at step t
 // the lane of segment t (forward) or P - 1 - t (back) takes its
@@ -1721,6 +1754,22 @@ __device__ __forceinline__ void part_passes(double2 *my, size_t fstride, int a, 
   }
 }
 
+// f(slot in LDS, element) for every row of the block's 64 / P systems, eight
+// rows a lane and all of them independent: with many short systems a block
+// (P < 16) a loop over the systems waits out one memory round trip each.
+template <class F>
+__device__ __forceinline__ void part_rows_each(const KGrid &g, int op, long sys0, int P, F f) {
+#pragma unroll
+  for (int q = 0; q < PART_LS; q++) {
+    const int row = (int)threadIdx.x + 64 * q, jp = row / (P * PART_LS), n = row - jp * P * PART_LS;
+    int m2, k2;
+    const int ndp = penta_rows(g, op, sys0 + jp, m2, k2);
+    if (n < ndp)
+      f((row / PART_LS) * (PART_LS + 1) + row % PART_LS,
+        (size_t)n + (size_t)g.nrchopdim * ((size_t)m2 + (size_t)g.ntchopdim * k2));
+  }
+}
+
 template <int NJ>
 __device__ void apply_penta_part(const KGrid &g, int op, int has_ln, const BandJobs &jobs, int grp, long sys0, int P,
                                  double2 *lds) {
@@ -1747,6 +1796,11 @@ __device__ void apply_penta_part(const KGrid &g, int op, int has_ln, const BandJ
 #pragma unroll
       for (int jj = 0; jj < NJ; jj++) lds[jj * fstride + sl] = jobs.j[jobs.gjob[grp][jj]].b[(size_t)n * nsys + sys0 + jp];
     }
+  } else if (P < 16) {
+    part_rows_each(g, op, sys0, P, [&](int sl, size_t i) {
+#pragma unroll
+      for (int jj = 0; jj < NJ; jj++) lds[jj * fstride + sl] = jobs.j[jobs.gjob[grp][jj]].b[i];
+    });
   } else {
     for (int jp = 0; jp < W; jp++) {
       int m2, k2;
@@ -1764,7 +1818,7 @@ __device__ void apply_penta_part(const KGrid &g, int op, int has_ln, const BandJ
   // LUBKSBB: row n's multipliers against rows n-1, n-2 and 1/pivot, then its
   // normalised upper entries against rows n+1, n+2
   part_passes<NJ, 2>(
-      my, fstride, seg * LS, nd, P, seg,
+      my, fstride, seg * LS, nd, (g.nrchop + LS - 1) / LS, seg,
       [&](int n, double(&c)[2], double &sc) {
         const double *ff = FV.ff + ((size_t)min(n, nlast) * ncls + cls) * 3;
         c[0] = (n >= 1 && n < nd) ? ff[0] : 0.0;
@@ -1790,6 +1844,13 @@ __device__ void apply_penta_part(const KGrid &g, int op, int has_ln, const BandJ
     }
   }
   __syncthreads();
+  if (P < 16) {
+    part_rows_each(g, op, sys0, P, [&](int sl, size_t i) {
+#pragma unroll
+      for (int jj = 0; jj < NJ; jj++) jobs.j[jobs.gjob[grp][jj]].a[i] = lds[jj * fstride + sl];
+    });
+    return;
+  }
   for (int jp = 0; jp < W; jp++) {
     int m2, k2;
     const int ndp = penta_rows(g, op, sys0 + jp, m2, k2);
@@ -1943,7 +2004,7 @@ __device__ void apply_m0_part(const KGrid &g, const double *bxm, int op, double 
   const int nlast = max(nd - 1, 0);
   auto rec = [&](int n) { return f7 + ((size_t)min(max(n, 0), nlast) * ncls + cls) * FSTRIDE; };
   part_passes<1, 3>(
-      lds + (size_t)lane * SLOT, 0, lane * LS, nd, 64, lane,
+      lds + (size_t)lane * SLOT, 0, lane * LS, nd, (nd + LS - 1) / LS, lane,
       [&](int n, double(&c)[3], double &sc) {
         const double *fr = rec(n);
 #pragma unroll
@@ -2002,12 +2063,15 @@ __global__ void __launch_bounds__(64, 3) k_band_apply_part(KGrid g, const double
 }
 
 // Lanes per penta-diagonal system of the partitioned solve: the smallest
-// power of two, at least 4, whose segments of PART_LS rows cover NRCHOP.
-// 0: one thread per system (NRCHOP below 64, where systems are short, or
-// above 64 PART_LS); that path is LUBKSBB's arithmetic, bitwise.
+// power of two, at least 2, whose segments of PART_LS rows cover NRCHOP.
+// 0: one thread per system (NRCHOP above 64 PART_LS); that path is
+// LUBKSBB's arithmetic, bitwise.  A solve (mean of IDEL2LN's and the three
+// fields' IHELM) takes 15.3 us on 8 lanes at NRCHOP 48 against 25.9 on one
+// thread per system; at 22 it takes 14.5 against 12.5, but its right-hand
+// sides in columns form the AB2 step on the way, two launches less.
 int band_lanes(const KGrid &g) {
-  if (g.nrchop < 64 || g.nrchop > 64 * PART_LS) return 0;
-  int p = 4;
+  if (g.nrchop > 64 * PART_LS) return 0;
+  int p = 2;
   while (p * PART_LS < g.nrchop) p *= 2;
   return p;
 }
@@ -2330,7 +2394,7 @@ __global__ void __launch_bounds__(64, 3) k_band_apply_t_part(KGrid g, const doub
       const int nlast = max(nd - 1, 0);
       auto rec = [&](int n) { return f7 + ((size_t)min(max(n, 0), nlast) * ncls + cls) * FSTRIDE; };
       part_passes<1, 3>(
-          xs + (size_t)lane * SLOT, 0, lane * LS, nd, 64, lane,
+          xs + (size_t)lane * SLOT, 0, lane * LS, nd, (nd + LS - 1) / LS, lane,
           [&](int n, double(&c)[3], double &sc) {
 #pragma unroll
             for (int t = 0; t < 3; t++) c[t] = (n >= t + 1 && n < nd) ? rec(n - 1 - t)[3 + t] : 0.0;
@@ -2357,19 +2421,20 @@ __global__ void __launch_bounds__(64, 3) k_band_apply_t_part(KGrid g, const doub
   if (pb < 0) return;
   const long sys0 = (long)pb * W;
   const size_t fstride = (size_t)64 * SLOT;
-  for (int jp = 0; jp < W; jp++) {
+  // eight independent rows a lane, as part_rows_each
+#pragma unroll
+  for (int q = 0; q < LS; q++) {
+    const int row = lane + 64 * q, jp = row / (P * LS), n = row - jp * P * LS;
     int m2, k2;
     const int ndp = penta_rows(g, op, sys0 + jp, m2, k2);
     const size_t colp = (size_t)R * ((size_t)m2 + (size_t)g.ntchopdim * k2);
-    const bool fix = op == 1 && m2 == 0 && ndp > 0;
-    const double2 a0 = fix ? J.in[colp] : zero2();
-    for (int n = lane; n < ndp; n += 64) {
+    if (n < ndp) {
       double2 v = J.in[colp + n];
-      if (fix) {
-        v = sub2(v, axc(at1[n] / at1[0], a0));
+      if (op == 1 && m2 == 0) {
+        v = sub2(v, axc(at1[n] / at1[0], J.in[colp]));
         if (k2 == 0 && n == 0) v = make_double2(g.norm0 * J.ln_in[0], 0.0);
       }
-      xs[(jp * P + n / LS) * SLOT + n % LS] = v;
+      xs[(row / LS) * SLOT + row % LS] = v;
     }
   }
   __syncthreads();
@@ -2383,7 +2448,7 @@ __global__ void __launch_bounds__(64, 3) k_band_apply_t_part(KGrid g, const doub
     const int nlast = max(nd - 1, 0);
     auto row = [&](int n) { return (size_t)min(max(n, 0), nlast) * ncls + cls; };
     part_passes<1, 2>(
-        xs + (size_t)lane * SLOT, fstride, seg * LS, nd, P, seg,
+        xs + (size_t)lane * SLOT, fstride, seg * LS, nd, (g.nrchop + LS - 1) / LS, seg,
         [&](int n, double(&c)[2], double &sc) {
           c[0] = (n >= 1 && n < nd) ? FV.fb[row(n - 1) * 2] : 0.0;
           c[1] = (n >= 2 && n < nd) ? FV.fb[row(n - 2) * 2 + 1] : 0.0;

@@ -221,17 +221,20 @@ static inline int nrchops_of(int nrchop, int m) {
 // ---- launchers: Legendre transforms (k_legendre.hip)
 int launch_rtran_bwd(mlg_ctx *c, const double2 *in, const double *ln_in, double2 *out);
 // n (<= MAX_TRANSFORM_JOBS) independent fields in one launch
-constexpr int MAX_TRANSFORM_JOBS = 9;
+constexpr int MAX_TRANSFORM_JOBS = 10;
 struct TransformJobs {
   const double2 *in[MAX_TRANSFORM_JOBS];
   const double *ln[MAX_TRANSFORM_JOBS];
   double2 *out[MAX_TRANSFORM_JOBS];
+  int dn[MAX_TRANSFORM_JOBS] = {0};  // RTRAN backward: job j is truncated at NRCHOP + dn[j], dn[j] <= 0
   unsigned dz = 0;  // VERFFT backward: bit j set = job j transforms i k times its input (d/dz)
   unsigned dm = 0;  // VERFFT backward: bit j set = job j transforms i m times its input (d/dtheta)
   double *zl[MAX_TRANSFORM_JOBS];  // VERFFT backward: LN coefficients set to zero by the launch
   int nzl = 0;
 };
-int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double *const *ln_in, double2 *const *out);
+// dn (optional): job j's truncation NRCHOP + dn[j], dn[j] <= 0
+int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double *const *ln_in, double2 *const *out,
+                       const int *dn = nullptr);
 // Grouped backward products (k_legendre.hip): any number of jobs, each one
 // run's product over a range of its modes with its own tile shape (radial
 // nodes x real columns), in one persistent launch.  Every shape gives the
@@ -314,6 +317,12 @@ int launch_vdot(mlg_ctx *c, const double2 *rar, const double2 *rap, const double
 int launch_force_products(mlg_ctx *c, const double2 *rur, const double2 *rup, const double2 *uz, double2 *ror, double2 *rop,
                           double2 *oz, const double2 *rbr, const double2 *rbp, const double2 *bz, const double2 *bphys,
                           double2 *bn, double two_omega, double n2, int linear);
+// VEL2PLN in one launch with the folded vectors of `vec` (launch_m0_vectors),
+// for the right-hand sides inside a step
+int launch_vel2pln_vec(mlg_ctx *c, double2 *rup, double *psi_ln, int ln_mode, double ln, const double *vec);
+// the m = 0, k = 0 column's vectors at the current truncation (k_legendre.hip),
+// built once per truncation and kept by the context
+int m0_vectors(mlg_ctx *c, const double **vec);
 // ln_mode: 0 psi LN = the computed value, 1 psi LN = ln, 2 psi LN unchanged
 int launch_vel2pln(mlg_ctx *c, double2 *rup, double *psi_ln, int ln_mode, double ln);
 // the same with the projections in a fixed per-device array of at most
@@ -350,9 +359,19 @@ struct Visc2Job {
   double alp;
   double2 *wk;
   double *ln_wk;
+  // with x: the AB2 step is formed here, A = COPY0(AO) + DT (1.5 X - 0.5 H)
+  // (a is not read), H = COPY0(X), and AO is chopped in place; LN likewise,
+  // A%LN = AO%LN + DT (1.5 X%LN - 0.5 H%LN) where ab2_ln is set
+  const double2 *x = nullptr;
+  const double *ln_x = nullptr;
+  double2 *h = nullptr;
+  double *ln_h = nullptr;
+  double2 *y = nullptr;  // AO, written
+  int ab2_ln = 0;
 };
 struct Visc2Jobs {
   Visc2Job j[3];
+  double dt = 0.0;
 };
 // n (<= 3) independent right-hand sides in one launch, WK written
 // row-interleaved over the systems (row n of system s = m + NTCHOPDIM k at
@@ -389,10 +408,13 @@ struct VelTriple {
 // H on the right is read from `base` when base.e[0] is not null
 int launch_pc2vel_hist(mlg_ctx *c, const double2 *psi, const double *ln_psi, const double2 *chi, const double *ln_chi,
                        double2 *hr, double2 *hp, double2 *hz, int hmode, double ha, const VelTriple &base);
-// PC2VEL and PC2VOR of one (psi, chi): outputs rur, rup, uz, ror, rop, oz
+// PC2VEL and PC2VOR of one (psi, chi): outputs rur, rup, uz, ror, rop, oz,
+// and, with b, the r d/dr component of GRAD(b) in e[6], ln[6]
 struct VelVorOut {
-  double2 *e[6];
-  double *ln[6];
+  double2 *e[7];
+  double *ln[7];
+  const double2 *b = nullptr;
+  const double *ln_b = nullptr;
 };
 int launch_pc2velvor(mlg_ctx *c, const double2 *psi, const double *ln_psi, const double2 *chi, const double *ln_chi,
                      const VelVorOut &o);
@@ -431,7 +453,8 @@ struct BandTJob {
 };
 int launch_band_solve_t_n(mlg_ctx *c, int op, int n, const BandTJob *jobs);
 int launch_axpby(mlg_ctx *c, int mode, double2 *y, double a, const double2 *x1, const double2 *x2, const double2 *x3, long n);
-// STEP_BOUSSI_AB_CN's middle for n (<= 3) FFF fields in one launch: y0 =
+// STEP_BOUSSI_AB_CN's middle for n (<= 3) FFF fields in one launch (where
+// VISC2's right-hand side does not form it): y0 =
 // COPY0(y), y = AB2(y, x, h), h = COPY0(x), with their LN (y's AB2 only
 // where ln is set)
 struct Ab2Job {
