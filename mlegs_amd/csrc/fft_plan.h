@@ -83,4 +83,63 @@ inline void fft_order(const FftFactors &f, std::vector<int> &freq, std::vector<i
   }
 }
 
+// The fused products at a theta length n (k_fused_any.hip): the line's last
+// inverse stage has radix R = 2..6 and leaves each thread R physical points;
+// before it come middle stages of radix 2..8 and, first, a direct stage over
+// the product D of the prime factors above 7.
+struct FusedPlan {
+  int n = 0;                         // 0: not planned
+  int R = 0, D = 1, nmid = 0;        // n = D mid[0] .. mid[nmid-1] R
+  int mid[FFT_MAX_STAGES] = {0};
+  int P = 0, T = 0;                  // radial lines and threads of a block
+};
+// LDS of a block in 16-byte values: the roots, one line buffer, and a second
+// one for the direct stage
+inline long fused_lds(const FusedPlan &f) {
+  return f.n + f.n / 2 + 1 + (long)f.n * f.P * (1 + (f.D > 1));
+}
+inline bool fused_plan(int n, FusedPlan &f) {
+  f = FusedPlan{};
+  int rest = n, D = 1;
+  for (int p : {2, 3, 5, 7})
+    while (rest % p == 0) rest /= p;
+  D = rest;
+  // a direct stage reads D / 2 values for each one it forms; at NR = 192, NX =
+  // 64 the kernel takes 426 us for NTH = 122 (D = 61) where the separate
+  // transforms and products take 601; no configured length has a larger one
+  if (D > 61) return false;
+  // six or five points a thread in blocks of four waves are the fastest (FORCE
+  // kernel at NTH = 204, NR = 408, NX = 128: 1.45 ms against 1.56 with four
+  // points in eight waves; NTH = 384, NX = 64: 0.81 against 1.21).  Seven and
+  // eight (NTH = 384: 1.30 ms) are slowed by their registers, and lengths that
+  // only they would take stay with the separate kernels (NTH = 608, NR = 64,
+  // NX = 64: 750 us with eight points, 688 apart)
+  for (int R : {6, 5, 4, 3, 2}) {
+    if (n % (D * R)) continue;
+    FusedPlan c;
+    c.n = n;
+    c.R = R;
+    c.D = D;
+    std::vector<int> cur, best;
+    const int m = n / (D * R);
+    if (m > 1) {
+      fft_search(m, 8, cur, best);
+      if (best.empty()) continue;
+    }
+    c.nmid = (int)best.size();
+    if (c.nmid + 2 > FFT_MAX_STAGES) continue;
+    for (int i = 0; i < c.nmid; i++) c.mid[i] = best[i];
+    c.P = (R == 5 || R == 6 ? 256 : 512) * R / n;
+    if (c.P < 4) c.P = 512 * R / n;
+    if (c.P > 32) c.P = 32;
+    while (c.P > 0 && fused_lds(c) * 16 > 156 * 1024) c.P--;
+    if (c.P < 4) continue;  // shorter runs of r than 64 bytes
+    c.T = (n / R * c.P + 63) / 64 * 64;
+    // the line's n / 2 + 1 pairs, R / 2 + 1 a thread
+    if ((n / 2 + 1) > (R / 2 + 1) * (c.T / c.P)) continue;
+    f = c;
+    return true;
+  }
+  return false;
+}
 }  // namespace mlg

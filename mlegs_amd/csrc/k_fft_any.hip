@@ -24,6 +24,7 @@
 // 0.40 and 0.73 -> 0.30 ms.
 #include <mutex>
 
+#include "fft_radix.h"
 #include "mlegs_internal.h"
 #include "xcd.h"
 
@@ -34,119 +35,7 @@ namespace mlg {
 
 namespace {
 
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-// a times the root w, or its conjugate for the inverse transform
-template <bool INV>
-__device__ __forceinline__ double2 rmul(double2 a, double2 w) {
-  return INV ? make_double2(a.x * w.x + a.y * w.y, a.y * w.x - a.x * w.y) : cmul(a, w);
-}
-__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-// -i a (forward) or i a (inverse)
-template <bool INV>
-__device__ __forceinline__ double2 mulj(double2 a) {
-  return INV ? make_double2(-a.y, a.x) : make_double2(a.y, -a.x);
-}
-
-// R-point DFT, natural order in and out; w[k st] = e^{-2 pi i k / R}
-// (uniform over the block: scalar loads).
-template <int R, bool INV>
-struct Dft;
-template <bool INV>
-struct Dft<2, INV> {
-  static __device__ __forceinline__ void run(double2 (&v)[2], const double2 *, int) {
-    const double2 a = v[0];
-    v[0] = cadd(a, v[1]);
-    v[1] = csub(a, v[1]);
-  }
-};
-template <bool INV>
-struct Dft<4, INV> {
-  static __device__ __forceinline__ void run(double2 (&v)[4], const double2 *, int) {
-    const double2 a = cadd(v[0], v[2]), b = csub(v[0], v[2]), c = cadd(v[1], v[3]), d = mulj<INV>(csub(v[1], v[3]));
-    v[0] = cadd(a, c);
-    v[1] = cadd(b, d);
-    v[2] = csub(a, c);
-    v[3] = csub(b, d);
-  }
-};
-// odd prime: outputs k and R - k from the sums and differences of inputs q
-// and R - q
-template <int R, bool INV>
-struct DftPrime {
-  static __device__ __forceinline__ void run(double2 (&v)[R], const double2 *__restrict__ w, int st) {
-    constexpr int H = (R - 1) / 2;
-    double2 a[H], d[H];
-    double2 s0 = v[0];
-#pragma unroll
-    for (int q = 1; q <= H; q++) {
-      a[q - 1] = cadd(v[q], v[R - q]);
-      d[q - 1] = csub(v[q], v[R - q]);
-      s0 = cadd(s0, a[q - 1]);
-    }
-    double2 c[H];
-#pragma unroll
-    for (int q = 1; q <= H; q++) c[q - 1] = w[q * st];
-#pragma unroll
-    for (int k = 1; k <= H; k++) {
-      double2 A = v[0], B = make_double2(0.0, 0.0);
-#pragma unroll
-      for (int q = 1; q <= H; q++) {
-        const int e = (q * k) % R, h = e <= H ? e : R - e;
-        const double cx = c[h - 1].x, cy = e <= H ? c[h - 1].y : -c[h - 1].y;
-        A.x += a[q - 1].x * cx;
-        A.y += a[q - 1].y * cx;
-        B.x += d[q - 1].x * cy;
-        B.y += d[q - 1].y * cy;
-      }
-      // forward: A + i B, inverse: A - i B (cy = -sin)
-      const double2 jb = INV ? make_double2(B.y, -B.x) : make_double2(-B.y, B.x);
-      v[k] = cadd(A, jb);
-      v[R - k] = csub(A, jb);
-    }
-    v[0] = s0;
-  }
-};
-template <bool INV> struct Dft<3, INV> : DftPrime<3, INV> {};
-template <bool INV> struct Dft<5, INV> : DftPrime<5, INV> {};
-template <bool INV> struct Dft<7, INV> : DftPrime<7, INV> {};
-template <bool INV> struct Dft<11, INV> : DftPrime<11, INV> {};
-template <bool INV> struct Dft<13, INV> : DftPrime<13, INV> {};
-template <bool INV> struct Dft<17, INV> : DftPrime<17, INV> {};
-template <bool INV> struct Dft<19, INV> : DftPrime<19, INV> {};
-// R = A B: A-point DFTs over stride B, W_R^{j k}, B-point DFTs
-template <int A, int B, bool INV>
-struct DftProduct {
-  static __device__ __forceinline__ void run(double2 (&v)[A * B], const double2 *__restrict__ w, int st) {
-    double2 t[B][A];
-#pragma unroll
-    for (int j = 0; j < B; j++) {
-#pragma unroll
-      for (int q = 0; q < A; q++) t[j][q] = v[j + B * q];
-      Dft<A, INV>::run(t[j], w, st * B);
-#pragma unroll
-      for (int k = 1; k < A; k++)
-        if (j > 0) t[j][k] = rmul<INV>(t[j][k], w[j * k * st]);
-    }
-#pragma unroll
-    for (int k = 0; k < A; k++) {
-      double2 u[B];
-#pragma unroll
-      for (int j = 0; j < B; j++) u[j] = t[j][k];
-      Dft<B, INV>::run(u, w, st * A);
-#pragma unroll
-      for (int j = 0; j < B; j++) v[k + A * j] = u[j];
-    }
-  }
-};
-template <bool INV> struct Dft<6, INV> : DftProduct<2, 3, INV> {};
-template <bool INV> struct Dft<8, INV> : DftProduct<2, 4, INV> {};
-template <bool INV> struct Dft<9, INV> : DftProduct<3, 3, INV> {};
-template <bool INV> struct Dft<10, INV> : DftProduct<2, 5, INV> {};
-template <bool INV> struct Dft<12, INV> : DftProduct<3, 4, INV> {};
-template <bool INV> struct Dft<16, INV> : DftProduct<4, 4, INV> {};
+using namespace fftr;
 
 // One stage: blocks of length L; i0, istep: the thread's first butterfly and
 // the stride to its next one.  ld(position) -> value; st(position, block,

@@ -25,6 +25,7 @@
 // Every value goes through the operations of the separate HORFFT and
 // product kernels, in the same order.  NTH = 256 has its own kernel (below)
 // with the same products and an 8 x 8 x 4 factorisation of the transforms.
+#include "fused_io.h"
 #include "mlegs_internal.h"
 #include "xcd.h"
 
@@ -192,12 +193,6 @@ __device__ void fz_forward(bool act, const KGrid &g, double2 *s, double2 *__rest
     }
   }
 }
-
-struct FusedIO {
-  const double2 *in[10];  // rur rup uz ror rop oz rbr rbp bz [W]
-  double2 *out[4];        // r N_r, r N_theta, N_z, N_b (PFP)
-  double *zl;             // an LN coefficient the launch sets to zero (N_b's), or null
-};
 
 template <int R1, int R2>
 __global__ void __launch_bounds__(256) k_fused_products(KGrid g, const double *__restrict__ rsq, const double2 *__restrict__ tw,
@@ -1141,8 +1136,7 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
 }
 
 bool fused_products_supported(const mlg_ctx *c) {
-  const int n = c->g.nth;
-  return n >= 2 && n <= 256 && (n & (n - 1)) == 0;
+  return fft4_length(c->g.nth) || c->fp.n;
 }
 
 int launch_fused_products(mlg_ctx *c, const double2 *const in[10], double2 *const out[4], double two_omega, double n2,
@@ -1181,6 +1175,7 @@ int launch_fused_products(mlg_ctx *c, const double2 *const in[10], double2 *cons
     MLG_CHECK_HIP(hipGetLastError());
     return 0;
   }
+  if (c->fp.n) return launch_fused_any(c, io, two_omega, n2, linear);
   dim3 grid(xcd_grid((g.ndimr + FP - 1) / FP * g.ndimx));
 #define L_FP(a_, b_)                                                                                                \
   hipLaunchKernelGGL((k_fused_products<a_, b_>), grid, dim3(256), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, \

@@ -44,6 +44,15 @@ struct FftAny {
   int *pos = nullptr;
 };
 
+// The fused products' plan at a theta length (k_fused_any.hip); n = 0: none.
+struct FusedAny {
+  int n = 0, R = 0, D = 1, nmid = 0, P = 0, T = 0;
+  int mid[FFT_MAX_STAGES] = {0};
+  int md = 0;  // n / D
+  unsigned magic[FFT_MAX_STAGES] = {0}, magic_d = 0;  // quotients by the stages' strides
+  long lds = 0;  // bytes a block
+};
+
 // Device copies of the tables and scratch.
 struct DevTables {
   double *pf = nullptr;       // [mm][n][i]  (i fastest), npf rows
@@ -121,6 +130,7 @@ struct mlg_ctx {
   mlg::KTimer timer;
   mlg::DevTables d;
   mlg::FftAny fz, ft;  // z and theta lengths that the four-step kernels do not take
+  mlg::FusedAny fp;    // fused products at such a theta length
   hipStream_t stream = nullptr;
   hipStream_t own_stream = nullptr;
   long n_fff = 0, n_pff = 0, n_ppp = 0, n_max = 0;
@@ -310,6 +320,10 @@ static inline bool fft4_length(int n) { return n >= 2 && n <= 256 && (n & (n - 1
 int fft_any_setup(int n, FftAny *f);  // allocates f's device tables
 int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd);
 int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd);
+// fused products (k_fused_any.hip); f->n = 0 where the length has no plan
+struct FusedIO;
+int fused_any_setup(int nth, FusedAny *f);
+int launch_fused_any(mlg_ctx *c, const FusedIO &io, double two_omega, double n2, int linear);
 // ---- physical-space products (k_physical.hip)
 int launch_vprod(mlg_ctx *c, const double2 *rur, const double2 *rup, const double2 *uz, double2 *ror, double2 *rop, double2 *oz);
 int launch_vdot(mlg_ctx *c, const double2 *rar, const double2 *rap, const double2 *az, const double2 *rbr,

@@ -46,6 +46,40 @@ def plans(tmp_path_factory):
     return out
 
 
+FUSED = r"""
+#include <cstdio>
+#include "fft_plan.h"
+int main() {
+  for (int n = 2; n <= 4096; n++) {
+    mlg::FusedPlan f;
+    if (!mlg::fused_plan(n, f)) continue;
+    std::printf("%d %d %d %d %d %ld %d", n, f.R, f.D, f.P, f.T, mlg::fused_lds(f), f.nmid);
+    for (int i = 0; i < f.nmid; i++) std::printf(" %d", f.mid[i]);
+    std::printf("\n");
+  }
+}
+"""
+
+
+def test_fused_plans_fit_their_block(tmp_path):
+    (tmp_path / "main.cpp").write_text(FUSED)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "mlegs_amd", "csrc"),
+                           str(tmp_path / "main.cpp"), "-o", str(tmp_path / "main")])
+    got = {}
+    for line in subprocess.check_output([str(tmp_path / "main")], text=True).splitlines():
+        n, R, D, P, T, lds, nmid, *mid = [int(x) for x in line.split()]
+        assert R * D * int(np.prod(mid, dtype=int)) == n and len(mid) == nmid and all(2 <= m <= 8 for m in mid) and 2 <= R <= 6
+        assert D % 2 == 1 and D <= 61 and all(D % q for q in (3, 5, 7))
+        assert T % 64 == 0 and n // R * P <= T <= 512 and 4 <= P <= 32
+        lines = n * P * (1 + (D > 1))
+        assert lines + n + n // 2 + 1 == lds and lds * 16 <= 160 * 1024
+        assert (n // 2 + 1) <= (R // 2 + 1) * (T // P)
+        got[n] = (R, D)
+    for n in (3, 9, 12, 45, 90, 100, 122, 204, 306, 384, 512, 600, 640, 768):
+        assert n in got, n
+    assert not {289, 607, 608, 1000, 1024} & set(got)
+
+
 def test_every_length_factors(plans):
     assert sorted(plans) == list(range(2, 4097))
     for n, (rad, direct, freq, pos) in plans.items():
