@@ -247,10 +247,8 @@ extern "C" int mlg_init(const mlg_params *p, mlg_ctx **out) {
     RET(upload(&d.tw_h, v));
   }
   if (!fft4_length(G.nx)) RET(fft_any_setup(G.nx, &c->fz));
-  if (!fft4_length(G.nth)) {
-    RET(fft_any_setup(G.nth, &c->ft));
-    RET(fused_any_setup(G.nth, &c->fp));
-  }
+  if (!fft4_length(G.nth)) RET(fft_any_setup(G.nth, &c->ft));
+  if (!fused_line_length(G.nth)) RET(fused_any_setup(G.nth, &c->fp));
   if (!G.hv_r.empty()) {
     std::vector<double> hv;
     hv.insert(hv.end(), G.hv_r.begin(), G.hv_r.end());

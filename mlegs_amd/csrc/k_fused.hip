@@ -3,28 +3,19 @@
 // CALC_BOUSSI_FORCE / CALC_BOUSSI_NONLIN (src/mod_boussinesq.f90:235-410)
 // take nine fields to physical space (HORFFT backward), form u x omega and
 // u . grad b there (VPRODSUB/VDOTPSUB, src/mod_legops.f90:1972-2232, plus
-// FORCE's linear terms) and bring four results back (HORFFT forward).  This
-// kernel does all of that for two radial pencils of one z plane at a time,
-// reading the inputs in PFP (r, m, z) and writing the outputs in PFP: the
-// 512-point physical theta lines live only in LDS.
-//
-// Block: 256 threads in groups of 32 (2 pencils x 16 threads at NTH = 256);
-// a group transforms one field with the four-step FFT of k_fft.hip.  LDS:
-// eight slots of 2 x NTH complex values (64 KiB at NTH = 256).
-//   phase 1: inverse transforms of rur, rup, uz, ror, rop, oz, rbr, rbp
-//   products A (every point): X = rup oz - uz rop (+ 2 Omega rup),
-//            Y = uz ror - rur oz (- 2 Omega rur), Z = (rur rop - rup ror) / r^2,
-//            T = rur rbr + rup rbp
-//   phase 2: forward transforms of X, Y (and Z without linear terms); then
-//            inverse transforms of bz (and of W = b for FORCE)
-//   products B: N_b = -(T / r^2 + uz bz) (+ Nbar^2 uz); Z = Z - W (FORCE)
-//   phase 3: forward transforms of N_b (and Z for FORCE)
-// Two pencils per block keep the LDS within two blocks per CU; the price is
-// 32-byte runs in the PFP reads and writes, which the XCD-aware block order
-// turns into shared L2 lines.
+// FORCE's linear terms) and bring four results back (HORFFT forward).  The
+// kernels here do all of that for some radial pencils of one z plane at a
+// time, reading the inputs in PFP (r, m, z) and writing the outputs in PFP:
+// the physical theta lines live only in registers and LDS.
+//   products: X = rup oz - uz rop (+ 2 Omega rup), Y = uz ror - rur oz
+//     (- 2 Omega rur), Z = (rur rop - rup ror) / r^2 (- W), N_b = -((rur rbr +
+//     rup rbp) / r^2 + uz bz) (+ Nbar^2 uz)
+//   powers of two up to 512: lines in the registers of 1 .. 64 lanes, all
+//     fields of a line in one wave (k_fused_products_256, k_fused_products_reg)
+//     or one wave a field (k_fused_products_wide); launch_line has the rule
+//   every other length: k_fused_any.hip
 // Every value goes through the operations of the separate HORFFT and
-// product kernels, in the same order.  NTH = 256 has its own kernel (below)
-// with the same products and an 8 x 8 x 4 factorisation of the transforms.
+// product kernels, in the same order.
 #include "fused_io.h"
 #include "mlegs_internal.h"
 #include "xcd.h"
@@ -39,237 +30,6 @@ __device__ __forceinline__ double2 fz_cmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 __device__ __forceinline__ double2 fz_conj(double2 a) { return make_double2(a.x, -a.y); }
-
-template <int R>
-struct FLog2 {
-  static constexpr int v = R <= 1 ? 0 : 1 + FLog2<R / 2>::v;
-};
-template <>
-struct FLog2<1> {
-  static constexpr int v = 0;
-};
-__device__ __forceinline__ constexpr int fz_bitrev(int i, int lg) {
-  int r = 0;
-  for (int b = 0; b < lg; b++) r |= ((i >> b) & 1) << (lg - 1 - b);
-  return r;
-}
-template <int R>
-__device__ __forceinline__ void fz_dft(double2 (&v)[R], const double2 (&wR)[R / 2 > 0 ? R / 2 : 1]) {
-  constexpr int LG = FLog2<R>::v;
-#pragma unroll
-  for (int i = 0; i < R; i++) {
-    const int j = fz_bitrev(i, LG);
-    if (j > i) {
-      double2 t = v[i];
-      v[i] = v[j];
-      v[j] = t;
-    }
-  }
-#pragma unroll
-  for (int half = 1; half < R; half *= 2) {
-#pragma unroll
-    for (int g0 = 0; g0 < R; g0 += 2 * half) {
-#pragma unroll
-      for (int p = 0; p < half; p++) {
-        const double2 w = wR[p * (R / (2 * half))];
-        double2 u = v[g0 + p], x = fz_cmul(v[g0 + p + half], w);
-        v[g0 + p] = make_double2(u.x + x.x, u.y + x.y);
-        v[g0 + p + half] = make_double2(u.x - x.x, u.y - x.y);
-      }
-    }
-  }
-}
-template <int R>
-__device__ __forceinline__ void fz_wr(double2 (&wR)[R / 2 > 0 ? R / 2 : 1], const double2 *__restrict__ tw, int N, bool inv) {
-#pragma unroll
-  for (int j = 0; j < (R / 2 > 0 ? R / 2 : 1); j++) {
-    double2 w = (R > 1) ? tw[j * (N / R)] : make_double2(1.0, 0.0);
-    if (inv) w.y = -w.y;
-    wR[j] = w;
-  }
-}
-
-constexpr int FP = 2;  // pencils per block
-
-// Four-step transform of the two pencils held by a group.  Pass 1 input in
-// v1 (thread t < R2 holds x[R2 n1 + t]); the exchange goes through `s`
-// (slot layout [index][pencil]); on return thread t < R1 holds
-// X[t + R1 k2] in v2.  All threads of the block call it (barriers).
-template <int R1, int R2>
-__device__ __forceinline__ void fz_fft(bool act, double2 (&v1)[R1], double2 (&v2)[R2], double2 *s, int p, int t,
-                                       const double2 *__restrict__ tw, bool inv) {
-  constexpr int N = R1 * R2;
-  if (act && t < R2) {
-    double2 w1[R1 / 2 > 0 ? R1 / 2 : 1];
-    fz_wr<R1>(w1, tw, N, inv);
-    fz_dft<R1>(v1, w1);
-#pragma unroll
-    for (int k1 = 0; k1 < R1; k1++) {
-      double2 w = tw[t * k1];
-      if (inv) w.y = -w.y;
-      s[(k1 * R2 + t) * FP + p] = (k1 == 0 || t == 0) ? v1[k1] : fz_cmul(v1[k1], w);
-    }
-  }
-  __syncthreads();
-  if (act && t < R1) {
-#pragma unroll
-    for (int n2 = 0; n2 < R2; n2++) v2[n2] = s[(t * R2 + n2) * FP + p];
-    double2 w2[R2 / 2 > 0 ? R2 / 2 : 1];
-    fz_wr<R2>(w2, tw, N, inv);
-    fz_dft<R2>(v2, w2);
-  }
-  __syncthreads();
-}
-
-// HORFFT backward of one PFP field into physical slots of `s`.
-template <int R1, int R2>
-__device__ void fz_inverse(bool act, const KGrid &g, const double2 *__restrict__ src, double2 *s, int r0, int z, int p, int t,
-                           const double2 *__restrict__ tw, const double2 *__restrict__ twh) {
-  constexpr int N = R1 * R2;
-  double2 v1[R1], v2[R2];
-  const int rr = r0 + p;
-  const int mmax = g.ntchopdim;
-  if (act && t < R2) {
-    auto X = [&](int m) -> double2 {
-      double2 v = make_double2(0.0, 0.0);
-      if (rr < g.nr && m < g.ntchop) v = src[(size_t)rr + (size_t)g.ndimr * ((size_t)m + (size_t)g.ndimth * z)];
-      if (m == 0) v.y = 0.0;
-      return v;
-    };
-#pragma unroll
-    for (int n1 = 0; n1 < R1; n1++) {
-      const int j = R2 * n1 + t;
-      double2 xm = (j < mmax) ? X(j) : make_double2(0.0, 0.0);
-      const int jc = N - j;
-      double2 xc = (jc < mmax && jc > 0 && j > 0) ? fz_conj(X(jc)) : make_double2(0.0, 0.0);
-      double2 e = make_double2(xm.x + xc.x, xm.y + xc.y);
-      double2 d = make_double2(xm.x - xc.x, xm.y - xc.y);
-      double2 o = fz_cmul(d, fz_conj(twh[j]));
-      v1[n1] = make_double2(e.x - o.y, e.y + o.x);
-    }
-  }
-  fz_fft<R1, R2>(act, v1, v2, s, p, t, tw, true);
-  if (act && t < R1) {
-    const bool live = rr < g.nr;
-#pragma unroll
-    for (int k2 = 0; k2 < R2; k2++) s[(t + R1 * k2) * FP + p] = live ? v2[k2] : make_double2(0.0, 0.0);
-  }
-  __syncthreads();
-}
-
-// HORFFT forward of physical slots in `s` into one PFP field.
-template <int R1, int R2>
-__device__ void fz_forward(bool act, const KGrid &g, double2 *s, double2 *__restrict__ dst, int r0, int z, int p, int t,
-                           int gt, const double2 *__restrict__ tw, const double2 *__restrict__ twh) {
-  constexpr int N = R1 * R2;
-  double2 v1[R1], v2[R2];
-  if (act && t < R2) {
-#pragma unroll
-    for (int n1 = 0; n1 < R1; n1++) v1[n1] = s[(R2 * n1 + t) * FP + p];
-  }
-  __syncthreads();
-  fz_fft<R1, R2>(act, v1, v2, s, p, t, tw, false);
-  if (act && t < R1) {
-#pragma unroll
-    for (int k2 = 0; k2 < R2; k2++) s[(t + R1 * k2) * FP + p] = v2[k2];
-  }
-  __syncthreads();
-  if (act) {
-    const double den = (double)(2 * N);
-    const int mmax = g.ntchopdim;
-    for (int idx = gt; idx < FP * mmax; idx += FP * (R1 > R2 ? R1 : R2)) {
-      const int pr = idx % FP, mm = idx / FP;
-      const int rr = r0 + pr;
-      if (rr >= g.ndimr) continue;
-      double2 zm = s[(mm % N) * FP + pr], zc = fz_conj(s[((N - mm) % N) * FP + pr]);
-      double2 e = make_double2(0.5 * (zm.x + zc.x), 0.5 * (zm.y + zc.y));
-      double2 d = make_double2(zm.x - zc.x, zm.y - zc.y);
-      double2 wd = fz_cmul(twh[mm], d);
-      double2 x = make_double2(e.x + 0.5 * wd.y, e.y - 0.5 * wd.x);
-      x = make_double2(x.x / den, x.y / den);
-      if (mm == 0) x.y = 0.0;
-      if (mm >= g.ntchop || rr >= g.nr) x = make_double2(0.0, 0.0);
-      dst[(size_t)rr + (size_t)g.ndimr * ((size_t)mm + (size_t)g.ndimth * z)] = x;
-    }
-  }
-}
-
-template <int R1, int R2>
-__global__ void __launch_bounds__(256) k_fused_products(KGrid g, const double *__restrict__ rsq, const double2 *__restrict__ tw,
-                                                        const double2 *__restrict__ twh, FusedIO io, double two_omega,
-                                                        double n2, int linear) {
-  if (blockIdx.x == 0 && threadIdx.x == 0 && io.zl) io.zl[0] = 0.0;
-  constexpr int N = R1 * R2, TPP = R1 > R2 ? R1 : R2, GS = FP * TPP, NG = 256 / GS, SL = FP * N;
-  static_assert(NG >= 8, "eight concurrent transforms");
-  __shared__ double2 S[8 * SL];
-  // logical block = (pencil pair, z) with the pair fastest: the four pairs
-  // of one 128-byte line run on one XCD
-  const int nrp = (g.ndimr + FP - 1) / FP;
-  const int lid = xcd_logical(nrp * g.ndimx);
-  if (lid < 0) return;
-  const int z = lid / nrp, r0 = (lid % nrp) * FP;
-  const int grp = threadIdx.x / GS, gt = threadIdx.x % GS, p = gt % FP, t = gt / FP;
-  auto slot = [&](int q) { return S + (size_t)q * SL; };
-
-  // phase 1: rur rup uz ror rop oz rbr rbp -> slots 0..7
-  {
-    const bool act = grp < 8;
-    const int q = act ? grp : 0;
-    fz_inverse<R1, R2>(act, g, io.in[q], slot(q), r0, z, p, t, tw, twh);
-  }
-  // products A
-  for (int q = threadIdx.x; q < SL; q += 256) {
-    const int pr = q % FP, rr = r0 + pr;
-    if (rr >= g.nr) continue;
-    const double r2 = rsq[rr];
-    const double2 A = slot(0)[q], B = slot(1)[q], C = slot(2)[q], D = slot(3)[q], E = slot(4)[q], F = slot(5)[q];
-    const double2 P = slot(6)[q], Q = slot(7)[q];
-    double2 xr = make_double2(B.x * F.x - C.x * E.x, B.y * F.y - C.y * E.y);
-    double2 xp = make_double2(C.x * D.x - A.x * F.x, C.y * D.y - A.y * F.y);
-    double2 xz = make_double2((A.x * E.x - B.x * D.x) / r2, (A.y * E.y - B.y * D.y) / r2);
-    double2 tt = make_double2(A.x * P.x + B.x * Q.x, A.y * P.y + B.y * Q.y);
-    if (linear) {
-      xr = make_double2(xr.x + two_omega * B.x, xr.y + two_omega * B.y);
-      xp = make_double2(xp.x - two_omega * A.x, xp.y - two_omega * A.y);
-    }
-    slot(3)[q] = xr;
-    slot(4)[q] = xp;
-    slot(5)[q] = xz;
-    slot(7)[q] = tt;
-  }
-  __syncthreads();
-  // phase 2: forward X, Y (Z if no linear terms); then inverse bz -> slot 6
-  // (and W -> slot 0, rur being no longer needed)
-  {
-    const bool fwd = grp < (linear ? 2 : 3);
-    fz_forward<R1, R2>(fwd, g, slot(3 + (fwd ? grp : 0)), io.out[fwd ? grp : 0], r0, z, p, t, gt, tw, twh);
-  }
-  {
-    const bool inv = (grp == 3) || (linear && grp == 4);
-    fz_inverse<R1, R2>(inv, g, io.in[grp == 4 ? 9 : 8], slot(grp == 4 ? 0 : 6), r0, z, p, t, tw, twh);
-  }
-  // products B
-  for (int q = threadIdx.x; q < SL; q += 256) {
-    const int pr = q % FP, rr = r0 + pr;
-    if (rr >= g.nr) continue;
-    const double r2 = rsq[rr];
-    const double2 C = slot(2)[q], R = slot(6)[q], T = slot(7)[q];
-    const double vr = T.x / r2 + C.x * R.x, vi = T.y / r2 + C.y * R.y;
-    double2 nb = make_double2(-vr, -vi);
-    if (linear) {
-      const double2 W = slot(0)[q], Z = slot(5)[q];
-      nb = make_double2(nb.x + n2 * C.x, nb.y + n2 * C.y);
-      slot(5)[q] = make_double2(Z.x - W.x, Z.y - W.y);
-    }
-    slot(7)[q] = nb;
-  }
-  __syncthreads();
-  // phase 3: forward N_b (and N_z with linear terms)
-  {
-    const bool act = (grp == 0) || (linear && grp == 1);
-    fz_forward<R1, R2>(act, g, slot(grp == 1 ? 5 : 7), io.out[grp == 1 ? 2 : 3], r0, z, p, t, gt, tw, twh);
-  }
-}
 
 // ---------------------------------------------------------------------------
 // NTH = 256: register-resident variant.
@@ -385,11 +145,20 @@ __device__ __forceinline__ double2 cj(double2 w, bool inv) {
   return w;
 }
 
+// Both terms of the Hermitian merge (truncations past 3/8 of NTH): xm = X[j],
+// xc = conj X[N-j], th = exp(-i pi j / N)
+__device__ __forceinline__ double2 merge_full(double2 xm, double2 xc, double2 th) {
+  const double2 e = cadd(xm, xc), o = fz_cmul(csub(xm, xc), fz_conj(th));
+  return make_double2(e.x - o.y, e.y + o.x);
+}
+
 // HORFFT backward of one PFP line (element m at src[lo + ndimr m], src the
 // same for the whole block); lane b ends with the physical points
 // P[c + 8 (gh + 4 s) + 64 h] in v[4 s + h], c = b >> 2, gh = b & 3.
-// Needs NTCHOPDIM <= MMAX96: only a = 0..2 hold modes, a = 5..7 partners.
+// Without FULL, NTCHOPDIM <= MMAX96: only a = 0..2 hold modes, a = 5..7
+// partners.
 constexpr int MMAX96 = 96;
+template <bool FULL>
 __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const double2 *__restrict__ src, int lo,
                                         bool live, double2 (&v)[8]) {
   const int b = x.b, mmax = g.ntchopdim;
@@ -407,17 +176,22 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
   // conj X[N-j] (j >= 160) times 1 - i conj(th[j]) = 1 + i th[N-j].
 #pragma unroll
   for (int a = 0; a < 8; a++) {
-    if (a == 3 || a == 4) {
+    if (!FULL && (a == 3 || a == 4)) {
       v[a] = make_double2(0.0, 0.0);
       continue;
     }
     const int j = 32 * a + b, jc = N - j;
+    if constexpr (FULL) {
+      v[a] = merge_full(X(j, j < mmax), fz_conj(X(jc, j > 0 && jc < mmax)), x.th[j]);
+      continue;
+    }
     const double2 t = x.th[a < 3 ? j : jc];
     const double2 xv = a < 3 ? X(j, j < mmax) : fz_conj(X(jc, jc < mmax));
     const double2 q = a < 3 ? make_double2(1.0 + t.y, t.x) : make_double2(1.0 - t.y, t.x);
     v[a] = fz_cmul(xv, q);
   }
-  dft8s_z34<1>(v);
+  if constexpr (FULL) dft8s<1>(v);
+  else dft8s_z34<1>(v);
   // twiddles W^0 = 1 multiply exactly
 #pragma unroll
   for (int c = 1; c < 8; c++) v[c] = fz_cmul(v[c], cj(x.t1[32 * c + b], true));
@@ -452,6 +226,7 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
 
 // HORFFT forward of this lane's physical points v (positions as left by
 // `inverse`) into one PFP line (element m at dst[lo + ndimr m]).
+template <bool FULL>
 __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *__restrict__ dst,
                                         int lo, bool inr, bool live) {
   const int b = x.b, c0 = b >> 2, f0 = b & 3;
@@ -489,7 +264,7 @@ __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const doub
   const double den = (double)(2 * N);
   const int src = (32 - b) & 31;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
+  for (int a = 0; a < (FULL ? 8 : 3); a++) {
     if (32 * a >= g.ntchopdim) break;
     const int m = 32 * a + b;
     double2 pc;
@@ -554,25 +329,25 @@ k_fused_products_256(KGrid g, const double *__restrict__ rsq, const double2 *tw,
   const double r2 = live ? rsq[rr] : 1.0;
 
   double2 A[8], B[8], C[8], U[8], V[8], T[8];
-  inverse(x, g, in(0), lo, live, A);  // rur
-  inverse(x, g, in(1), lo, live, B);  // rup
-  inverse(x, g, in(2), lo, live, C);  // uz
+  inverse<false>(x, g, in(0), lo, live, A);  // rur
+  inverse<false>(x, g, in(1), lo, live, B);  // rup
+  inverse<false>(x, g, in(2), lo, live, C);  // uz
   // oz: U = rup oz, V = rur oz
-  inverse(x, g, in(5), lo, live, T);
+  inverse<false>(x, g, in(5), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     U[i] = make_double2(B[i].x * T[i].x, B[i].y * T[i].y);
     V[i] = make_double2(A[i].x * T[i].x, A[i].y * T[i].y);
   }
   // ror: Y = uz ror - rur oz (to LDS); V = rup ror
-  inverse(x, g, in(3), lo, live, T);
+  inverse<false>(x, g, in(3), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     ys[32 * i] = make_double2(C[i].x * T[i].x - V[i].x, C[i].y * T[i].y - V[i].y);
     V[i] = make_double2(B[i].x * T[i].x, B[i].y * T[i].y);
   }
   // rop: X = rup oz - uz rop in U; Z = (rur rop - rup ror) / r^2 in V
-  inverse(x, g, in(4), lo, live, T);
+  inverse<false>(x, g, in(4), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     U[i] = make_double2(U[i].x - C[i].x * T[i].x, U[i].y - C[i].y * T[i].y);
@@ -583,29 +358,29 @@ k_fused_products_256(KGrid g, const double *__restrict__ rsq, const double2 *tw,
 #pragma unroll
     for (int i = 0; i < 8; i++) U[i] = make_double2(U[i].x + two_omega * B[i].x, U[i].y + two_omega * B[i].y);
   }
-  forward(x, g, U, out(0), lo, inr, live);
+  forward<false>(x, g, U, out(0), lo, inr, live);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     T[i] = ys[32 * i];
     if (LINEAR) T[i] = make_double2(T[i].x - two_omega * A[i].x, T[i].y - two_omega * A[i].y);
   }
-  forward(x, g, T, out(1), lo, inr, live);
+  forward<false>(x, g, T, out(1), lo, inr, live);
   if (LINEAR) {
     // W: N_z = Z - W
-    inverse(x, g, in(9), lo, live, T);
+    inverse<false>(x, g, in(9), lo, live, T);
 #pragma unroll
     for (int i = 0; i < 8; i++) V[i] = make_double2(V[i].x - T[i].x, V[i].y - T[i].y);
   }
-  forward(x, g, V, out(2), lo, inr, live);
+  forward<false>(x, g, V, out(2), lo, inr, live);
   // rbr, rbp: A = rur rbr + rup rbp
-  inverse(x, g, in(6), lo, live, T);
+  inverse<false>(x, g, in(6), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) A[i] = make_double2(A[i].x * T[i].x, A[i].y * T[i].y);
-  inverse(x, g, in(7), lo, live, T);
+  inverse<false>(x, g, in(7), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) A[i] = make_double2(A[i].x + B[i].x * T[i].x, A[i].y + B[i].y * T[i].y);
   // bz: N_b = -(T / r^2 + uz bz) (+ Nbar^2 uz)
-  inverse(x, g, in(8), lo, live, T);
+  inverse<false>(x, g, in(8), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     const double vr = A[i].x / r2 + C[i].x * T[i].x, vi = A[i].y / r2 + C[i].y * T[i].y;
@@ -613,7 +388,7 @@ k_fused_products_256(KGrid g, const double *__restrict__ rsq, const double2 *tw,
     if (LINEAR) nb = make_double2(nb.x + n2 * C[i].x, nb.y + n2 * C[i].y);
     A[i] = nb;
   }
-  forward(x, g, A, out(3), lo, inr, live);
+  forward<false>(x, g, A, out(3), lo, inr, live);
 }
 
 // ---------------------------------------------------------------------------
@@ -643,6 +418,7 @@ using w256::cj;
 using w256::csub;
 using w256::dft4s;
 using w256::dft8s;
+using w256::merge_full;
 using w256::dft8s_z34;
 using w256::wave_sync;
 using w256::Ctx;  // t1[16 c + b] = W_N^{b c}, t2[4 g + f] = W_N^{8 f g}, th[k] = exp(-i pi k / N)
@@ -650,6 +426,7 @@ using w256::Ctx;  // t1[16 c + b] = W_N^{b c}, t2[4 g + f] = W_N^{8 f g}, th[k] 
 // HORFFT backward of one PFP line (element m at src[lo + ndimr m]); lane b
 // ends with the physical points P[c + 8 g + 32 h] in v[4 s + h], c = c2 + 4 s,
 // c2 = b >> 2, g = b & 3.
+template <bool FULL>
 __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const double2 *__restrict__ src, int lo,
                                         bool live, double2 (&v)[8]) {
   const int b = x.b, mmax = g.ntchopdim;
@@ -663,17 +440,22 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
   // Hermitian merge with one term per point, as at NTH = 256
 #pragma unroll
   for (int a = 0; a < 8; a++) {
-    if (a == 3 || a == 4) {
+    if (!FULL && (a == 3 || a == 4)) {
       v[a] = make_double2(0.0, 0.0);
       continue;
     }
     const int j = 16 * a + b, jc = N - j;
+    if constexpr (FULL) {
+      v[a] = merge_full(X(j, j < mmax), fz_conj(X(jc, j > 0 && jc < mmax)), x.th[j]);
+      continue;
+    }
     const double2 t = x.th[a < 3 ? j : jc];
     const double2 xv = a < 3 ? X(j, j < mmax) : fz_conj(X(jc, jc < mmax));
     const double2 q = a < 3 ? make_double2(1.0 + t.y, t.x) : make_double2(1.0 - t.y, t.x);
     v[a] = fz_cmul(xv, q);
   }
-  dft8s_z34<1>(v);
+  if constexpr (FULL) dft8s<1>(v);
+  else dft8s_z34<1>(v);
 #pragma unroll
   for (int c = 1; c < 8; c++) v[c] = fz_cmul(v[c], cj(x.t1[16 * c + b], true));
   // exchange 1: lane b holds y_b[c]; lane 4 c2 + f takes y_{4 e + f}[c], c = c2, c2 + 4
@@ -714,6 +496,7 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
 
 // HORFFT forward of this lane's physical points v (positions as left by
 // `inverse`) into one PFP line (element m at dst[lo + ndimr m]).
+template <bool FULL>
 __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *__restrict__ dst,
                                         int lo, bool inr, bool live) {
   const int b = x.b, c2 = b >> 2, g0 = b & 3;
@@ -756,7 +539,7 @@ __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const doub
   const double den = (double)(2 * N);
   const int src = (16 - b) & 15;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
+  for (int a = 0; a < (FULL ? 8 : 3); a++) {
     if (16 * a >= g.ntchopdim) break;
     const int m = 16 * a + b;
     double2 pc;
@@ -795,9 +578,11 @@ __device__ __forceinline__ int e1(int c, int b) { return c * 9 + b; }
 using w256::cj;
 using w256::Ctx;  // t1[8 c + b] = W_N^{b c}, th[k] = exp(-i pi k / N)
 using w256::dft8s;
+using w256::merge_full;
 using w256::dft8s_z34;
 using w256::wave_sync;
 
+template <bool FULL>
 __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const double2 *__restrict__ src, int lo,
                                         bool live, double2 (&v)[8]) {
   const int b = x.b, mmax = g.ntchopdim;
@@ -810,17 +595,22 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
   };
 #pragma unroll
   for (int a = 0; a < 8; a++) {
-    if (a == 3 || a == 4) {
+    if (!FULL && (a == 3 || a == 4)) {
       v[a] = make_double2(0.0, 0.0);
       continue;
     }
     const int j = 8 * a + b, jc = N - j;
+    if constexpr (FULL) {
+      v[a] = merge_full(X(j, j < mmax), fz_conj(X(jc, j > 0 && jc < mmax)), x.th[j]);
+      continue;
+    }
     const double2 t = x.th[a < 3 ? j : jc];
     const double2 xv = a < 3 ? X(j, j < mmax) : fz_conj(X(jc, jc < mmax));
     const double2 q = a < 3 ? make_double2(1.0 + t.y, t.x) : make_double2(1.0 - t.y, t.x);
     v[a] = fz_cmul(xv, q);
   }
-  dft8s_z34<1>(v);
+  if constexpr (FULL) dft8s<1>(v);
+  else dft8s_z34<1>(v);
 #pragma unroll
   for (int c = 1; c < 8; c++) v[c] = fz_cmul(v[c], cj(x.t1[8 * c + b], true));
 #pragma unroll
@@ -832,6 +622,7 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
   dft8s<1>(v);
 }
 
+template <bool FULL>
 __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *__restrict__ dst,
                                         int lo, bool inr, bool live) {
   const int b = x.b;
@@ -853,7 +644,7 @@ __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const doub
   const double den = (double)(2 * N);
   const int src = (8 - b) & 7;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
+  for (int a = 0; a < (FULL ? 8 : 3); a++) {
     if (8 * a >= g.ntchopdim) break;
     const int m = 8 * a + b;
     double2 pc;
@@ -893,9 +684,11 @@ using w256::cj;
 using w256::Ctx;  // t1[4 c + b] = W_N^{b c}, th[k] = exp(-i pi k / N)
 using w256::dft4s;
 using w256::dft8s;
+using w256::merge_full;
 using w256::dft8s_z34;
 using w256::wave_sync;
 
+template <bool FULL>
 __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const double2 *__restrict__ src, int lo,
                                         bool live, double2 (&v)[8]) {
   const int b = x.b, mmax = g.ntchopdim;
@@ -908,17 +701,22 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
   };
 #pragma unroll
   for (int a = 0; a < 8; a++) {
-    if (a == 3 || a == 4) {
+    if (!FULL && (a == 3 || a == 4)) {
       v[a] = make_double2(0.0, 0.0);
       continue;
     }
     const int j = 4 * a + b, jc = N - j;
+    if constexpr (FULL) {
+      v[a] = merge_full(X(j, j < mmax), fz_conj(X(jc, j > 0 && jc < mmax)), x.th[j]);
+      continue;
+    }
     const double2 t = x.th[a < 3 ? j : jc];
     const double2 xv = a < 3 ? X(j, j < mmax) : fz_conj(X(jc, jc < mmax));
     const double2 q = a < 3 ? make_double2(1.0 + t.y, t.x) : make_double2(1.0 - t.y, t.x);
     v[a] = fz_cmul(xv, q);
   }
-  dft8s_z34<1>(v);
+  if constexpr (FULL) dft8s<1>(v);
+  else dft8s_z34<1>(v);
 #pragma unroll
   for (int c = 1; c < 8; c++) v[c] = fz_cmul(v[c], cj(x.t1[4 * c + b], true));
 #pragma unroll
@@ -938,6 +736,7 @@ __device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const doub
   }
 }
 
+template <bool FULL>
 __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *__restrict__ dst,
                                         int lo, bool inr, bool live) {
   const int b = x.b;
@@ -963,7 +762,7 @@ __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const doub
   const double den = (double)(2 * N);
   const int src = (4 - b) & 3;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
+  for (int a = 0; a < (FULL ? 8 : 3); a++) {
     if (4 * a >= g.ntchopdim) break;
     const int m = 4 * a + b;
     double2 pc;
@@ -986,64 +785,402 @@ __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const doub
 
 }  // namespace w32
 
-// Line shapes of the register-resident kernel below: lanes per theta line,
+// ---------------------------------------------------------------------------
+// NTH = 512: a wave owns one theta line, each lane 8 of its points; eight
+// waves, and eight adjacent radial nodes, a block.  The 512-point transform is
+// 8 x 8 x 8:
+//   j = 64 a + b (lane b holds a = 0..7)          -> 8-point DFT over a, twiddle
+//   exchange: lane 8 c + f (b = 8 e + f) holds e = 0..7 of c
+//                                                  -> 8-point DFT over e, twiddle
+//   exchange: lane 8 c + g holds f = 0..7          -> 8-point DFT over f
+// so lane 8 c + g ends with the points k = c + 8 g + 64 h, h = 0..7.
+// ---------------------------------------------------------------------------
+namespace w512 {
+
+constexpr int N = 512;
+constexpr int LP = 576;       // LDS double2 per line (rows of 9 against bank conflicts)
+constexpr int MMAX192 = 192;  // NTCHOPDIM bound without FULL: slots a = 3, 4 hold no mode
+__device__ __forceinline__ int e1(int c, int b) { return c * 72 + b; }
+__device__ __forceinline__ int e2(int c, int f, int g) { return c * 72 + f * 9 + g; }
+using w256::cj;
+using w256::Ctx;  // t1[64 c + b] = W_N^{b c}, t2[8 g + f] = W_N^{8 f g}, th[k] = exp(-i pi k / N)
+using w256::dft8s;
+using w256::dft8s_z34;
+using w256::merge_full;
+using w256::wave_sync;
+
+template <bool FULL>
+__device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const double2 *__restrict__ src, int lo,
+                                        bool live, double2 (&v)[8]) {
+  const int b = x.b, mmax = g.ntchopdim;
+  auto X = [&](int m, bool use) -> double2 {
+    use = use && live && m < g.ntchop;
+    double2 t = src[lo + (use ? g.ndimr * m : 0)];
+    if (!use) t = make_double2(0.0, 0.0);
+    if (m == 0) t.y = 0.0;
+    return t;
+  };
+#pragma unroll
+  for (int a = 0; a < 8; a++) {
+    if (!FULL && (a == 3 || a == 4)) {
+      v[a] = make_double2(0.0, 0.0);
+      continue;
+    }
+    const int j = 64 * a + b, jc = N - j;
+    if constexpr (FULL) {
+      v[a] = merge_full(X(j, j < mmax), fz_conj(X(jc, j > 0 && jc < mmax)), x.th[j]);
+      continue;
+    }
+    const double2 t = x.th[a < 3 ? j : jc];
+    const double2 xv = a < 3 ? X(j, j < mmax) : fz_conj(X(jc, jc < mmax));
+    const double2 q = a < 3 ? make_double2(1.0 + t.y, t.x) : make_double2(1.0 - t.y, t.x);
+    v[a] = fz_cmul(xv, q);
+  }
+  if constexpr (FULL) dft8s<1>(v);
+  else dft8s_z34<1>(v);
+#pragma unroll
+  for (int c = 1; c < 8; c++) v[c] = fz_cmul(v[c], cj(x.t1[64 * c + b], true));
+#pragma unroll
+  for (int c = 0; c < 8; c++) x.s[e1(c, b)] = v[c];
+  wave_sync();
+  const int c0 = b >> 3, f0 = b & 7;
+#pragma unroll
+  for (int e = 0; e < 8; e++) v[e] = x.s[e1(c0, 8 * e + f0)];
+  wave_sync();
+  dft8s<1>(v);
+#pragma unroll
+  for (int gg = 1; gg < 8; gg++) v[gg] = fz_cmul(v[gg], cj(x.t2[8 * gg + f0], true));
+#pragma unroll
+  for (int gg = 0; gg < 8; gg++) x.s[e2(c0, f0, gg)] = v[gg];
+  wave_sync();
+#pragma unroll
+  for (int f = 0; f < 8; f++) v[f] = x.s[e2(c0, f, f0)];
+  wave_sync();
+  dft8s<1>(v);
+}
+
+template <bool FULL>
+__device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *__restrict__ dst,
+                                        int lo, bool inr, bool live) {
+  const int b = x.b, c0 = b >> 3, f0 = b & 7;
+  double2 u[8];
+#pragma unroll
+  for (int h = 0; h < 8; h++) u[h] = v[h];
+  dft8s<-1>(u);
+#pragma unroll
+  for (int f = 1; f < 8; f++) u[f] = fz_cmul(u[f], x.t2[8 * f0 + f]);
+#pragma unroll
+  for (int f = 0; f < 8; f++) x.s[e2(c0, f, f0)] = u[f];
+  wave_sync();
+#pragma unroll
+  for (int gg = 0; gg < 8; gg++) u[gg] = x.s[e2(c0, f0, gg)];
+  wave_sync();
+  dft8s<-1>(u);
+#pragma unroll
+  for (int e = 0; e < 8; e++) x.s[e1(c0, 8 * e + f0)] = u[e];
+  wave_sync();
+#pragma unroll
+  for (int c = 0; c < 8; c++) u[c] = x.s[e1(c, b)];
+  wave_sync();
+#pragma unroll
+  for (int c = 1; c < 8; c++) u[c] = fz_cmul(u[c], x.t1[64 * c + b]);
+  dft8s<-1>(u);
+  // u[a] = Y[64 a + b]; Y[N - m] sits in lane (64 - b) mod 64 at a' = 7 - a
+  // (lane 0: a' = (8 - a) mod 8)
+  const double den = (double)(2 * N);
+  const int src = (64 - b) & 63;
+#pragma unroll
+  for (int a = 0; a < (FULL ? 8 : 3); a++) {
+    if (64 * a >= g.ntchopdim) break;
+    const int m = 64 * a + b;
+    double2 pc;
+    pc.x = __shfl(u[7 - a].x, src, 64);
+    pc.y = __shfl(u[7 - a].y, src, 64);
+    if (b == 0) pc = u[(8 - a) & 7];
+    if (m < g.ntchopdim && inr) {
+      double2 zm = u[a], zc = fz_conj(pc);
+      double2 e = make_double2(0.5 * (zm.x + zc.x), 0.5 * (zm.y + zc.y));
+      double2 d = make_double2(zm.x - zc.x, zm.y - zc.y);
+      double2 wd = fz_cmul(x.th[m], d);
+      double2 o = make_double2(e.x + 0.5 * wd.y, e.y - 0.5 * wd.x);
+      o = make_double2(o.x / den, o.y / den);
+      if (m == 0) o.y = 0.0;
+      if (m >= g.ntchop || !live) o = make_double2(0.0, 0.0);
+      dst[lo + g.ndimr * m] = o;
+    }
+  }
+}
+
+}  // namespace w512
+
+// ---------------------------------------------------------------------------
+// NTH = 16: 2 lanes own one theta line (32 lines per wave), each keeping 8 of
+// its points, with a 8 x 2 transform: j = 2 a + b (lane b holds a = 0..7) ->
+// 8-point DFT over a, twiddle, 2-point DFT between the two lanes; lane b ends
+// with the points k = c + 8 b.  No LDS.
+// ---------------------------------------------------------------------------
+namespace w16 {
+
+constexpr int N = 16;
+constexpr int MMAX6 = 6;  // NTCHOPDIM bound without FULL: slots a = 3, 4 hold no mode
+using w256::cj;
+using w256::Ctx;  // t1[2 c + b] = W_N^{b c}, th[k] = exp(-i pi k / N)
+using w256::dft8s;
+using w256::dft8s_z34;
+using w256::merge_full;
+
+// v[c] = v0[c] + v1[c] in lane 0, v0[c] - v1[c] in lane 1
+__device__ __forceinline__ void pair2(int b, double2 (&v)[8]) {
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    const double ox = __shfl_xor(v[c].x, 1, 64), oy = __shfl_xor(v[c].y, 1, 64);
+    v[c] = b ? make_double2(ox - v[c].x, oy - v[c].y) : make_double2(v[c].x + ox, v[c].y + oy);
+  }
+}
+
+template <bool FULL>
+__device__ __forceinline__ void inverse(const Ctx &x, const KGrid &g, const double2 *__restrict__ src, int lo,
+                                        bool live, double2 (&v)[8]) {
+  const int b = x.b, mmax = g.ntchopdim;
+  auto X = [&](int m, bool use) -> double2 {
+    use = use && live && m < g.ntchop;
+    double2 t = src[lo + (use ? g.ndimr * m : 0)];
+    if (!use) t = make_double2(0.0, 0.0);
+    if (m == 0) t.y = 0.0;
+    return t;
+  };
+#pragma unroll
+  for (int a = 0; a < 8; a++) {
+    if (!FULL && (a == 3 || a == 4)) {
+      v[a] = make_double2(0.0, 0.0);
+      continue;
+    }
+    const int j = 2 * a + b, jc = N - j;
+    if constexpr (FULL) {
+      v[a] = merge_full(X(j, j < mmax), fz_conj(X(jc, j > 0 && jc < mmax)), x.th[j]);
+      continue;
+    }
+    const double2 t = x.th[a < 3 ? j : jc];
+    const double2 xv = a < 3 ? X(j, j < mmax) : fz_conj(X(jc, jc < mmax));
+    const double2 q = a < 3 ? make_double2(1.0 + t.y, t.x) : make_double2(1.0 - t.y, t.x);
+    v[a] = fz_cmul(xv, q);
+  }
+  if constexpr (FULL) dft8s<1>(v);
+  else dft8s_z34<1>(v);
+#pragma unroll
+  for (int c = 1; c < 8; c++) v[c] = fz_cmul(v[c], cj(x.t1[2 * c + b], true));
+  pair2(b, v);
+}
+
+template <bool FULL>
+__device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *__restrict__ dst,
+                                        int lo, bool inr, bool live) {
+  const int b = x.b;
+  double2 u[8];
+#pragma unroll
+  for (int c = 0; c < 8; c++) u[c] = v[c];
+  pair2(b, u);
+#pragma unroll
+  for (int c = 1; c < 8; c++) u[c] = fz_cmul(u[c], x.t1[2 * c + b]);
+  dft8s<-1>(u);
+  // u[a] = Y[2 a + b]; Y[N - m] is this lane's a' = (8 - a) mod 8 (b = 0), 7 - a (b = 1)
+  const double den = (double)(2 * N);
+#pragma unroll
+  for (int a = 0; a < (FULL ? 8 : 3); a++) {
+    const int m = 2 * a + b;
+    const double2 pc = b ? u[7 - a] : u[(8 - a) & 7];
+    if (m < g.ntchopdim && inr) {
+      double2 zm = u[a], zc = fz_conj(pc);
+      double2 e = make_double2(0.5 * (zm.x + zc.x), 0.5 * (zm.y + zc.y));
+      double2 d = make_double2(zm.x - zc.x, zm.y - zc.y);
+      double2 wd = fz_cmul(x.th[m], d);
+      double2 o = make_double2(e.x + 0.5 * wd.y, e.y - 0.5 * wd.x);
+      o = make_double2(o.x / den, o.y / den);
+      if (m == 0) o.y = 0.0;
+      if (m >= g.ntchop || !live) o = make_double2(0.0, 0.0);
+      dst[lo + g.ndimr * m] = o;
+    }
+  }
+}
+
+}  // namespace w16
+
+// ---------------------------------------------------------------------------
+// NTH = N = 2, 4, 8: a lane owns a theta line, its points in the first N of
+// the 8 slots.
+// ---------------------------------------------------------------------------
+template <int N>
+struct w8 {
+  template <int S>
+  __device__ __forceinline__ static void dft(double2 (&v)[8]) {
+    if constexpr (N == 8) {
+      w256::dft8s<S>(v);
+    } else if constexpr (N == 4) {
+      double2 y[4] = {v[0], v[1], v[2], v[3]};
+      w256::dft4s<S>(y);
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[k] = y[k];
+    } else {
+      const double2 a = v[0], b = v[1];
+      v[0] = w256::cadd(a, b);
+      v[1] = w256::csub(a, b);
+    }
+  }
+  __device__ __forceinline__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *__restrict__ src, int lo,
+                                                 bool live, double2 (&v)[8]) {
+    const int mmax = g.ntchopdim;
+    auto X = [&](int m, bool use) -> double2 {
+      use = use && live && m < g.ntchop;
+      double2 t = src[lo + (use ? g.ndimr * m : 0)];
+      if (!use) t = make_double2(0.0, 0.0);
+      if (m == 0) t.y = 0.0;
+      return t;
+    };
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      v[j] = j < N ? w256::merge_full(X(j, j < mmax), fz_conj(X(N - j, j > 0 && N - j < mmax)), x.th[j < N ? j : 0])
+                   : make_double2(0.0, 0.0);
+    dft<1>(v);
+  }
+  __device__ __forceinline__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8],
+                                                 double2 *__restrict__ dst, int lo, bool inr, bool live) {
+    double2 u[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) u[c] = v[c];
+    dft<-1>(u);
+    const double den = (double)(2 * N);
+#pragma unroll
+    for (int m = 0; m < N; m++) {
+      if (m < g.ntchopdim && inr) {
+        double2 zm = u[m], zc = fz_conj(u[(N - m) % N]);
+        double2 e = make_double2(0.5 * (zm.x + zc.x), 0.5 * (zm.y + zc.y));
+        double2 d = make_double2(zm.x - zc.x, zm.y - zc.y);
+        double2 wd = fz_cmul(x.th[m], d);
+        double2 o = make_double2(e.x + 0.5 * wd.y, e.y - 0.5 * wd.x);
+        o = make_double2(o.x / den, o.y / den);
+        if (m == 0) o.y = 0.0;
+        if (m >= g.ntchop || !live) o = make_double2(0.0, 0.0);
+        dst[lo + g.ndimr * m] = o;
+      }
+    }
+  }
+};
+
+// Line shapes of the kernels below: lanes per theta line,
 // LDS per line, the NTCHOPDIM bound of the pruned first stage, and the
 // per-lane twiddle tables (T1[LANES c + b] = W_N^{b c}; T2 of NTH = 128's
 // middle stage, T2[4 g + f] = W_N^{8 f g}).
+template <int NN>
+struct LineTiny {
+  static constexpr int N = NN, LANES = 1, LP = 8, MMAX = 0, NT2 = 1;
+  __device__ static void tables(int, double2 *, double2 *, const double2 *) {}
+  template <bool FULL>
+  __device__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *src, int lo, bool live,
+                                 double2 (&v)[8]) {
+    w8<N>::inverse(x, g, src, lo, live, v);
+  }
+  template <bool FULL>
+  __device__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *dst, int lo, bool inr,
+                                 bool live) {
+    w8<N>::forward(x, g, v, dst, lo, inr, live);
+  }
+};
+struct Line16 {
+  static constexpr int N = 16, LANES = 2, THREADS = 256, LP = 16, MMAX = w16::MMAX6, NT2 = 1;
+  __device__ static void tables(int q, double2 *T1, double2 *, const double2 *tw) {
+    if (q < 16) T1[q] = tw[(q & 1) * (q >> 1)];
+  }
+  template <bool FULL>
+  __device__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *src, int lo, bool live,
+                                 double2 (&v)[8]) {
+    w16::inverse<FULL>(x, g, src, lo, live, v);
+  }
+  template <bool FULL>
+  __device__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *dst, int lo, bool inr,
+                                 bool live) {
+    w16::forward<FULL>(x, g, v, dst, lo, inr, live);
+  }
+};
 struct Line128 {
-  static constexpr int N = 128, LANES = 16, LP = w128::LP, MMAX = w128::MMAX48, NT2 = 16;
+  static constexpr int N = 128, LANES = 16, THREADS = 256, LP = w128::LP, MMAX = w128::MMAX48, NT2 = 16;
   __device__ static void tables(int q, double2 *T1, double2 *T2, const double2 *tw) {
     if (q < 128) T1[q] = tw[(q & 15) * (q >> 4)];
     if (q < 16) T2[q] = tw[8 * (q & 3) * (q >> 2)];
   }
+  template <bool FULL>
   __device__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *src, int lo, bool live,
                                  double2 (&v)[8]) {
-    w128::inverse(x, g, src, lo, live, v);
+    w128::inverse<FULL>(x, g, src, lo, live, v);
   }
+  template <bool FULL>
   __device__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *dst, int lo, bool inr,
                                  bool live) {
-    w128::forward(x, g, v, dst, lo, inr, live);
+    w128::forward<FULL>(x, g, v, dst, lo, inr, live);
   }
 };
 struct Line32 {
-  static constexpr int N = 32, LANES = 4, LP = w32::LP, MMAX = w32::MMAX12, NT2 = 1;
+  static constexpr int N = 32, LANES = 4, THREADS = 256, LP = w32::LP, MMAX = w32::MMAX12, NT2 = 1;
   __device__ static void tables(int q, double2 *T1, double2 *, const double2 *tw) {
     if (q < 32) T1[q] = tw[(q & 3) * (q >> 2)];
   }
+  template <bool FULL>
   __device__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *src, int lo, bool live,
                                  double2 (&v)[8]) {
-    w32::inverse(x, g, src, lo, live, v);
+    w32::inverse<FULL>(x, g, src, lo, live, v);
   }
+  template <bool FULL>
   __device__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *dst, int lo, bool inr,
                                  bool live) {
-    w32::forward(x, g, v, dst, lo, inr, live);
+    w32::forward<FULL>(x, g, v, dst, lo, inr, live);
   }
 };
 struct Line64 {
-  static constexpr int N = 64, LANES = 8, LP = w64::LP, MMAX = w64::MMAX24, NT2 = 1;
+  static constexpr int N = 64, LANES = 8, THREADS = 256, LP = w64::LP, MMAX = w64::MMAX24, NT2 = 1;
   __device__ static void tables(int q, double2 *T1, double2 *, const double2 *tw) {
     if (q < 64) T1[q] = tw[(q & 7) * (q >> 3)];
   }
+  template <bool FULL>
   __device__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *src, int lo, bool live,
                                  double2 (&v)[8]) {
-    w64::inverse(x, g, src, lo, live, v);
+    w64::inverse<FULL>(x, g, src, lo, live, v);
   }
+  template <bool FULL>
   __device__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *dst, int lo, bool inr,
                                  bool live) {
-    w64::forward(x, g, v, dst, lo, inr, live);
+    w64::forward<FULL>(x, g, v, dst, lo, inr, live);
   }
 };
 
-// The NTH = 256 kernel's products and field order on the lines of NTH = 128
+struct Line512 {
+  static constexpr int N = 512, LANES = 64, THREADS = 512, LP = w512::LP, MMAX = w512::MMAX192, NT2 = 64;
+  __device__ static void tables(int q, double2 *T1, double2 *T2, const double2 *tw) {
+    T1[q] = tw[(q & 63) * (q >> 6)];
+    if (q < 64) T2[q] = tw[8 * (q & 7) * (q >> 3)];
+  }
+  template <bool FULL>
+  __device__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *src, int lo, bool live,
+                                 double2 (&v)[8]) {
+    w512::inverse<FULL>(x, g, src, lo, live, v);
+  }
+  template <bool FULL>
+  __device__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *dst, int lo, bool inr,
+                                 bool live) {
+    w512::forward<FULL>(x, g, v, dst, lo, inr, live);
+  }
+};
+
+// The NTH = 256 kernel's products and field order on the lines of NTH = 512
+// (Line512: 64 lanes, 8 lines per block of eight waves), NTH = 128
 // (Line128: 16 lanes, 16 lines per block), NTH = 64 (Line64: 8 lanes, 32
-// lines) or NTH = 32 (Line32: 4 lanes, 64 lines); a block takes adjacent
+// lines), NTH = 32 (Line32: 4 lanes, 64 lines) or NTH = 16 (Line16: 2 lanes,
+// 128 lines); a block takes adjacent
 // radial nodes of one z plane.
 template <class L, bool LINEAR>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(L::THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw, const double2 *twh, FusedIO io,
                      double two_omega, double n2) {
   if (blockIdx.x == 0 && threadIdx.x == 0 && io.zl) io.zl[0] = 0.0;
-  constexpr int N = L::N, LANES = L::LANES, LINES = 256 / LANES;
+  constexpr int N = L::N, LANES = L::LANES, LINES = L::THREADS / LANES;
   __shared__ double2 S[LINES * L::LP];
   __shared__ double2 Y[LINES * N];  // [line][point i][lane]
   __shared__ double2 T1[N], T2[L::NT2], TH[N + 1];
@@ -1054,6 +1191,7 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
     const int q = threadIdx.x;
     L::tables(q, T1, T2, tw);
     if (q <= N) TH[q] = twh[q];
+    if (L::THREADS == N && q == 0) TH[N] = twh[N];
   }
   __syncthreads();
   const int z = lid / nrb, line = threadIdx.x / LANES;
@@ -1073,25 +1211,25 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
   const double r2 = live ? rsq[rr] : 1.0;
 
   double2 A[8], B[8], C[8], U[8], V[8], T[8];
-  L::inverse(x, g, in(0), lo, live, A);  // rur
-  L::inverse(x, g, in(1), lo, live, B);  // rup
-  L::inverse(x, g, in(2), lo, live, C);  // uz
+  L::template inverse<false>(x, g, in(0), lo, live, A);  // rur
+  L::template inverse<false>(x, g, in(1), lo, live, B);  // rup
+  L::template inverse<false>(x, g, in(2), lo, live, C);  // uz
   // oz: U = rup oz, V = rur oz
-  L::inverse(x, g, in(5), lo, live, T);
+  L::template inverse<false>(x, g, in(5), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     U[i] = make_double2(B[i].x * T[i].x, B[i].y * T[i].y);
     V[i] = make_double2(A[i].x * T[i].x, A[i].y * T[i].y);
   }
   // ror: Y = uz ror - rur oz (to LDS); V = rup ror
-  L::inverse(x, g, in(3), lo, live, T);
+  L::template inverse<false>(x, g, in(3), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     ys[LANES * i] = make_double2(C[i].x * T[i].x - V[i].x, C[i].y * T[i].y - V[i].y);
     V[i] = make_double2(B[i].x * T[i].x, B[i].y * T[i].y);
   }
   // rop: X = rup oz - uz rop in U; Z = (rur rop - rup ror) / r^2 in V
-  L::inverse(x, g, in(4), lo, live, T);
+  L::template inverse<false>(x, g, in(4), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     U[i] = make_double2(U[i].x - C[i].x * T[i].x, U[i].y - C[i].y * T[i].y);
@@ -1102,29 +1240,29 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
 #pragma unroll
     for (int i = 0; i < 8; i++) U[i] = make_double2(U[i].x + two_omega * B[i].x, U[i].y + two_omega * B[i].y);
   }
-  L::forward(x, g, U, out(0), lo, inr, live);
+  L::template forward<false>(x, g, U, out(0), lo, inr, live);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     T[i] = ys[LANES * i];
     if (LINEAR) T[i] = make_double2(T[i].x - two_omega * A[i].x, T[i].y - two_omega * A[i].y);
   }
-  L::forward(x, g, T, out(1), lo, inr, live);
+  L::template forward<false>(x, g, T, out(1), lo, inr, live);
   if (LINEAR) {
     // W: N_z = Z - W
-    L::inverse(x, g, in(9), lo, live, T);
+    L::template inverse<false>(x, g, in(9), lo, live, T);
 #pragma unroll
     for (int i = 0; i < 8; i++) V[i] = make_double2(V[i].x - T[i].x, V[i].y - T[i].y);
   }
-  L::forward(x, g, V, out(2), lo, inr, live);
+  L::template forward<false>(x, g, V, out(2), lo, inr, live);
   // rbr, rbp: A = rur rbr + rup rbp
-  L::inverse(x, g, in(6), lo, live, T);
+  L::template inverse<false>(x, g, in(6), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) A[i] = make_double2(A[i].x * T[i].x, A[i].y * T[i].y);
-  L::inverse(x, g, in(7), lo, live, T);
+  L::template inverse<false>(x, g, in(7), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) A[i] = make_double2(A[i].x + B[i].x * T[i].x, A[i].y + B[i].y * T[i].y);
   // bz: N_b = -(T / r^2 + uz bz) (+ Nbar^2 uz)
-  L::inverse(x, g, in(8), lo, live, T);
+  L::template inverse<false>(x, g, in(8), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     const double vr = A[i].x / r2 + C[i].x * T[i].x, vi = A[i].y / r2 + C[i].y * T[i].y;
@@ -1132,11 +1270,142 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
     if (LINEAR) nb = make_double2(nb.x + n2 * C[i].x, nb.y + n2 * C[i].y);
     A[i] = nb;
   }
-  L::forward(x, g, A, out(3), lo, inr, live);
+  L::template forward<false>(x, g, A, out(3), lo, inr, live);
+}
+
+struct Line256 {
+  static constexpr int N = 256, LANES = 32, LP = w256::LP, MMAX = w256::MMAX96, NT2 = 32;
+  __device__ static void tables(int q, double2 *T1, double2 *T2, const double2 *tw) {
+    if (q < 256) T1[q] = tw[(q & 31) * (q >> 5)];
+    if (q < 32) T2[q] = tw[8 * (q & 3) * (q >> 2)];
+  }
+  template <bool FULL>
+  __device__ static void inverse(const w256::Ctx &x, const KGrid &g, const double2 *src, int lo, bool live,
+                                 double2 (&v)[8]) {
+    w256::inverse<FULL>(x, g, src, lo, live, v);
+  }
+  template <bool FULL>
+  __device__ static void forward(const w256::Ctx &x, const KGrid &g, const double2 (&v)[8], double2 *dst, int lo, bool inr,
+                                 bool live) {
+    w256::forward<FULL>(x, g, v, dst, lo, inr, live);
+  }
+};
+
+// Small grids: the register kernels' lines, a wave a field.  Each wave takes
+// its field of the block's 64 / LANES lines to physical space and leaves the
+// points in LDS, where the first four waves form one product each, at the
+// same points as their lanes' own, and transform it forward.  The ten inverse
+// and four forward transforms that a line of the register kernels runs one
+// after the other are here one of each, in return for a fourth of the work
+// per wave.
+template <class L, bool LINEAR, bool FULL>
+__global__ void __launch_bounds__(LINEAR ? 640 : 576)
+k_fused_products_wide(KGrid g, const double *__restrict__ rsq, const double2 *tw, const double2 *twh, FusedIO io,
+                      double two_omega, double n2) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && io.zl) io.zl[0] = 0.0;
+  constexpr int N = L::N, LANES = L::LANES, LINES = 64 / LANES, NF = LINEAR ? 10 : 9;
+  constexpr int SL = LINES * L::LP;  // >= 512: the exchanges of a wave, then its 8 points a lane
+  static_assert(SL >= 512, "a field's points");
+  __shared__ double2 S[NF * SL];
+  __shared__ double2 T1[N], T2[L::NT2], TH[N + 1];
+  const int nrb = (g.ndimr + LINES - 1) / LINES;
+  const int lid = xcd_logical(nrb * g.ndimx);
+  if (lid < 0) return;
+  {
+    const int q = threadIdx.x;
+    if (q < 512) L::tables(q, T1, T2, tw);
+    if (q <= N) TH[q] = twh[q];
+  }
+  __syncthreads();
+  const int z = lid / nrb, lane = threadIdx.x & 63, line = lane / LANES;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rr = (lid % nrb) * LINES + line;
+  const bool inr = rr < g.ndimr, live = rr < g.nr;
+  w256::Ctx x;
+  x.t1 = T1;
+  x.t2 = T2;
+  x.th = TH;
+  x.s = S + w * SL + line * L::LP;
+  x.b = lane % LANES;
+  const size_t off = (size_t)(rr - line) + (size_t)g.ndimr * g.ndimth * z;  // same for the block
+  const int lo = inr ? line : 0;
+  double2 v[8];
+  L::template inverse<FULL>(x, g, io.in[w] + off, lo, live, v);
+  w256::wave_sync();
+#pragma unroll
+  for (int i = 0; i < 8; i++) S[w * SL + 64 * i + lane] = v[i];
+  __syncthreads();
+  auto F = [&](int q, int i) { return S[q * SL + 64 * i + lane]; };
+  if (w < 4) {
+    const double r2 = live ? rsq[rr] : 1.0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if (w == 0) {
+        const double2 B = F(1, i), C = F(2, i), E = F(4, i), O = F(5, i);
+        v[i] = make_double2(B.x * O.x - C.x * E.x, B.y * O.y - C.y * E.y);
+        if (LINEAR) v[i] = make_double2(v[i].x + two_omega * B.x, v[i].y + two_omega * B.y);
+      } else if (w == 1) {
+        const double2 A = F(0, i), C = F(2, i), D = F(3, i), O = F(5, i);
+        v[i] = make_double2(C.x * D.x - A.x * O.x, C.y * D.y - A.y * O.y);
+        if (LINEAR) v[i] = make_double2(v[i].x - two_omega * A.x, v[i].y - two_omega * A.y);
+      } else if (w == 2) {
+        const double2 A = F(0, i), B = F(1, i), D = F(3, i), E = F(4, i);
+        v[i] = make_double2((A.x * E.x - B.x * D.x) / r2, (A.y * E.y - B.y * D.y) / r2);
+        if (LINEAR) {
+          const double2 W = F(9, i);
+          v[i] = make_double2(v[i].x - W.x, v[i].y - W.y);
+        }
+      } else {
+        const double2 A = F(0, i), B = F(1, i), C = F(2, i), P = F(6, i), Q = F(7, i), R = F(8, i);
+        const double tr = A.x * P.x + B.x * Q.x, ti = A.y * P.y + B.y * Q.y;
+        v[i] = make_double2(-(tr / r2 + C.x * R.x), -(ti / r2 + C.y * R.y));
+        if (LINEAR) v[i] = make_double2(v[i].x + n2 * C.x, v[i].y + n2 * C.y);
+      }
+    }
+  }
+  __syncthreads();
+  if (w < 4) L::template forward<FULL>(x, g, v, io.out[w] + off, lo, inr, live);
 }
 
 bool fused_products_supported(const mlg_ctx *c) {
-  return fft4_length(c->g.nth) || c->fp.n;
+  return fused_line_length(c->g.nth) || c->fp.n;
+}
+
+// One wave a field or a line's fields in one wave.  Truncations past 3/8 of
+// NTH (FULL: both terms in the merge) spill in the kernels that hold all
+// fields, so they always go a wave a field: at 256 x NTH x 256, NTH = 32, 64,
+// 128 163, 335, 777 us against 295, 541, 884; 128 x 512 x 128 1019 against
+// 898.  Others do while the blocks fill the chip at most three times (one
+// block a CU): at NR = 64, NX = 32 8.1 us against 20.3 (NTH = 32, 160 blocks),
+// 14.3 against 20.4 (64, 288) and 25.2 against 28.8 (128, 544), but 33.6
+// against 28.5 at 128 x 64 x 64 (1088) and 234 against 150 at 256 x 64 x 256.
+template <class L, bool LINEAR>
+static int launch_line(mlg_ctx *c, const FusedIO &io, double two_omega, double n2) {
+  KGrid g = kgrid(c);
+  constexpr int wl = 64 / L::LANES;
+  const int wide = (g.ndimr + wl - 1) / wl * g.ndimx;
+  const bool full = g.ntchopdim > L::MMAX;
+  if (full) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_wide<L, LINEAR, true>), dim3(xcd_grid(wide)),
+                       dim3(LINEAR ? 640 : 576), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
+  } else if constexpr (L::MMAX > 0) {
+    if (wide <= 3 * 256)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_wide<L, LINEAR, false>), dim3(xcd_grid(wide)),
+                         dim3(LINEAR ? 640 : 576), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
+    else if constexpr (L::N == 256)
+      hipLaunchKernelGGL(k_fused_products_256<LINEAR>, dim3(xcd_grid((g.ndimr + 7) / 8 * g.ndimx)), dim3(256), 0,
+                         c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
+    else
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_reg<L, LINEAR>),
+                         dim3(xcd_grid((g.ndimr + L::THREADS / L::LANES - 1) / (L::THREADS / L::LANES) * g.ndimx)),
+                         dim3(L::THREADS), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
+  }
+  MLG_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+template <class L>
+static int launch_lines(mlg_ctx *c, const FusedIO &io, double two_omega, double n2, int linear) {
+  return linear ? launch_line<L, true>(c, io, two_omega, n2) : launch_line<L, false>(c, io, two_omega, n2);
 }
 
 int launch_fused_products(mlg_ctx *c, const double2 *const in[10], double2 *const out[4], double two_omega, double n2,
@@ -1148,52 +1417,20 @@ int launch_fused_products(mlg_ctx *c, const double2 *const in[10], double2 *cons
   io.zl = zl;
   // PFP traffic: 9 (10) live input fields read, 4 written
   KScope ks(c, K_PRODUCTS, 16.0 * g.nr * g.ntchopdim * (double)g.nx * ((linear ? 10 : 9) + 4));
-#define L_REG(L_)                                                                                                    \
-  do {                                                                                                               \
-    dim3 grid(xcd_grid((g.ndimr + 256 / L_::LANES - 1) / (256 / L_::LANES) * g.ndimx));                             \
-    if (linear)                                                                                                      \
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_reg<L_, true>), grid, dim3(256), 0, c->stream, g, c->d.r,  \
-                         c->d.tw_t, c->d.tw_h, io, two_omega, n2);                                                   \
-    else                                                                                                             \
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_reg<L_, false>), grid, dim3(256), 0, c->stream, g, c->d.r, \
-                         c->d.tw_t, c->d.tw_h, io, two_omega, n2);                                                   \
-    MLG_CHECK_HIP(hipGetLastError());                                                                                \
-    return 0;                                                                                                        \
-  } while (0)
-  if (g.nth == 128 && g.ntchopdim <= Line128::MMAX) L_REG(Line128);
-  if (g.nth == 64 && g.ntchopdim <= Line64::MMAX) L_REG(Line64);
-  if (g.nth == 32 && g.ntchopdim <= Line32::MMAX) L_REG(Line32);
-#undef L_REG
-  if (g.nth == 256 && g.ntchopdim <= w256::MMAX96) {
-    dim3 grid(xcd_grid((g.ndimr + 7) / 8 * g.ndimx));
-    if (linear)
-      hipLaunchKernelGGL(k_fused_products_256<true>, grid, dim3(256), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io,
-                         two_omega, n2);
-    else
-      hipLaunchKernelGGL(k_fused_products_256<false>, grid, dim3(256), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h,
-                         io, two_omega, n2);
-    MLG_CHECK_HIP(hipGetLastError());
-    return 0;
+  switch (g.nth) {
+    case 2: return launch_lines<LineTiny<2>>(c, io, two_omega, n2, linear);
+    case 4: return launch_lines<LineTiny<4>>(c, io, two_omega, n2, linear);
+    case 8: return launch_lines<LineTiny<8>>(c, io, two_omega, n2, linear);
+    case 16: return launch_lines<Line16>(c, io, two_omega, n2, linear);
+    case 32: return launch_lines<Line32>(c, io, two_omega, n2, linear);
+    case 64: return launch_lines<Line64>(c, io, two_omega, n2, linear);
+    case 128: return launch_lines<Line128>(c, io, two_omega, n2, linear);
+    case 256: return launch_lines<Line256>(c, io, two_omega, n2, linear);
+    case 512: return launch_lines<Line512>(c, io, two_omega, n2, linear);
+    default: break;
   }
   if (c->fp.n) return launch_fused_any(c, io, two_omega, n2, linear);
-  dim3 grid(xcd_grid((g.ndimr + FP - 1) / FP * g.ndimx));
-#define L_FP(a_, b_)                                                                                                \
-  hipLaunchKernelGGL((k_fused_products<a_, b_>), grid, dim3(256), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, \
-                     two_omega, n2, linear)
-  switch (g.nth) {
-    case 2: L_FP(2, 1); break;
-    case 4: L_FP(4, 1); break;
-    case 8: L_FP(8, 1); break;
-    case 16: L_FP(16, 1); break;
-    case 64: L_FP(8, 8); break;
-    case 32: L_FP(16, 2); break;
-    case 128: L_FP(16, 8); break;
-    case 256: L_FP(16, 16); break;
-    default: return MLG_E_ARG;
-  }
-#undef L_FP
-  MLG_CHECK_HIP(hipGetLastError());
-  return 0;
+  return MLG_E_ARG;
 }
 
 }  // namespace mlg

@@ -320,7 +320,9 @@ static inline bool fft4_length(int n) { return n >= 2 && n <= 256 && (n & (n - 1
 int fft_any_setup(int n, FftAny *f);  // allocates f's device tables
 int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd);
 int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd);
-// fused products (k_fused_any.hip); f->n = 0 where the length has no plan
+// theta lengths with a register-resident products kernel (k_fused.hip)
+static inline bool fused_line_length(int n) { return n >= 2 && n <= 512 && (n & (n - 1)) == 0; }
+// fused products elsewhere (k_fused_any.hip); f->n = 0 where the length has no plan
 struct FusedIO;
 int fused_any_setup(int nth, FusedAny *f);
 int launch_fused_any(mlg_ctx *c, const FusedIO &io, double two_omega, double n2, int linear);

@@ -1,5 +1,5 @@
-"""The fused products at theta lengths of k_fused_any (FORCE with its linear
-terms, NONLIN without) against the FP64 oracle: every radix of the last stage
+"""The fused products (FORCE with its linear terms, NONLIN without) at theta
+lengths of k_fused_any against the FP64 oracle: every radix of the last stage
 (6, 5, 4, 3, 2), middle stages, a direct stage (factors 11 .. 61), both
 truncations in use (a third and two thirds of NTH), radial counts that leave
 part of a block empty; and lengths without a plan (49, 289, 608), which take
@@ -16,16 +16,27 @@ from test_gpu_parity import TOL, Pair, state
 
 pytestmark = pytest.mark.gpu
 
-LENGTHS = [3, 5, 6, 7, 9, 10, 12, 14, 20, 22, 45, 49, 66, 81, 90, 100, 104, 126, 153, 204, 289, 306, 310, 366, 384, 512, 608, 640, 768]
+LENGTHS = [2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 20, 22, 32, 45, 49, 66, 81, 90, 100, 104, 126, 153, 204, 289, 306, 310, 366, 384, 512, 608, 640, 768]
 
 
 @pytest.mark.parametrize("nth", LENGTHS)
 @pytest.mark.parametrize("full", [False, True], ids=["third", "twothirds"])
 def test_right_hand_sides(nth, full):
-    nr = 36 if nth < 100 else 12
-    nrchop = 24 if nth < 100 else 8
     ntc = min(max(1, 2 * nth // 3 if full else nth // 3 + 1), nth)
-    p = Pair(dict(CFG1, nr=nr, nth=nth, nx=6, nrchop=nrchop, ntchop=ntc, nxchop=3))
+    nr, nrchop = (36, 24) if nth < 100 else (12, 8)
+    compare(dict(CFG1, nr=nr, nth=nth, nx=6, nrchop=nrchop, ntchop=ntc, nxchop=3))
+
+
+# more than 768 blocks of a wave a field (64, 32, .. 1 of the 15 lines of a plane each)
+@pytest.mark.parametrize("nth,nx", [(8, 800), (16, 800), (32, 800), (64, 400), (128, 200), (256, 100), (512, 54)])
+@pytest.mark.parametrize("full", [False, True], ids=["third", "twothirds"])
+def test_right_hand_sides_on_large_grids(nth, nx, full):
+    ntc = 2 * nth // 3 if full else nth // 3
+    compare(dict(CFG1, nr=12, nth=nth, nx=nx, nrchop=8, ntchop=ntc, nxchop=3))
+
+
+def compare(cfg):
+    p = Pair(cfg)
     try:
         st = state(p, 1e-3)
         outs = [p.empty() for _ in range(3)]
