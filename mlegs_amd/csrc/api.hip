@@ -1139,39 +1139,41 @@ extern "C" int mlg_energy(const mlg_field *psi, const mlg_field *chi, const mlg_
   MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
   MLG_CHECK_HIP(hipMemcpy(&bln, b->ln, sizeof(double), hipMemcpyDeviceToHost));
   if (bln != 0.0) return 13;
+  if (psi->space != MLG_FFF || chi->space != MLG_FFF) return 3;
+  if (b->space != MLG_FFF) return 2;
+  constexpr int NF = 5;
   Temps T(c);
-  mlg_field *w1 = T.get(), *w2 = T.get(), *w3 = T.get();
+  mlg_field *zero = T.get(), *ln2 = T.buffer(), *a = T.buffer(), *d2 = T.buffer(), *dh = T.buffer(), *t[NF];
+  for (auto &q : t) q = T.buffer();
   RET(T.ready());
   const int nt = G.ntchop, nxc = G.nxchop, nxd = G.nxchopdim;
   const size_t na = (size_t)nt * nxd;
   double *dall = c->d.red;  // [4][nt*nxd]
   RET(launch_zero(c, (double2 *)dall, (long)(4 * na / 2 + 1)));
+  RET(launch_set_ln(c, ln2->ln, psi->ln, 2.0, 0.0));
   RET(mlg_chopset(c, 3));
-  int rc = copy0(w1, psi);
-  if (!rc) rc = launch_set_ln(c, w1->ln, psi->ln, 2.0, 0.0);
-  if (!rc) rc = mlg_delsqh(w1, w2);
-  if (!rc) rc = launch_set_ln(c, w1->ln, nullptr, 0, 0);
-  if (!rc) rc = launch_set_ln(c, w2->ln, nullptr, 0, 0);
-  if (!rc) rc = mlg_rtran(w1, 1);
-  if (!rc) rc = mlg_rtran(w2, 1);
-  if (!rc) rc = launch_energy_terms(c, w1->e, w2->e, 0, dall);
-  if (!rc) rc = mlg_del2(chi, w1);
-  if (!rc) rc = mlg_delsqh(chi, w2);
-  if (!rc) rc = launch_set_ln(c, w1->ln, nullptr, 0, 0);
-  if (!rc) rc = launch_set_ln(c, w2->ln, nullptr, 0, 0);
-  if (!rc) rc = mlg_rtran(w1, 1);
-  if (!rc) rc = mlg_rtran(w2, 1);
-  if (!rc) rc = launch_energy_terms(c, w1->e, w2->e, 0, dall + na);
-  if (!rc) rc = copy0(w3, b);
-  if (!rc) rc = launch_set_ln(c, w3->ln, nullptr, 0, 0);
-  if (!rc) rc = mlg_rtran(w3, 1);
-  if (!rc) rc = launch_energy_terms(c, w3->e, w2->e, 0, dall + 2 * na);
-  if (!rc) rc = launch_energy_terms(c, w3->e, nullptr, 1, dall + 3 * na);
+  // psi, DELSQH(psi, 2 LN), DEL2(chi), DELSQH(chi) and b, without their LN,
+  // share one backward launch and one copy to the host
+  const double2 *in[NF] = {psi->e, a->e, d2->e, dh->e, b->e};
+  const double *ln[NF];
+  double2 *pff[NF];
+  for (int q = 0; q < NF; q++) {
+    ln[q] = zero->ln;
+    pff[q] = t[q]->e;
+  }
+  int rc = launch_delsqh(c, psi->e, ln2->ln, a->e, a->ln);
+  if (!rc) rc = mlg_del2(chi, d2);
+  if (!rc) rc = mlg_delsqh(chi, dh);
+  if (!rc) rc = launch_rtran_bwd_n(c, NF, in, ln, pff);
+  if (!rc) rc = launch_energy_terms(c, pff[0], pff[1], 0, dall);
+  if (!rc) rc = launch_energy_terms(c, pff[2], pff[3], 0, dall + na);
+  if (!rc) rc = launch_energy_terms(c, pff[4], pff[3], 0, dall + 2 * na);
+  if (!rc) rc = launch_energy_terms(c, pff[4], nullptr, 1, dall + 3 * na);
   mlg_chopset(c, -3);
   RET(rc);
   std::vector<double> h(4 * na);
   MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  MLG_CHECK_HIP(hipMemcpy(h.data(), dall, sizeof(double) * 4 * na, hipMemcpyDeviceToHost));
+  MLG_CHECK_HIP(hipMemcpy(h.data(), dall, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
   // fold +-k into the NXCHOP non-negative wavenumbers (PRODCT_MK_HALFK)
   auto fold = [&](const double *all, double *out) {
     for (int i = 0; i < nt * nxc; i++) out[i] = 0.0;

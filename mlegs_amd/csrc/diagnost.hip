@@ -5,10 +5,11 @@
 //
 // The fields are formed by the library's operators at NRCHOP+3; the
 // integrals are the first FFF coefficient (INTEG, src/mod_scalar3.f90:
-// 312-353) or Gauss sums over PFF columns (PRODCT :398-468, the per-(m, k)
-// product launch of the energy diagnostics); the two physical-space
-// products of CALCXY (ABSVEC2 :2050-2099, MULRCOSTH / MULRSINTH / MULR2
-// :2102-2225) are pointwise kernels on PPP.
+// 312-353), Gauss sums over PFF columns (PRODCT :398-468, the per-(m, k)
+// product launch of the energy diagnostics) or sums over the physical grid
+// (CALCXY's, of ABSVEC2 :2050-2099 times MULRCOSTH / MULRSINTH / MULR2's
+// factors :2102-2225).
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -24,204 +25,178 @@ using namespace mlg;
 
 namespace mlg {
 
-// ABSVEC2: a = ((u^2 + v^2) / r^2 + w^2) / (1-x)^2 on each theta sub-grid
-// (the real and imaginary slots), r < NR, theta < NTH; a may be w
-__global__ void __launch_bounds__(256) k_absvec2(KGrid g, const double2 *u, const double2 *v, const double2 *w, double2 *a,
-                                                 const double *__restrict__ r2, const double *__restrict__ x) {
-  const long n = (long)g.nr * g.nth * g.ndimx;
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256L) {
-    const int r = (int)(i % g.nr);
-    const long rest = i / g.nr;
-    const int j = (int)(rest % g.nth), z = (int)(rest / g.nth);
-    const size_t at = (size_t)r + (size_t)g.ndimr * ((size_t)j + (size_t)g.ndimth * z);
-    const double2 uu = u[at], vv = v[at], ww = w[at];
-    const double om = 1 - x[r], f = om * om;
-    const double aaa = ((uu.x * uu.x + vv.x * vv.x) / r2[r] + ww.x * ww.x);
-    const double bbb = ((uu.y * uu.y + vv.y * vv.y) / r2[r] + ww.y * ww.y);
-    a[at] = make_double2(aaa / f, bbb / f);
-  }
-}
-
-// a(r, theta, z) times fr(r, theta) (real slot) and fi(r, theta) (imaginary
-// slot), r < NR, theta < NTH; fr, fi [NTH][NR]
-__global__ void __launch_bounds__(256) k_mul_rtheta(KGrid g, double2 *a, const double *__restrict__ fr,
-                                                    const double *__restrict__ fi) {
-  const long n = (long)g.nr * g.nth * g.ndimx;
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256L) {
-    const int r = (int)(i % g.nr);
-    const long rest = i / g.nr;
-    const int j = (int)(rest % g.nth), z = (int)(rest / g.nth);
-    const size_t at = (size_t)r + (size_t)g.ndimr * ((size_t)j + (size_t)g.ndimth * z);
-    const size_t t = (size_t)r + (size_t)g.nr * j;
-    const double2 v = a[at];
-    a[at] = make_double2(fr[t] * v.x, fi[t] * v.y);
-  }
-}
-
-static int blocks_ppp(const KGrid &g) {
-  const long n = (long)g.nr * g.nth * g.ndimx;
-  return (int)std::min<long>((n + 255) / 256, 4096);
-}
-
-// INTEG: 4 pi ZLEN ELL^2 Re(f(0,0,0)) NORM(0, m=0) of an FFF field
-static int integ(mlg_ctx *c, const mlg_field *f, double *out) {
-  if (f->space != MLG_FFF) return 2;
-  double2 e0;
-  MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  MLG_CHECK_HIP(hipMemcpy(&e0, f->e, sizeof(double2), hipMemcpyDeviceToHost));
-  const double pi = 3.14159265358979323846;
-  *out = 4.0 * pi * c->g.zlen * c->g.ell2 * e0.x * c->g.norm[0];
-  return 0;
-}
-
-// PRODCT: 2 pi ZLEN ELL^2 sum over r, m, k of w_r Re(a conj b), the modes
-// m >= 1 twice (the per-(m, k) sums with m = 0 halved, added up)
-static int prodct(mlg_ctx *c, const mlg_field *a, const mlg_field *b, double *out) {
-  const Grid &G = c->g;
-  const size_t na = (size_t)G.ntchop * G.nxchopdim;
-  RET(launch_energy_terms(c, a->e, b->e, 0, c->d.red));
-  std::vector<double> h(na);
-  MLG_CHECK_HIP(hipMemcpyAsync(h.data(), c->d.red, sizeof(double) * na, hipMemcpyDeviceToHost, c->stream));
-  MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  double s = 0.0;
-  for (double v : h) s = s + v;
-  *out = s;
-  return 0;
-}
-
-// CALCAT1 (src/mod_scalar3.f90:286-310): per k, sum over n < NRCHOP of
-// f(n, m=0, k) AT1(n); returns |value at k = 0| and max - min of |value|
-static int calcat1(mlg_ctx *c, const mlg_field *f, double *at0, double *spread) {
-  const Grid &G = c->g;
-  const int nn = G.nrchop, nxd = G.nxchopdim;
-  std::vector<double2> col((size_t)nn * nxd);
-  MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
-  MLG_CHECK_HIP(hipMemcpy2D(col.data(), sizeof(double2) * nn, f->e, sizeof(double2) * (size_t)G.nrchopdim * G.ntchopdim,
-                            sizeof(double2) * nn, nxd, hipMemcpyDeviceToHost));
-  double mx = -1.0, mn = 1e300;
-  for (int k = 0; k < nxd; k++) {
-    double re = 0.0, im = 0.0;
-    for (int n = 0; n < nn; n++) {
-      re = re + col[(size_t)nn * k + n].x * G.at1[n];
-      im = im + col[(size_t)nn * k + n].y * G.at1[n];
+// ABSVEC2, ((u^2 + v^2) / r^2 + w^2) / (1-x)^2, summed over z per (r, theta):
+// out[j][r], the real and the imaginary theta sub-grid.  Block: 64 radial nodes x 4 ranges of z at one theta.
+__global__ void __launch_bounds__(256) k_absvec2_sum(KGrid g, const double2 *__restrict__ u, const double2 *__restrict__ v,
+                                                     const double2 *__restrict__ w, const double *__restrict__ r2,
+                                                     const double *__restrict__ x, double2 *__restrict__ out) {
+  __shared__ double2 S[4][64];
+  const int rl = threadIdx.x & 63, q = threadIdx.x >> 6, r = blockIdx.x * 64 + rl, j = blockIdx.y;
+  double2 s = make_double2(0.0, 0.0);
+  if (r < g.nr) {
+    const double om = 1 - x[r], f = om * om, rr = r2[r];
+    for (int z = q; z < g.nx; z += 4) {
+      const size_t at = (size_t)r + (size_t)g.ndimr * ((size_t)j + (size_t)g.ndimth * z);
+      const double2 uu = u[at], vv = v[at], ww = w[at];
+      s.x += ((uu.x * uu.x + vv.x * vv.x) / rr + ww.x * ww.x) / f;
+      s.y += ((uu.y * uu.y + vv.y * vv.y) / rr + ww.y * ww.y) / f;
     }
-    const double a = std::hypot(re, im);
-    if (k == 0) *at0 = a;
-    mx = std::max(mx, a);
-    mn = std::min(mn, a);
   }
-  *spread = mx - mn;
-  return 0;
+  S[q][rl] = s;
+  __syncthreads();
+  if (q == 0 && r < g.nr)
+    out[(size_t)r + (size_t)g.nr * j] = make_double2(S[0][rl].x + S[1][rl].x + S[2][rl].x + S[3][rl].x,
+                                                     S[0][rl].y + S[1][rl].y + S[2][rl].y + S[3][rl].y);
 }
 
+// Inputs of k_it1_values; every sum of the section in one launch.
+struct It1 {
+  const double2 *dp, *dc, *ang;  // FFF: DELSQH(psi) = -OZ/(1-x)^2, DELSQH(chi) = -UZ/(1-x)^2, XXDX(psi)
+  const double2 *f[2];             // psi, chi
+  const double *at1, *x, *w, *r2, *terms;  // terms: the PRODCTs' per-(m, k) sums, 3 x na
+  const double2 *abs;              // ABSVEC2 summed over z, [theta][r]
+  double p00;                      // P_0^0, normalised
+  int na, nn;                      // nn: NRCHOP
+  double minc;
+};
+// VALVOR, VALZMO, the INTEG_P sum, 3 PRODCTs, 4 moments (1, x, y, r^2), then
+// CALCAT1's |value| per k of psi and of chi; a block of 1024 threads each
+constexpr int IT1_AT1 = 10;
+__global__ void __launch_bounds__(1024) k_it1_values(KGrid g, It1 v, double *out) {
+  __shared__ double2 S[1024];
+  const int t = threadIdx.x, q = blockIdx.x;
+  double2 s = make_double2(0.0, 0.0);
+  if (q < 2) {
+    if (t == 0) s.x = -(q == 0 ? v.dp : v.dc)[0].x;
+  } else if (q == 2) {
+    // the first NR stored coefficients in storage order
+    for (int i = t; i < g.nr; i += 1024) {
+      const double om = 1 - v.x[i];
+      s.x += v.ang[i].x / (om * om) * v.w[i];
+    }
+  } else if (q < 6) {
+    for (int i = t; i < v.na; i += 1024) s.x += v.terms[(size_t)(q - 3) * v.na + i];
+  } else if (q < IT1_AT1) {
+    // The (0, 0, 0) coefficient of ABSVEC2 times the factor: HORFFT's m = 0
+    // and VERFFT's k = 0 are means, RTRAN's n = 0 the Gauss sum with P_0^0.
+    // theta = 2 pi j / NTH in the real slots, 2 pi (j + 1/2) / NTH in the imaginary ones
+    const double pi = 3.14159265358979323846;
+    for (long i = t; i < (long)g.nr * g.nth; i += 1024) {
+      const int r = (int)(i % g.nr), j = (int)(i / g.nr);
+      double2 a = v.abs[i];
+      const double rad = q == 6 ? 1.0 : (q == 9 ? v.r2[r] : sqrt(v.r2[r]));
+      if (q == 7 || q == 8) {
+        const double thr = 2 * pi / v.minc / g.nth * j, thi = 2 * pi / v.minc / g.nth * (j + 0.5);
+        a.x *= q == 7 ? cos(thr) : sin(thr);
+        a.y *= q == 7 ? cos(thi) : sin(thi);
+      }
+      s.x += v.w[r] * rad * (a.x + a.y);
+    }
+  } else {
+    const int k = (q - IT1_AT1) % g.nxchopdim, fi = (q - IT1_AT1) / g.nxchopdim;
+    const double2 *col = v.f[fi] + (size_t)g.nrchopdim * g.ntchopdim * k;
+    for (int n = t; n < v.nn; n += 1024) {
+      s.x += col[n].x * v.at1[n];
+      s.y += col[n].y * v.at1[n];
+    }
+  }
+  S[t] = s;
+  __syncthreads();
+  for (int h = 512; h > 0; h >>= 1) {
+    if (t < h) S[t] = make_double2(S[t].x + S[t + h].x, S[t].y + S[t + h].y);
+    __syncthreads();
+  }
+  if (t) return;
+  if (q >= IT1_AT1) out[q] = hypot(S[0].x, S[0].y);
+  else if (q >= 6) out[q] = S[0].x * v.p00 / (2.0 * g.nth * g.nx);
+  else out[q] = S[0].x;
+}
+
+// The section without a wait or a host table on the way: every integral ends
+// in k_it1_values, whose results come in one copy.  CALCXY's four integrals
+// are sums of ABSVEC2 over the physical grid with their factors, in place of
+// four fields transformed for one coefficient each (MULRCOSTH / MULRSINTH /
+// MULR2 and INTEG), and the eight fields that leave FFF share one backward
+// launch.  At 128x64x64 the section with the energies and ENEMON, which share
+// launches in the same way, takes 0.39 ms where they took 1.86.
 static int diagnost_it1(const mlg_field *psi, const mlg_field *chi, double *out) {
   mlg_ctx *c = psi->ctx;
   const Grid &G = c->g;
   const double pi = 3.14159265358979323846;
+  constexpr int NF = 8;
   Temps T(c);
-  mlg_field *rur = T.get(), *rup = T.get(), *uzh = T.get(), *ror = T.get(), *rop = T.get(), *ozh = T.get();
+  mlg_field *ror = T.buffer(), *rop = T.buffer(), *oz = T.buffer(), *a = T.buffer(), *d2c = T.buffer(), *dc = T.buffer(),
+            *dp = T.buffer(), *ang = T.buffer(), *m1 = T.buffer(), *t[NF];
+  for (auto &q : t) q = T.buffer();
   RET(T.ready());
-  // PC2VEL(..., 'H'): only UZ/(1-x)^2 = -DELSQH(chi) is read (INTEG); the
-  // minus sign takes the elements, not LN
-  RET(mlg_delsqh(chi, uzh));
-  RET(launch_negate(c, uzh->e, c->n_fff));
-  // PC2VOR(..., 'H'): ROR, ROP of PC2VOR and OZ/(1-x)^2 = -DELSQH(psi)
-  RET(mlg_pc2vor(psi, chi, ror, rop, ozh));
-  RET(mlg_delsqh(psi, ozh));
-  RET(launch_negate(c, ozh->e, c->n_fff));
-  RET(integ(c, ozh, &out[0]));  // VALVOR
-  RET(integ(c, uzh, &out[1]));  // VALZMO
+  // PC2VOR(..., 'H'): ROR, ROP of PC2VOR, OZ/(1-x)^2 = -DELSQH(psi);
+  // PC2VEL(..., 'H'): only UZ/(1-x)^2 = -DELSQH(chi) is read (INTEG)
+  RET(mlg_pc2vor(psi, chi, ror, rop, ang));
+  RET(mlg_delsqh(psi, dp));  // LN 0
+  RET(mlg_delsqh(chi, dc));
+  RET(launch_set_ln(c, m1->ln, psi->ln, 2.0, 0.0));
+  RET(launch_delsqh(c, psi->e, m1->ln, a->e, a->ln));
+  RET(mlg_del2(chi, d2c));
   // VALANG = -INTEG_P(XXDX(psi with LN = 0)).  INTEG_P (src/mod_march.f90:
   // 3649-3682) sums Re(F%E(:NR,1,1)) w / (1-x)^2 of its FFF argument: the
   // first NR stored coefficients in storage order (past the m = 0, k = 0
   // column when NRCHOPDIM < NR), as the reference reads them
-  RET(copy_field(rur, psi));
-  RET(launch_set_ln(c, rur->ln, nullptr, 0.0, 0.0));
-  RET(mlg_xxdx(rur, rup));
-  {
-    std::vector<double2> e((size_t)G.nr);
-    MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
-    MLG_CHECK_HIP(hipMemcpy(e.data(), rup->e, sizeof(double2) * G.nr, hipMemcpyDeviceToHost));
-    double dot = 0.0;
-    for (int i = 0; i < G.nr; i++) {
-      const double om = 1 - G.x[i];
-      dot = dot + e[i].x / (om * om) * G.w[i];
-    }
-    out[4] = -(2.0 * pi * G.zlen * G.ell2 * dot);
-  }
+  RET(launch_band3(c, 1, psi->e, dp->ln, ang->e, ang->ln));
+  // OZH (1-x)^2 = OZ, but for its sign, which ABSVEC2 squares
+  RET(launch_band3(c, 0, dp->e, dp->ln, m1->e, m1->ln));
+  RET(launch_band3(c, 0, m1->e, m1->ln, oz->e, oz->ln));
+  // to PFF: DELSQH(psi, 2 LN), psi with LN = 0, DEL2(chi), DELSQH(chi), DELSQH(psi) and the vorticity
+  const double2 *in[NF] = {a->e, psi->e, d2c->e, dc->e, dp->e, ror->e, rop->e, oz->e};
+  const double *ln[NF] = {a->ln, dp->ln, d2c->ln, dc->ln, dp->ln, ror->ln, rop->ln, oz->ln};
+  double2 *pff[NF];
+  for (int q = 0; q < NF; q++) pff[q] = t[q]->e;
+  RET(launch_rtran_bwd_n(c, NF, in, ln, pff));
   // VALENE = -PRODCT(DELSQH(psi, 2 LN), psi) + PRODCT(DELSQH(chi), DEL2(chi)),
-  // VALHEL = 2 PRODCT(DELSQH(psi), DEL2(chi)), all in PFF
-  double ene1, ene2, hel1;
-  RET(copy_field(rup, psi));
-  RET(launch_set_ln(c, rup->ln, psi->ln, 2.0, 0.0));
-  RET(mlg_delsqh(rup, rur));
-  RET(mlg_rtran(rur, 1));
-  RET(copy_field(rup, psi));
-  RET(launch_set_ln(c, rup->ln, nullptr, 0.0, 0.0));
-  RET(mlg_rtran(rup, 1));
-  RET(prodct(c, rur, rup, &ene1));
-  RET(mlg_del2(chi, rup));
-  RET(mlg_rtran(rup, 1));
-  RET(mlg_delsqh(chi, rur));
-  RET(mlg_rtran(rur, 1));
-  RET(prodct(c, rur, rup, &ene2));
-  out[2] = -ene1 + ene2;
-  RET(mlg_delsqh(psi, rur));
-  RET(mlg_rtran(rur, 1));
-  RET(prodct(c, rur, rup, &hel1));
-  out[3] = 2 * hel1;
-  // psi and chi at r = infinity
-  RET(calcat1(c, psi, &out[5], &out[6]));
-  RET(calcat1(c, chi, &out[7], &out[8]));
-  // OZH (1-x)^2 = OZ, then CALCXY
-  RET(mlg_mulxm(ozh, rur));
-  RET(mlg_mulxm(rur, ozh));
-  RET(mlg_tofp(ror));
-  RET(mlg_tofp(rop));
-  RET(mlg_tofp(ozh));
+  // VALHEL = 2 PRODCT(DELSQH(psi), DEL2(chi))
+  const size_t na = (size_t)G.ntchop * G.nxchopdim;
+  RET(launch_energy_terms(c, pff[0], pff[1], 0, c->d.red));
+  RET(launch_energy_terms(c, pff[3], pff[2], 0, c->d.red + na));
+  RET(launch_energy_terms(c, pff[4], pff[2], 0, c->d.red + 2 * na));
+  // CALCXY: the vorticity to physical space
+  const double2 *vin[3] = {pff[5], pff[6], pff[7]};
+  double2 *vor[3] = {ror->e, rop->e, oz->e};
+  RET(launch_verfft_bwd_n(c, 3, vin, vor));
+  RET(launch_horfft_bwd_n(c, 3, vor, 1.0, 1.0, nullptr));
   KGrid g = kgrid(c);
-  hipLaunchKernelGGL(k_absvec2, dim3(blocks_ppp(g)), dim3(256), 0, c->stream, g, ror->e, rop->e, ozh->e, ozh->e, c->d.r,
-                     c->d.x);
+  hipLaunchKernelGGL(k_absvec2_sum, dim3((g.nr + 63) / 64, g.nth), dim3(256), 0, c->stream, g, ror->e, rop->e, oz->e, c->d.r,
+                     c->d.x, t[0]->e);
   MLG_CHECK_HIP(hipGetLastError());
-  // the (r, theta) factors r cos(theta), r sin(theta), r^2 on both sub-grids
-  // (THR = 2 pi j / NTH, THI = 2 pi (j + 1/2) / NTH; MINC = 1)
-  const size_t nt = (size_t)G.nr * G.nth;
-  std::vector<double> f(6 * nt);
-  for (int j = 0; j < G.nth; j++) {
-    const double thr = 2 * pi / G.p.minc / G.nth * j, thi = 2 * pi / G.p.minc / G.nth * (j + 0.5);
-    for (int r = 0; r < G.nr; r++) {
-      const size_t t = (size_t)r + (size_t)G.nr * j;
-      f[t] = G.r[r] * std::cos(thr);
-      f[nt + t] = G.r[r] * std::cos(thi);
-      f[2 * nt + t] = G.r[r] * std::sin(thr);
-      f[3 * nt + t] = G.r[r] * std::sin(thi);
-      f[4 * nt + t] = G.r[r] * G.r[r];
-      f[5 * nt + t] = G.r[r] * G.r[r];
-    }
+  const int nxd = G.nxchopdim, nval = IT1_AT1 + 2 * nxd;
+  It1 v;
+  v.dp = dp->e, v.dc = dc->e, v.ang = ang->e;
+  v.f[0] = psi->e, v.f[1] = chi->e;
+  v.at1 = c->d.at1, v.x = c->d.x, v.w = c->d.w, v.r2 = c->d.r, v.terms = c->d.red;
+  v.abs = t[0]->e;
+  v.p00 = G.pf[0];
+  v.na = (int)na, v.nn = G.nrchop;
+  v.minc = G.p.minc;
+  double *res = reinterpret_cast<double *>(t[1]->e);  // nval doubles: far fewer than a field's
+  hipLaunchKernelGGL(k_it1_values, dim3(nval), dim3(1024), 0, c->stream, g, v, res);
+  MLG_CHECK_HIP(hipGetLastError());
+  std::vector<double> h(nval);
+  MLG_CHECK_HIP(hipMemcpyAsync(h.data(), res, sizeof(double) * nval, hipMemcpyDeviceToHost, c->stream));
+  MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  // INTEG (src/mod_scalar3.f90:312-353): 4 pi ZLEN ELL^2 Re(f(0,0,0)) NORM(0, m=0)
+  const double fi = 4.0 * pi * G.zlen * G.ell2;
+  out[0] = fi * h[0] * G.norm[0];  // VALVOR
+  out[1] = fi * h[1] * G.norm[0];  // VALZMO
+  out[2] = -h[3] + h[4];           // VALENE
+  out[3] = 2 * h[5];               // VALHEL
+  out[4] = -(2.0 * pi * G.zlen * G.ell2 * h[2]);
+  // psi and chi at r = infinity (CALCAT1, src/mod_scalar3.f90:286-310)
+  for (int q = 0; q < 2; q++) {
+    const double *at = h.data() + IT1_AT1 + q * nxd;
+    out[5 + 2 * q] = at[0];
+    out[6 + 2 * q] = *std::max_element(at, at + nxd) - *std::min_element(at, at + nxd);
   }
-  double *df = nullptr;
-  MLG_CHECK_HIP(hipMalloc((void **)&df, sizeof(double) * f.size()));
-  int rc = hipMemcpy(df, f.data(), sizeof(double) * f.size(), hipMemcpyHostToDevice) == hipSuccess ? 0 : MLG_E_HIP;
-  double valens = 0.0, mom[3] = {0.0, 0.0, 0.0};
-  if (!rc) rc = copy_field(ror, ozh);
-  if (!rc) rc = mlg_toff(ror);
-  if (!rc) rc = integ(c, ror, &valens);
-  for (int q = 0; q < 3 && !rc; q++) {
-    rc = copy_field(ror, ozh);
-    if (!rc) {
-      hipLaunchKernelGGL(k_mul_rtheta, dim3(blocks_ppp(g)), dim3(256), 0, c->stream, g, ror->e, df + 2 * q * nt,
-                         df + (2 * q + 1) * nt);
-      if (hipGetLastError() != hipSuccess) rc = MLG_E_HIP;
-    }
-    if (!rc) rc = mlg_toff(ror);
-    if (!rc) rc = integ(c, ror, &mom[q]);
-  }
-  (void)hipStreamSynchronize(c->stream);
-  (void)hipFree(df);
-  RET(rc);
-  out[9] = mom[0] / valens;             // <X>
-  out[10] = mom[1] / valens;            // <Y>
-  out[11] = std::sqrt(mom[2] / valens); // <R>
+  out[9] = h[7] / h[6];              // <X>
+  out[10] = h[8] / h[6];             // <Y>
+  out[11] = std::sqrt(h[9] / h[6]);  // <R>
   return 0;
 }
 

@@ -209,21 +209,24 @@ static int ringcut(mlg_field *wk, int ns0, int ns, int divxm2) {
 // the per-(m, k) products of PRODCT_MK_HALFK (l2 = 0: Re(a conj b); 1:
 // L2NORM_MK_HALFK's |a|^2 / (1-x)^2) folded to the NXCHOP non-negative k
 // (src/mod_scalar3.f90:470-554)
-static int halfk(mlg_ctx *c, const double2 *a, const double2 *b, int l2, std::vector<double> &out) {
-  const Grid &G = c->g;
+static void fold_halfk(const Grid &G, const double *h, std::vector<double> &out) {
   const int nt = G.ntchop, nxc = G.nxchop, nxd = G.nxchopdim;
-  const size_t na = (size_t)nt * nxd;
-  double *dall = c->d.red;
-  RET(launch_energy_terms(c, a, b, l2, dall));
-  std::vector<double> h(na);
-  MLG_CHECK_HIP(hipMemcpyAsync(h.data(), dall, sizeof(double) * na, hipMemcpyDeviceToHost, c->stream));
-  MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
   out.assign((size_t)nt * nxc, 0.0);
   for (int mm = 0; mm < nt; mm++) out[mm] = h[mm];
   for (int kk = 2; kk <= nxc; kk++) {
     const int kc = nxd + 2 - kk;
     for (int mm = 0; mm < nt; mm++) out[mm + (size_t)nt * (kk - 1)] = h[mm + (size_t)nt * (kc - 1)] + h[mm + (size_t)nt * (kk - 1)];
   }
+}
+static int halfk(mlg_ctx *c, const double2 *a, const double2 *b, int l2, std::vector<double> &out) {
+  const Grid &G = c->g;
+  const size_t na = (size_t)G.ntchop * G.nxchopdim;
+  double *dall = c->d.red;
+  RET(launch_energy_terms(c, a, b, l2, dall));
+  std::vector<double> h(na);
+  MLG_CHECK_HIP(hipMemcpyAsync(h.data(), dall, sizeof(double) * na, hipMemcpyDeviceToHost, c->stream));
+  MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  fold_halfk(G, h.data(), out);
   return 0;
 }
 
@@ -247,25 +250,31 @@ static int enemon(const mlg_field *psi, const mlg_field *chi, double *em, double
   mlg_ctx *c = psi->ctx;
   const Grid &G = c->g;
   const int nt = G.ntchop, nxc = G.nxchop;
+  // DELSQH(psi, 2 LN), psi with LN = 0, DEL2(chi) and DELSQH(chi) share one
+  // backward launch, and the two products one copy to the host
+  constexpr int NF = 4;
   Temps T(c);
-  mlg_field *w1 = T.get(), *w2 = T.get();
+  mlg_field *zero = T.get(), *ln2 = T.buffer(), *a = T.buffer(), *d2 = T.buffer(), *dh = T.buffer(), *t[NF];
+  for (auto &q : t) q = T.buffer();
   RET(T.ready());
-  std::vector<double> mk;
-  std::vector<double> am(nt), ak(nxc);
-  RET(copy_field(w1, psi));
-  RET(launch_set_ln(c, w1->ln, psi->ln, 2.0, 0.0));  // W1%LN = 2 PSI%LN
-  RET(mlg_delsqh(w1, w2));
-  RET(mlg_rtran(w2, 1));
-  RET(copy_field(w1, psi));
-  RET(launch_set_ln(c, w1->ln, nullptr, 0.0, 0.0));
-  RET(mlg_rtran(w1, 1));
-  RET(halfk(c, w2->e, w1->e, 0, mk));
+  RET(launch_set_ln(c, ln2->ln, psi->ln, 2.0, 0.0));  // W1%LN = 2 PSI%LN
+  RET(launch_delsqh(c, psi->e, ln2->ln, a->e, a->ln));
+  RET(mlg_del2(chi, d2));
+  RET(mlg_delsqh(chi, dh));
+  const double2 *in[NF] = {a->e, psi->e, d2->e, dh->e};
+  const double *ln[NF] = {a->ln, zero->ln, d2->ln, dh->ln};
+  double2 *pff[NF];
+  for (int q = 0; q < NF; q++) pff[q] = t[q]->e;
+  RET(launch_rtran_bwd_n(c, NF, in, ln, pff));
+  const size_t na = (size_t)nt * G.nxchopdim;
+  RET(launch_energy_terms(c, pff[0], pff[1], 0, c->d.red));
+  RET(launch_energy_terms(c, pff[3], pff[2], 0, c->d.red + na));
+  std::vector<double> h(2 * na), mk, am(nt), ak(nxc);
+  MLG_CHECK_HIP(hipMemcpyAsync(h.data(), c->d.red, sizeof(double) * 2 * na, hipMemcpyDeviceToHost, c->stream));
+  MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
+  fold_halfk(G, h.data(), mk);
   sums(mk, nt, nxc, nt, em, ek);
-  RET(mlg_del2(chi, w1));
-  RET(mlg_rtran(w1, 1));
-  RET(mlg_delsqh(chi, w2));
-  RET(mlg_rtran(w2, 1));
-  RET(halfk(c, w2->e, w1->e, 0, mk));
+  fold_halfk(G, h.data() + na, mk);
   sums(mk, nt, nxc, nt, am.data(), ak.data());
   for (int mm = 0; mm < nt; mm++) em[mm] = -em[mm] + am[mm];
   for (int kk = 0; kk < nxc; kk++) ek[kk] = -ek[kk] + ak[kk];
