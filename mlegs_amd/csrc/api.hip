@@ -2,6 +2,7 @@
 // the Boussinesq step.  Kernels live in k_*.hip; this file sequences them on
 // the context's stream, mirroring the reference's call structure and CHOPSET
 // (truncation) state so results match the reference routine by routine.
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <cstdlib>
@@ -735,7 +736,9 @@ extern "C" int mlg_vdotpsub(const mlg_field *rar, const mlg_field *rap, const ml
   if (rar->space != MLG_PPP || rbr->space != MLG_PPP) return MLG_E_SPACE;
   mlg_ctx *c = rar->ctx;
   out->space = MLG_PPP;
-  RET(launch_zero(c, out->e, c->n_ppp));
+  // an output that is one of the inputs is cleared before they are read
+  const mlg_field *const in[6] = {rar, rap, az, rbr, rbp, bz};
+  if (std::find(in, in + 6, out) != in + 6) RET(launch_zero(c, out->e, c->n_ppp));
   RET(launch_set_ln(c, out->ln, nullptr, 0.0, 0.0));
   return launch_vdot(c, rar->e, rap->e, az->e, rbr->e, rbp->e, bz->e, out->e, 1.0);
 }

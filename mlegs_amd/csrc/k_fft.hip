@@ -380,6 +380,21 @@ int launch_verfft_bwd_n(mlg_ctx *c, int n, const double2 *const *in, double2 *co
 
 int launch_verfft_bwd(mlg_ctx *c, const double2 *in, double2 *out) { return launch_verfft_bwd_n(c, 1, &in, &out); }
 
+// Unscaled theta transforms of 16 .. 512 points go on the line kernels of the
+// fused products: backward 208 -> 166 us at 384x256x256, 52 -> 32 at
+// 384x128x128, 55 -> 16 at 384x32x256, 8.1 -> 6.3 at 128x64x64.  Forward,
+// their reads are runs of 32 bytes, which costs fields that exceed the caches
+// (174 us against 156 at 384x256x256, 44 against 40 at 384x128x128, 102 MB)
+// what it gains smaller ones (28 -> 20 at 200x256x64, 53 MB; 27 -> 15 at
+// NTH = 32, where the runs are longer); NTH = 512 has no other kernel of that
+// kind and the mixed-radix one takes as long (106 us at 192x512x128) or
+// longer (12.8 against 7.8 at 64x512x16).
+static bool horfft_on_lines(const KGrid &g, const HorJobs &j, bool fwd) {
+  const int n = g.nth;
+  if (n < 16 || n > 512 || (n & (n - 1)) || j.s0 != 1.0 || j.s1 != 1.0 || j.wr) return false;
+  const double bytes = 16.0 * g.ndimr * g.ndimth * (double)g.ndimx * j.n;
+  return !fwd || n <= 32 || n == 512 || bytes <= 64e6;
+}
 int launch_horfft_fwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double s1) {
   if (n < 1 || n > MAX_HOR_JOBS) return MLG_E_ARG;
   KGrid g = kgrid(c);
@@ -387,8 +402,9 @@ int launch_horfft_fwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double 
   for (int i = 0; i < n; i++) jobs.a[i] = a[i];
   jobs.n = n;
   jobs.s0 = s0, jobs.s1 = s1, jobs.wr = nullptr;
-  if (!fft4_length(g.nth)) return launch_horfft_any(c, jobs, true);
   KScope ks(c, K_HORFFT_FWD, n * 16.0 * g.nr * g.nx * (double)(g.nth + g.ntchopdim));
+  if (horfft_on_lines(g, jobs, true)) return launch_horfft_line(c, jobs, true);
+  if (!fft4_length(g.nth)) return launch_horfft_any(c, jobs, true);
 #define L_HF(a_, b_)                                                                                            \
   hipLaunchKernelGGL((k_horfft_fwd4<a_, b_>), dim3((g.ndimr + Fft4<a_, b_>::P - 1) / Fft4<a_, b_>::P, g.ndimx, n), \
                      dim3(256), 0, c->stream, g, c->d.tw_t, c->d.tw_h, jobs)
@@ -406,8 +422,9 @@ int launch_horfft_bwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double 
   for (int i = 0; i < n; i++) jobs.a[i] = a[i];
   jobs.n = n;
   jobs.s0 = s0, jobs.s1 = s1, jobs.wr = wr;
-  if (!fft4_length(g.nth)) return launch_horfft_any(c, jobs, false);
   KScope ks(c, K_HORFFT_BWD, n * 16.0 * g.nr * g.nx * (double)(g.nth + g.ntchopdim));
+  if (horfft_on_lines(g, jobs, false)) return launch_horfft_line(c, jobs, false);
+  if (!fft4_length(g.nth)) return launch_horfft_any(c, jobs, false);
 #define L_HB(a_, b_)                                                                                            \
   hipLaunchKernelGGL((k_horfft_bwd4<a_, b_>), dim3((g.ndimr + Fft4<a_, b_>::P - 1) / Fft4<a_, b_>::P, g.ndimx, n), \
                      dim3(256), 0, c->stream, g, c->d.tw_t, c->d.tw_h, jobs)

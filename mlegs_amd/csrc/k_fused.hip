@@ -1087,6 +1087,8 @@ struct LineTiny {
 };
 struct Line16 {
   static constexpr int N = 16, LANES = 2, THREADS = 256, LP = 16, MMAX = w16::MMAX6, NT2 = 1;
+  // theta index of the point in slot i of lane b
+  __device__ static int point(int b, int i) { return i + 8 * b; }
   __device__ static void tables(int q, double2 *T1, double2 *, const double2 *tw) {
     if (q < 16) T1[q] = tw[(q & 1) * (q >> 1)];
   }
@@ -1103,6 +1105,8 @@ struct Line16 {
 };
 struct Line128 {
   static constexpr int N = 128, LANES = 16, THREADS = 256, LP = w128::LP, MMAX = w128::MMAX48, NT2 = 16;
+  // theta index of the point in slot i of lane b
+  __device__ static int point(int b, int i) { return ((b >> 2) + 4 * (i >> 2)) + 8 * (b & 3) + 32 * (i & 3); }
   __device__ static void tables(int q, double2 *T1, double2 *T2, const double2 *tw) {
     if (q < 128) T1[q] = tw[(q & 15) * (q >> 4)];
     if (q < 16) T2[q] = tw[8 * (q & 3) * (q >> 2)];
@@ -1120,6 +1124,8 @@ struct Line128 {
 };
 struct Line32 {
   static constexpr int N = 32, LANES = 4, THREADS = 256, LP = w32::LP, MMAX = w32::MMAX12, NT2 = 1;
+  // theta index of the point in slot i of lane b
+  __device__ static int point(int b, int i) { return (b + 4 * (i >> 2)) + 8 * (i & 3); }
   __device__ static void tables(int q, double2 *T1, double2 *, const double2 *tw) {
     if (q < 32) T1[q] = tw[(q & 3) * (q >> 2)];
   }
@@ -1136,6 +1142,8 @@ struct Line32 {
 };
 struct Line64 {
   static constexpr int N = 64, LANES = 8, THREADS = 256, LP = w64::LP, MMAX = w64::MMAX24, NT2 = 1;
+  // theta index of the point in slot i of lane b
+  __device__ static int point(int b, int i) { return b + 8 * i; }
   __device__ static void tables(int q, double2 *T1, double2 *, const double2 *tw) {
     if (q < 64) T1[q] = tw[(q & 7) * (q >> 3)];
   }
@@ -1153,6 +1161,8 @@ struct Line64 {
 
 struct Line512 {
   static constexpr int N = 512, LANES = 64, THREADS = 512, LP = w512::LP, MMAX = w512::MMAX192, NT2 = 64;
+  // theta index of the point in slot i of lane b
+  __device__ static int point(int b, int i) { return (b >> 3) + 8 * (b & 7) + 64 * i; }
   __device__ static void tables(int q, double2 *T1, double2 *T2, const double2 *tw) {
     T1[q] = tw[(q & 63) * (q >> 6)];
     if (q < 64) T2[q] = tw[8 * (q & 7) * (q >> 3)];
@@ -1274,7 +1284,9 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
 }
 
 struct Line256 {
-  static constexpr int N = 256, LANES = 32, LP = w256::LP, MMAX = w256::MMAX96, NT2 = 32;
+  static constexpr int N = 256, LANES = 32, THREADS = 256, LP = w256::LP, MMAX = w256::MMAX96, NT2 = 32;
+  // theta index of the point in slot i of lane b
+  __device__ static int point(int b, int i) { return (b >> 2) + 8 * ((b & 3) + 4 * (i >> 2)) + 64 * (i & 3); }
   __device__ static void tables(int q, double2 *T1, double2 *T2, const double2 *tw) {
     if (q < 256) T1[q] = tw[(q & 31) * (q >> 5)];
     if (q < 32) T2[q] = tw[8 * (q & 3) * (q >> 2)];
@@ -1365,6 +1377,84 @@ k_fused_products_wide(KGrid g, const double *__restrict__ rsq, const double2 *tw
   }
   __syncthreads();
   if (w < 4) L::template forward<FULL>(x, g, v, io.out[w] + off, lo, inr, live);
+}
+
+// HORFFT of one field (PFP m < NTCHOPDIM <-> PPP slots, in place) on the same
+// lines: a wave transforms whole theta lines without a barrier, and a block
+// takes adjacent radial nodes of one plane.  Radial lines are not whole cache
+// lines; the blocks that share one run on one XCD.
+template <class L, bool FULL, bool FWD>
+__global__ void __launch_bounds__(L::THREADS) k_horfft_line(KGrid g, const double2 *tw, const double2 *twh, HorJobs jobs) {
+  constexpr int N = L::N, LANES = L::LANES, LINES = L::THREADS / LANES;
+  __shared__ double2 S[LINES * L::LP];
+  __shared__ double2 T1[N], T2[L::NT2], TH[N + 1];
+  const int nrb = (g.ndimr + LINES - 1) / LINES;
+  const int lid = xcd_logical(nrb * g.ndimx * jobs.n);
+  if (lid < 0) return;
+  {
+    const int q = threadIdx.x;
+    L::tables(q, T1, T2, tw);
+    if (q <= N) TH[q] = twh[q];
+    if (L::THREADS == N && q == 0) TH[N] = twh[N];
+  }
+  __syncthreads();
+  const int z = lid / nrb % g.ndimx, line = threadIdx.x / LANES;
+  const int rr = (lid % nrb) * LINES + line;
+  const bool inr = rr < g.ndimr, live = rr < g.nr;
+  w256::Ctx x;
+  x.t1 = T1;
+  x.t2 = T2;
+  x.th = TH;
+  x.s = S + line * L::LP;
+  x.b = threadIdx.x % LANES;
+  double2 *a = jobs.a[lid / nrb / g.ndimx] + (size_t)(rr - line) + (size_t)g.ndimr * g.ndimth * z;  // same for the block
+  const int lo = inr ? line : 0;
+  double2 v[8];
+  if constexpr (FWD) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      v[i] = a[lo + g.ndimr * L::point(x.b, i)];
+      if (!live) v[i] = make_double2(0.0, 0.0);
+    }
+    L::template forward<FULL>(x, g, v, a, lo, inr, live);
+  } else {
+    L::template inverse<FULL>(x, g, a, lo, live, v);
+    if (!inr) return;
+#pragma unroll
+    for (int i = 0; i < 8; i++) a[lo + g.ndimr * L::point(x.b, i)] = live ? v[i] : make_double2(0.0, 0.0);
+    if (x.b == 0) a[lo + g.ndimr * N] = make_double2(0.0, 0.0);
+  }
+}
+
+template <class L, bool FULL>
+static void horfft_line(mlg_ctx *c, const KGrid &g, const HorJobs &jobs, bool fwd) {
+  constexpr int lines = L::THREADS / L::LANES;
+  const dim3 grid(xcd_grid((g.ndimr + lines - 1) / lines * g.ndimx * jobs.n));
+  if (fwd)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_horfft_line<L, FULL, true>), grid, dim3(L::THREADS), 0, c->stream, g, c->d.tw_t,
+                       c->d.tw_h, jobs);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_horfft_line<L, FULL, false>), grid, dim3(L::THREADS), 0, c->stream, g, c->d.tw_t,
+                       c->d.tw_h, jobs);
+}
+template <class L>
+static int horfft_lines(mlg_ctx *c, const HorJobs &jobs, bool fwd) {
+  const KGrid g = kgrid(c);
+  if (g.ntchopdim <= L::MMAX) horfft_line<L, false>(c, g, jobs, fwd);
+  else horfft_line<L, true>(c, g, jobs, fwd);
+  MLG_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+int launch_horfft_line(mlg_ctx *c, const HorJobs &jobs, bool fwd) {
+  switch (c->g.nth) {
+    case 16: return horfft_lines<Line16>(c, jobs, fwd);
+    case 32: return horfft_lines<Line32>(c, jobs, fwd);
+    case 64: return horfft_lines<Line64>(c, jobs, fwd);
+    case 128: return horfft_lines<Line128>(c, jobs, fwd);
+    case 256: return horfft_lines<Line256>(c, jobs, fwd);
+    case 512: return horfft_lines<Line512>(c, jobs, fwd);
+    default: return MLG_E_ARG;
+  }
 }
 
 bool fused_products_supported(const mlg_ctx *c) {

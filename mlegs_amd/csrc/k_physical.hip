@@ -30,19 +30,24 @@ __global__ void k_vprod(KGrid g, const double *__restrict__ rr, const double2 *_
   }
 }
 
+// Over the whole PPP array: zero past NR and NTH, in place of clearing the
+// result first (75 us of 395 at 384x256x256).
 __global__ void k_vdot(KGrid g, const double *__restrict__ rr, const double2 *__restrict__ rar,
                        const double2 *__restrict__ rap, const double2 *__restrict__ az, const double2 *__restrict__ rbr,
                        const double2 *__restrict__ rbp, const double2 *__restrict__ bz, double2 *__restrict__ out,
                        double sign, long total) {
   for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
-    const unsigned u = (unsigned)idx, q = u / (unsigned)g.nr, zz = q / (unsigned)g.nth;
-    const int r = (int)(u - q * (unsigned)g.nr), j = (int)(q - zz * (unsigned)g.nth), z = (int)zz;
-    size_t id = (size_t)r + (size_t)g.ndimr * ((size_t)j + (size_t)g.ndimth * z);
-    double2 a1 = rar[id], a2 = rap[id], a3 = az[id], b1 = rbr[id], b2 = rbp[id], b3 = bz[id];
-    double r2 = rr[r];  // r_i^2
-    double vr = (a1.x * b1.x + a2.x * b2.x) / r2 + a3.x * b3.x;
-    double vi = (a1.y * b1.y + a2.y * b2.y) / r2 + a3.y * b3.y;
-    out[id] = make_double2(sign * vr, sign * vi);
+    const unsigned u = (unsigned)idx, q = u / (unsigned)g.ndimr, zz = q / (unsigned)g.ndimth;
+    const int r = (int)(u - q * (unsigned)g.ndimr), j = (int)(q - zz * (unsigned)g.ndimth);
+    double2 v = make_double2(0.0, 0.0);
+    if (r < g.nr && j < g.nth) {
+      double2 a1 = rar[idx], a2 = rap[idx], a3 = az[idx], b1 = rbr[idx], b2 = rbp[idx], b3 = bz[idx];
+      double r2 = rr[r];  // r_i^2
+      double vr = (a1.x * b1.x + a2.x * b2.x) / r2 + a3.x * b3.x;
+      double vi = (a1.y * b1.y + a2.y * b2.y) / r2 + a3.y * b3.y;
+      v = make_double2(sign * vr, sign * vi);
+    }
+    out[idx] = v;
   }
 }
 
@@ -97,7 +102,7 @@ int launch_vprod(mlg_ctx *c, const double2 *rur, const double2 *rup, const doubl
 int launch_vdot(mlg_ctx *c, const double2 *rar, const double2 *rap, const double2 *az, const double2 *rbr, const double2 *rbp,
                 const double2 *bz, double2 *out, double sign) {
   KGrid g = kgrid(c);
-  long total = (long)g.nr * g.nth * g.ndimx;
+  long total = (long)g.ndimr * g.ndimth * g.ndimx;
   KScope ks(c, K_PRODUCTS, 16.0 * total * 7);
   hipLaunchKernelGGL(k_vdot, dim3(grid_for(total)), dim3(256), 0, c->stream, g, c->d.r, rar, rap, az, rbr, rbp, bz, out, sign,
                      total);

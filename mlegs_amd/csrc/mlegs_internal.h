@@ -320,6 +320,8 @@ static inline bool fft4_length(int n) { return n >= 2 && n <= 256 && (n & (n - 1
 int fft_any_setup(int n, FftAny *f);  // allocates f's device tables
 int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd);
 int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd);
+// NTH = 16, 32, .. 512 without scale factors, on the lines of the fused products (k_fused.hip)
+int launch_horfft_line(mlg_ctx *c, const HorJobs &jobs, bool fwd);
 // theta lengths with a register-resident products kernel (k_fused.hip)
 static inline bool fused_line_length(int n) { return n >= 2 && n <= 512 && (n & (n - 1)) == 0; }
 // fused products elsewhere (k_fused_any.hip); f->n = 0 where the length has no plan
