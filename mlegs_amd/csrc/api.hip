@@ -922,11 +922,12 @@ static int to_pfp_b(mlg_ctx *c, mlg_field *const *fs, const mlg_field *b, mlg_fi
 // W = TOFP(B) at NRCHOP and GRAD's i m b and i k b at NRCHOP+3 are Legendre
 // jobs of the one batch (the z-transform multiplies by i m or i k as it
 // loads), GRAD's r d/dr b comes with PC2VEL and PC2VOR, N_b's z-transform
-// runs with PROJECT's, and psi's fix-up at infinity with chi's: eleven
-// launches, where the routines called one by one are twenty-two.  A launch
-// is about 4.4 us of a captured step whatever it does.  With the AB2 step and
-// VISC2's right-hand sides in one launch (visc_cn) a step is thirteen launches
-// instead of twenty-seven: 178 -> 115 us at 64x32x32, 225 -> 160 at 128x64x64.
+// runs with PROJECT's, and the chop and fixes at infinity of psi and chi with
+// N_b's RTRAN: ten launches, where the routines called one by one are
+// twenty-two.  A launch is about 4.4 us of a captured step whatever it does.
+// With the AB2 step and VISC2's right-hand sides in one launch (visc_cn) a
+// step is twelve launches instead of twenty-seven: 178 -> 102 us at 64x32x32,
+// 225 -> 159 at 128x64x64.
 static int force_fused(const mlg_field *psi, const mlg_field *chi, const mlg_field *b, mlg_field *psin, mlg_field *chin,
                        mlg_field *bn) {
   mlg_ctx *c = psi->ctx;
@@ -973,8 +974,11 @@ static int force_fused(const mlg_field *psi, const mlg_field *chi, const mlg_fie
   RET(project_impl(f[3], f[4], f[5], psin, w2, 1, 0.0, nullptr, true));
   RET(solve_op(w2, chin, 1, 0.0, 0, 0.0, false));  // IDEL2LN
   double2 *const fix[2] = {psin->e, chin->e};
-  RET(launch_chopdo_fff_n(c, 2, fix, true));  // CHOPDO, and the fixes at infinity of PROJECT and IDEL2LN
-  return mlg_toff(bn);
+  // N_b to FFF; CHOPDO, and the fixes at infinity of PROJECT and IDEL2LN
+  RET(launch_rtran_fwd_fix(c, bn->e, w2->e, bn->ln, fix));
+  swap_storage(bn, w2);
+  bn->space = MLG_FFF;
+  return 0;
 }
 
 // CALC_BOUSSI_FORCE (src/mod_boussinesq.f90:317-410)

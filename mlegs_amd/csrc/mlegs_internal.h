@@ -283,6 +283,8 @@ int launch_verfft_fwd_n(mlg_ctx *c, int n, const double2 *const *in, double2 *co
 // zl: an LN set to 0; w: the Gauss weights of the sums (null: the grid's;
 // the adjoint passes ones, FP64 products only)
 int launch_rtran_fwd(mlg_ctx *c, const double2 *in, double2 *out, double *zl = nullptr, const double *w = nullptr);
+// launch_rtran_fwd with launch_chopdo_fff_n(fix, true) of two other fields
+int launch_rtran_fwd_fix(mlg_ctx *c, const double2 *in, double2 *out, double *zl, double2 *const fix[2]);
 // n (<= MAX_TRANSFORM_JOBS) fields in one launch (FP64 products only)
 int launch_rtran_fwd_n(mlg_ctx *c, int n, const double2 *const *in, double2 *const *out, const double *w = nullptr);
 int launch_project(mlg_ctx *c, const double2 *rur, const double2 *rup, const double2 *uz, double2 *psi, double2 *chi);
