@@ -413,12 +413,43 @@ __device__ __forceinline__ void rtran_bwd_tile(const KGrid &g, const typename Le
   }
 }
 
+template <int TI, int TC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 k_rtran_bwd(KGrid g, const double *__restrict__ pf, TransformJobs jobs, int nj, const double *__restrict__ lnx) {
-  __shared__ RtranBwdLds<false, 64, 64> L;
-  const int lid = xcd_logical(rtran_bwd_tiles<64, 64>(g, nj));
+  __shared__ RtranBwdLds<false, TI, TC> L;
+  const int lid = xcd_logical(rtran_bwd_tiles<TI, TC>(g, nj));
   if (lid < 0) return;
-  rtran_bwd_tile<false, 64, 64>(g, pf, jobs, nj, lnx, nullptr, lid, L);
+  rtran_bwd_tile<false, TI, TC>(g, pf, jobs, nj, lnx, nullptr, lid, L);
+}
+// The tile shape of a product: the least padded nodes x columns, the smaller
+// shapes' at 1.1 (32 x 64) and 1.2 (64 x 32) times where the blocks fill the
+// chip (three a CU), for they read the tables and data more often (384x256x256
+// one field: 90 us at 64 x 64, 101 at 32 x 64 and at 64 x 32; 384x128x128 nine
+// fields 182, 201, 206).  64 nodes leave half a tile empty at NR = 150 (nine
+// fields at 150x90x100: 42.0 us, 37.5 at 32 x 64), 192 (192x128x128: 72.9,
+// 60.3) or 64 and less (64x32x32: 9.0, 7.0); 64 columns a third of them at
+// 22 k (128x64x64: 17.6 us, 16.1 at 64 x 32).  Every shape gives the same bits.
+static BwdTile bwd_shape(const KGrid &g, int nj) {
+  auto up = [](int n, int t) { return (double)((n + t - 1) / t * t); };
+  const int nodes = g.nrh, cols = 2 * g.nxchopdim;
+  const bool full = rtran_bwd_tiles<64, 64>(g, nj) > 3 * 256;
+  const double a = up(nodes, 64) * up(cols, 64), b = up(nodes, 32) * up(cols, 64) * (full ? 1.1 : 1.0),
+               d = up(nodes, 64) * up(cols, 32) * (full ? 1.2 : 1.0);
+  if (b < a && b <= d) return BWD_TILE_32x64;
+  return d < a ? BWD_TILE_64x32 : BWD_TILE_64x64;
+}
+static int launch_bwd_fp64(mlg_ctx *c, const KGrid &g, const TransformJobs &jobs, int n) {
+#define L_BWD(TI_, TC_)                                                                                                \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_rtran_bwd<TI_, TC_>), dim3(xcd_grid(rtran_bwd_tiles<TI_, TC_>(g, n))), dim3(256), 0, \
+                     c->stream, g, c->d.pf, jobs, n, c->d.lnx)
+  switch (bwd_shape(g, n)) {
+    case BWD_TILE_32x64: L_BWD(32, 64); break;
+    case BWD_TILE_64x32: L_BWD(64, 32); break;
+    default: L_BWD(64, 64); break;
+  }
+#undef L_BWD
+  MLG_CHECK_HIP(hipGetLastError());
+  return 0;
 }
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -488,18 +519,16 @@ int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double
   if (!c->leg_split) {
     if (c->rec) return sweep_defer_bwd(c, g, jobs, n);
     KScope ks(c, K_RTRAN_BWD, per_k * (double)sum_nrchops(c));
-    hipLaunchKernelGGL(k_rtran_bwd, dim3(xcd_grid(rtran_bwd_tiles<64, 64>(g, n))), dim3(256), 0, c->stream, g, c->d.pf,
-                       jobs, n, c->d.lnx);
-    MLG_CHECK_HIP(hipGetLastError());
+    const int rc = launch_bwd_fp64(c, g, jobs, n);
+    if (rc) return rc;
     return 0;
   }
   KGrid g0, g1;
   split_modes(c, g, g0, g1);
   {
     KScope ks(c, K_RTRAN_BWD, per_k * split_fp64_sum(g0, 1));
-    hipLaunchKernelGGL(k_rtran_bwd, dim3(xcd_grid(rtran_bwd_tiles<64, 64>(g0, n))), dim3(256), 0, c->stream, g0, c->d.pf,
-                       jobs, n, c->d.lnx);
-    MLG_CHECK_HIP(hipGetLastError());
+    const int rc = launch_bwd_fp64(c, g0, jobs, n);
+    if (rc) return rc;
   }
   if (g1.mcnt > 0) {
     KScope ks(c, K_RTRAN_BWD, per_k * ((double)sum_nrchops(c) - split_fp64_sum(g0, 1)));
