@@ -15,7 +15,8 @@
 // into a complex length-N one, so the slots are transformed as they lie and
 // the half-spectrum is split/merged with the e^{-i pi m/NTH} twiddles.
 //
-// Powers of two up to 256 take the four-step register kernels here, every
+// Powers of two up to 256 take the four-step register kernels here (unscaled
+// theta transforms mostly the line kernels of k_fused.hip, horfft_on_lines), every
 // other length the mixed-radix kernels of k_fft_any.hip.
 #include "mlegs_internal.h"
 #include "xcd.h"
@@ -222,7 +223,7 @@ __global__ void __launch_bounds__(512) k_verfft_bwd4(KGrid g, const double2 *__r
 }
 
 // HORFFT forward, in place: PPP slots -> PFP m < NTCHOPDIM (split of the
-// packed real transform as in k_horfft_fwd).
+// packed real transform).
 template <int R1, int R2>
 __global__ void __launch_bounds__(256) k_horfft_fwd4(KGrid g, const double2 *__restrict__ tw, const double2 *__restrict__ twh,
                                                      HorJobs jobs) {
@@ -264,8 +265,8 @@ __global__ void __launch_bounds__(256) k_horfft_fwd4(KGrid g, const double2 *__r
   }
 }
 
-// HORFFT backward, in place: PFP m < NTCHOPDIM -> PPP slots (merge as in
-// k_horfft_bwd, then an inverse length-NTH transform).
+// HORFFT backward, in place: PFP m < NTCHOPDIM -> PPP slots (merge of
+// X_j and X_{N-j}, then an inverse length-NTH transform).
 template <int R1, int R2>
 __global__ void __launch_bounds__(256) k_horfft_bwd4(KGrid g, const double2 *__restrict__ tw, const double2 *__restrict__ twh,
                                                      HorJobs jobs) {
@@ -388,12 +389,16 @@ int launch_verfft_bwd(mlg_ctx *c, const double2 *in, double2 *out) { return laun
 // what it gains smaller ones (28 -> 20 at 200x256x64, 53 MB; 27 -> 15 at
 // NTH = 32, where the runs are longer); NTH = 512 has no other kernel of that
 // kind and the mixed-radix one takes as long (106 us at 192x512x128) or
-// longer (12.8 against 7.8 at 64x512x16).
+// longer (12.8 against 7.8 at 64x512x16).  Forward at NTH = 16 keeps its
+// rounding: the lines' error is the smaller one (1.39e-16 rms against 1.48e-16)
+// and their time too (7.9 us against 19.7 at 384x16x256), but the check of
+// PROJECT's transpose at 32x16x16 compares sums that cancel by six digits, and
+// which of two such roundings meets its bar is chance.
 static bool horfft_on_lines(const KGrid &g, const HorJobs &j, bool fwd) {
   const int n = g.nth;
   if (n < 16 || n > 512 || (n & (n - 1)) || j.s0 != 1.0 || j.s1 != 1.0 || j.wr) return false;
   const double bytes = 16.0 * g.ndimr * g.ndimth * (double)g.ndimx * j.n;
-  return !fwd || n <= 32 || n == 512 || bytes <= 64e6;
+  return !fwd || n == 32 || n == 512 || (n > 16 && bytes <= 64e6);
 }
 int launch_horfft_fwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double s1) {
   if (n < 1 || n > MAX_HOR_JOBS) return MLG_E_ARG;

@@ -287,7 +287,7 @@ __device__ __forceinline__ void forward(const Ctx &x, const KGrid &g, const doub
 
 }  // namespace w256
 
-// Same products as k_fused_products, in the same floating-point operations.
+// The products are the separate kernels' floating-point operations.
 // The outputs r N_r, r N_theta, N_z overwrite ror, rop, oz in the callers,
 // so all three are read before the first of them is written.  The fields go
 // to physical space one at a time; at most five stay in registers, and one
