@@ -357,7 +357,6 @@ int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd) {
   const int lg = any_lgp(f.n, copies), P = 1 << lg;
   const dim3 grid(xcd_grid((g.ndimr + P - 1) / P * g.ndimx * jobs.n));
   const size_t lds = sizeof(double2) * ((size_t)f.n << lg) * copies;
-  KScope ks(c, fwd ? K_HORFFT_FWD : K_HORFFT_BWD, jobs.n * 16.0 * g.nr * g.nx * (double)(g.nth + g.ntchopdim));
   if (fwd)
     hipLaunchKernelGGL(k_horfft_fwd_any, grid, dim3(256), lds, c->stream, g, f, lg, c->d.tw_t, c->d.tw_h, jobs);
   else

@@ -321,8 +321,8 @@ int launch_horfft_bwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double 
 static inline bool fft4_length(int n) { return n >= 2 && n <= 256 && (n & (n - 1)) == 0; }
 int fft_any_setup(int n, FftAny *f);  // allocates f's device tables
 int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd);
-int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd);
-// NTH = 16, 32, .. 512 without scale factors, on the lines of the fused products (k_fused.hip)
+int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd);  // inside the caller's KScope
+// NTH = 16, 32, .. 512 without scale factors, on the lines of the fused products (k_fused.hip); inside the caller's KScope
 int launch_horfft_line(mlg_ctx *c, const HorJobs &jobs, bool fwd);
 // theta lengths with a register-resident products kernel (k_fused.hip)
 static inline bool fused_line_length(int n) { return n >= 2 && n <= 512 && (n & (n - 1)) == 0; }
