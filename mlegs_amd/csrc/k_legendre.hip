@@ -503,6 +503,13 @@ k_rtran_bwd_grouped(const BwdJob *__restrict__ jb, const int *__restrict__ b0, i
   }
 }
 
+// sum over the jobs and the modes of g of NRCHOPS(m)
+static double bwd_rows(const KGrid &g, const TransformJobs &jobs, int n) {
+  double s = 0;
+  for (int j = 0; j < n; j++)
+    for (int m = g.mlo; m < g.mlo + g.mcnt; m++) s += nrchops_of(g.nrchop + jobs.dn[j], m * g.minc);
+  return s;
+}
 int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double *const *ln_in, double2 *const *out,
                        const int *dn) {
   if (n < 1 || n > MAX_TRANSFORM_JOBS) return MLG_E_ARG;
@@ -515,23 +522,21 @@ int launch_rtran_bwd_n(mlg_ctx *c, int n, const double2 *const *in, const double
     jobs.dn[i] = dn ? dn[i] : 0;
   }
   // 2 NR sum_m NRCHOPS(m) NXCHOPDIM flops per field (real table x complex data, folded)
-  const double per_k = n * 2.0 * g.nr * g.nxchopdim;
+  const double per_k = 2.0 * g.nr * g.nxchopdim;
   if (!c->leg_split) {
     if (c->rec) return sweep_defer_bwd(c, g, jobs, n);
-    KScope ks(c, K_RTRAN_BWD, per_k * (double)sum_nrchops(c));
-    const int rc = launch_bwd_fp64(c, g, jobs, n);
-    if (rc) return rc;
-    return 0;
+    KScope ks(c, K_RTRAN_BWD, per_k * bwd_rows(g, jobs, n));
+    return launch_bwd_fp64(c, g, jobs, n);
   }
   KGrid g0, g1;
   split_modes(c, g, g0, g1);
   {
-    KScope ks(c, K_RTRAN_BWD, per_k * split_fp64_sum(g0, 1));
+    KScope ks(c, K_RTRAN_BWD, per_k * bwd_rows(g0, jobs, n));
     const int rc = launch_bwd_fp64(c, g0, jobs, n);
     if (rc) return rc;
   }
   if (g1.mcnt > 0) {
-    KScope ks(c, K_RTRAN_BWD, per_k * ((double)sum_nrchops(c) - split_fp64_sum(g0, 1)));
+    KScope ks(c, K_RTRAN_BWD, per_k * bwd_rows(g1, jobs, n));
     hipLaunchKernelGGL(k_rtran_bwd_split, dim3(xcd_grid(rtran_bwd_tiles<64, 64>(g1, n))), dim3(256), 0, c->stream, g1,
                        c->d.pf_sb, jobs, n, c->d.lnx, c->d.pf_eb);
     MLG_CHECK_HIP(hipGetLastError());

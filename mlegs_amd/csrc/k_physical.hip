@@ -103,7 +103,7 @@ int launch_vdot(mlg_ctx *c, const double2 *rar, const double2 *rap, const double
                 const double2 *bz, double2 *out, double sign) {
   KGrid g = kgrid(c);
   long total = (long)g.ndimr * g.ndimth * g.ndimx;
-  KScope ks(c, K_PRODUCTS, 16.0 * total * 7);
+  KScope ks(c, K_PRODUCTS, 16.0 * g.nr * g.nth * g.ndimx * 7);
   hipLaunchKernelGGL(k_vdot, dim3(grid_for(total)), dim3(256), 0, c->stream, g, c->d.r, rar, rap, az, rbr, rbp, bz, out, sign,
                      total);
   MLG_CHECK_HIP(hipGetLastError());

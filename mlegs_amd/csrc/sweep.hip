@@ -439,8 +439,9 @@ static int sweep_build(mlg_sweep *w) {
     q.pos = l / ncls;
     for (const BwdJob &j : pj[l]) {
       long sk = 0;
-      for (int m = j.g.mlo; m < j.g.mlo + j.g.mcnt; m++) sk += nrchops_of(j.g.nrchop, m * j.g.minc);
-      w->gflop += 2.0 * j.g.nr * j.g.nxchopdim * j.nj * (double)sk * 1e-9;
+      for (int f = 0; f < j.nj; f++)
+        for (int m = j.g.mlo; m < j.g.mlo + j.g.mcnt; m++) sk += nrchops_of(j.g.nrchop + j.jobs.dn[f], m * j.g.minc);
+      w->gflop += 2.0 * j.g.nr * j.g.nxchopdim * (double)sk * 1e-9;
     }
     gjobs += q.njobs;
     at_pos[q.pos].push_back((int)w->gl.size());
