@@ -260,7 +260,12 @@ extern "C" int mlg_init(const mlg_params *p, mlg_ctx **out) {
     hv.insert(hv.end(), G.hd_x.begin(), G.hd_x.end());
     RET(upload(&d.hv, hv));
   }
-  MLG_CHECK_HIP(hipMalloc((void **)&d.red, sizeof(double) * (4 * (size_t)G.ntchop * G.nxchopdim + 2)));
+  {
+    const size_t nred = 4 * (size_t)G.ntchop * G.nxchopdim + 2;
+    RET(upload(&d.red, std::vector<double>(nred + LNV + IT1_FIXED + 2 * (size_t)G.nxchopdim, 0.0)));
+    d.lnv = d.red + nred;
+    d.it1 = d.lnv + LNV;
+  }
   MLG_CHECK_HIP(hipMalloc((void **)&d.vproj, sizeof(double) * ((size_t)G.nrchopdim + 1)));
   MLG_CHECK_HIP(hipMalloc((void **)&d.err, sizeof(int)));
   MLG_CHECK_HIP(hipMemset(d.err, 0, sizeof(int)));
@@ -1148,34 +1153,42 @@ extern "C" int mlg_energy(const mlg_field *psi, const mlg_field *chi, const mlg_
   if (bln != 0.0) return 13;
   if (psi->space != MLG_FFF || chi->space != MLG_FFF) return 3;
   if (b->space != MLG_FFF) return 2;
-  constexpr int NF = 5;
-  Temps T(c);
-  mlg_field *zero = T.get(), *ln2 = T.buffer(), *a = T.buffer(), *d2 = T.buffer(), *dh = T.buffer(), *t[NF];
-  for (auto &q : t) q = T.buffer();
-  RET(T.ready());
   const int nt = G.ntchop, nxc = G.nxchop, nxd = G.nxchopdim;
   const size_t na = (size_t)nt * nxd;
-  double *dall = c->d.red;  // [4][nt*nxd]
-  RET(launch_zero(c, (double2 *)dall, (long)(4 * na / 2 + 1)));
-  RET(launch_set_ln(c, ln2->ln, psi->ln, 2.0, 0.0));
-  RET(mlg_chopset(c, 3));
-  // psi, DELSQH(psi, 2 LN), DEL2(chi), DELSQH(chi) and b, without their LN,
-  // share one backward launch and one copy to the host
-  const double2 *in[NF] = {psi->e, a->e, d2->e, dh->e, b->e};
-  const double *ln[NF];
-  double2 *pff[NF];
-  for (int q = 0; q < NF; q++) {
-    ln[q] = zero->ln;
-    pff[q] = t[q]->e;
+  double *dall = c->d.red, *lnv = c->d.lnv;  // [4][nt*nxd]; [zero, 2 LN, the fields' own]
+  // psi, DELSQH(psi, 2 LN), DEL2(chi), DELSQH(chi) and b, without their LN, to
+  // PFF, in four buffers
+  Temps T(c);
+  Pack P(T, 4);
+  double2 *p[5], *a, *d2, *dh;
+  for (auto &q : p) q = P.take(c->n_pff);
+  a = P.take(c->n_fff), d2 = P.take(c->n_fff), dh = P.take(c->n_fff);
+  PffProducts q{c, !P.ok};
+  if (q.lean) {
+    P.grow(4);
+    a = d2 = dh = P.e[0];
+    p[0] = p[2] = P.e[1], p[1] = p[3] = P.e[2], p[4] = P.e[3];
   }
-  int rc = launch_delsqh(c, psi->e, ln2->ln, a->e, a->ln);
-  if (!rc) rc = mlg_del2(chi, d2);
-  if (!rc) rc = mlg_delsqh(chi, dh);
-  if (!rc) rc = launch_rtran_bwd_n(c, NF, in, ln, pff);
-  if (!rc) rc = launch_energy_terms(c, pff[0], pff[1], 0, dall);
-  if (!rc) rc = launch_energy_terms(c, pff[2], pff[3], 0, dall + na);
-  if (!rc) rc = launch_energy_terms(c, pff[4], pff[3], 0, dall + 2 * na);
-  if (!rc) rc = launch_energy_terms(c, pff[4], nullptr, 1, dall + 3 * na);
+  RET(T.ready());
+  RET(launch_zero(c, (double2 *)dall, (long)(4 * na / 2 + 1)));
+  RET(launch_set_ln(c, lnv + 1, psi->ln, 2.0, 0.0));
+  RET(mlg_chopset(c, 3));
+  int rc = launch_delsqh(c, psi->e, lnv + 1, a, lnv + 2);
+  q.field(a, lnv, p[0]);
+  q.field(psi->e, lnv, p[1]);
+  q.term(p[1], p[0], 0, dall);
+  if (!rc) rc = q.group();
+  if (!rc) rc = launch_check_top_m1(c, chi->e);
+  if (!rc) rc = launch_del2(c, chi->e, chi->ln, d2, lnv + 3);
+  q.field(d2, lnv, p[2]);
+  if (!rc) rc = q.group();
+  if (!rc) rc = launch_delsqh(c, chi->e, chi->ln, dh, lnv + 4);
+  q.field(dh, lnv, p[3]);
+  q.field(b->e, lnv, p[4]);
+  q.term(p[2], p[3], 0, dall + na);
+  q.term(p[4], p[3], 0, dall + 2 * na);
+  q.term(p[4], nullptr, 1, dall + 3 * na);
+  if (!rc) rc = q.flush();
   mlg_chopset(c, -3);
   RET(rc);
   std::vector<double> h(4 * na);

@@ -57,26 +57,26 @@ struct It1 {
   const double2 *abs;              // ABSVEC2 summed over z, [theta][r]
   double p00;                      // P_0^0, normalised
   int na, nn;                      // nn: NRCHOP
+  long nfff;                       // stored coefficients
   double minc;
 };
 // VALVOR, VALZMO, the INTEG_P sum, 3 PRODCTs, 4 moments (1, x, y, r^2), then
-// CALCAT1's |value| per k of psi and of chi; a block of 1024 threads each
-constexpr int IT1_AT1 = 10;
-__global__ void __launch_bounds__(1024) k_it1_values(KGrid g, It1 v, double *out) {
+// CALCAT1's |value| per k of psi and of chi, from value q0 on; a block of 1024 threads each
+__global__ void __launch_bounds__(1024) k_it1_values(KGrid g, It1 v, double *out, int q0) {
   __shared__ double2 S[1024];
-  const int t = threadIdx.x, q = blockIdx.x;
+  const int t = threadIdx.x, q = q0 + blockIdx.x;
   double2 s = make_double2(0.0, 0.0);
   if (q < 2) {
     if (t == 0) s.x = -(q == 0 ? v.dp : v.dc)[0].x;
   } else if (q == 2) {
     // the first NR stored coefficients in storage order
-    for (int i = t; i < g.nr; i += 1024) {
+    for (int i = t; i < min((long)g.nr, v.nfff); i += 1024) {
       const double om = 1 - v.x[i];
       s.x += v.ang[i].x / (om * om) * v.w[i];
     }
   } else if (q < 6) {
     for (int i = t; i < v.na; i += 1024) s.x += v.terms[(size_t)(q - 3) * v.na + i];
-  } else if (q < IT1_AT1) {
+  } else if (q < IT1_FIXED) {
     // The (0, 0, 0) coefficient of ABSVEC2 times the factor: HORFFT's m = 0
     // and VERFFT's k = 0 are means, RTRAN's n = 0 the Gauss sum with P_0^0.
     // theta = 2 pi j / NTH in the real slots, 2 pi (j + 1/2) / NTH in the imaginary ones
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(1024) k_it1_values(KGrid g, It1 v, double *out
       s.x += v.w[r] * rad * (a.x + a.y);
     }
   } else {
-    const int k = (q - IT1_AT1) % g.nxchopdim, fi = (q - IT1_AT1) / g.nxchopdim;
+    const int k = (q - IT1_FIXED) % g.nxchopdim, fi = (q - IT1_FIXED) / g.nxchopdim;
     const double2 *col = v.f[fi] + (size_t)g.nrchopdim * g.ntchopdim * k;
     for (int n = t; n < v.nn; n += 1024) {
       s.x += col[n].x * v.at1[n];
@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(1024) k_it1_values(KGrid g, It1 v, double *out
     __syncthreads();
   }
   if (t) return;
-  if (q >= IT1_AT1) out[q] = hypot(S[0].x, S[0].y);
+  if (q >= IT1_FIXED) out[q] = hypot(S[0].x, S[0].y);
   else if (q >= 6) out[q] = S[0].x * v.p00 / (2.0 * g.nth * g.nx);
   else out[q] = S[0].x;
 }
@@ -118,68 +118,96 @@ __global__ void __launch_bounds__(1024) k_it1_values(KGrid g, It1 v, double *out
 // four fields transformed for one coefficient each (MULRCOSTH / MULRSINTH /
 // MULR2 and INTEG), and the eight fields that leave FFF share one backward
 // launch.  At 128x64x64 the section with the energies and ENEMON, which share
-// launches in the same way, takes 0.39 ms where they took 1.86.
+// launches in the same way, takes 0.39 ms where they took 1.86.  The fields
+// lie in seven buffers, one routine's at a time where they would not fit.
 static int diagnost_it1(const mlg_field *psi, const mlg_field *chi, double *out) {
   mlg_ctx *c = psi->ctx;
   const Grid &G = c->g;
   const double pi = 3.14159265358979323846;
-  constexpr int NF = 8;
+  const long nf = c->n_fff, np = c->n_pff;
+  const size_t na = (size_t)G.ntchop * G.nxchopdim;
+  // LN: zero, 2 psi's, then those of a, d2c, dc, dp, ror, rop, oz and scratch
+  double *const lnv = c->d.lnv, *const l2 = lnv + 1, *const la = lnv + 2, *const ld2 = lnv + 3, *const ldc = lnv + 4,
+               *const ldp = lnv + 5, *const lr = lnv + 6, *const lp = lnv + 7, *const lo = lnv + 8, *const lx = lnv + 9;
   Temps T(c);
-  mlg_field *ror = T.buffer(), *rop = T.buffer(), *oz = T.buffer(), *a = T.buffer(), *d2c = T.buffer(), *dc = T.buffer(),
-            *dp = T.buffer(), *ang = T.buffer(), *m1 = T.buffer(), *t[NF];
-  for (auto &q : t) q = T.buffer();
+  Pack P(T, 7, 3);
+  // p: PFF of a, psi, d2c, dc, dp and the vorticity; the first three buffers
+  // take the vorticity in physical space once what is packed there is done with
+  double2 *p[8], *dp, *dc, *ang, *sum, *a, *d2c, *ror, *rop, *oz, *m1, *vor[3];
+  for (int q = 0; q < 8; q++) p[q] = P.take(np, q >= 5);
+  dp = P.take(nf, true), dc = P.take(nf, true), ang = P.take(nf, true), sum = P.take((long)G.nr * G.nth, true);
+  a = P.take(nf), d2c = P.take(nf), ror = P.take(nf), rop = P.take(nf), oz = P.take(nf);
+  m1 = p[0];
+  PffProducts q{c, !P.ok};
+  if (q.lean) {
+    P.grow(6);
+    dp = p[7] = P.e[0];
+    dc = ror = P.e[1];
+    ang = a = d2c = rop = P.e[2];
+    p[0] = p[2] = m1 = p[5] = sum = P.e[3];
+    p[1] = p[3] = oz = P.e[4];
+    p[4] = p[6] = P.e[5];
+  }
+  for (int i = 0; i < 3; i++) vor[i] = q.lean ? (i == 0 ? ror : i == 1 ? rop : oz) : P.e[i];
   RET(T.ready());
-  // PC2VOR(..., 'H'): ROR, ROP of PC2VOR, OZ/(1-x)^2 = -DELSQH(psi);
-  // PC2VEL(..., 'H'): only UZ/(1-x)^2 = -DELSQH(chi) is read (INTEG)
-  RET(mlg_pc2vor(psi, chi, ror, rop, ang));
-  RET(mlg_delsqh(psi, dp));  // LN 0
-  RET(mlg_delsqh(chi, dc));
-  RET(launch_set_ln(c, m1->ln, psi->ln, 2.0, 0.0));
-  RET(launch_delsqh(c, psi->e, m1->ln, a->e, a->ln));
-  RET(mlg_del2(chi, d2c));
+  It1 v;
+  v.f[0] = psi->e, v.f[1] = chi->e;
+  v.at1 = c->d.at1, v.x = c->d.x, v.w = c->d.w, v.r2 = c->d.r, v.terms = c->d.red;
+  v.dp = dp, v.dc = dc, v.ang = ang, v.abs = sum;
+  v.p00 = G.pf[0];
+  v.na = (int)na, v.nn = G.nrchop, v.nfff = nf;
+  v.minc = G.p.minc;
+  const int nxd = G.nxchopdim, nval = IT1_FIXED + 2 * nxd, nfff = 3;  // the first nfff values read FFF fields
+  auto values = [&](int q0, int q1) -> int {
+    hipLaunchKernelGGL(k_it1_values, dim3(q1 - q0), dim3(1024), 0, c->stream, kgrid(c), v, c->d.it1, q0);
+    MLG_CHECK_HIP(hipGetLastError());
+    return 0;
+  };
+  // PC2VOR(..., 'H')'s OZ/(1-x)^2 = -DELSQH(psi); PC2VEL(..., 'H'): only
+  // UZ/(1-x)^2 = -DELSQH(chi) is read (INTEG)
+  RET(launch_delsqh(c, psi->e, psi->ln, dp, ldp));
+  RET(launch_delsqh(c, chi->e, chi->ln, dc, ldc));
   // VALANG = -INTEG_P(XXDX(psi with LN = 0)).  INTEG_P (src/mod_march.f90:
   // 3649-3682) sums Re(F%E(:NR,1,1)) w / (1-x)^2 of its FFF argument: the
   // first NR stored coefficients in storage order (past the m = 0, k = 0
   // column when NRCHOPDIM < NR), as the reference reads them
-  RET(launch_band3(c, 1, psi->e, dp->ln, ang->e, ang->ln));
-  // OZH (1-x)^2 = OZ, but for its sign, which ABSVEC2 squares
-  RET(launch_band3(c, 0, dp->e, dp->ln, m1->e, m1->ln));
-  RET(launch_band3(c, 0, m1->e, m1->ln, oz->e, oz->ln));
-  // to PFF: DELSQH(psi, 2 LN), psi with LN = 0, DEL2(chi), DELSQH(chi), DELSQH(psi) and the vorticity
-  const double2 *in[NF] = {a->e, psi->e, d2c->e, dc->e, dp->e, ror->e, rop->e, oz->e};
-  const double *ln[NF] = {a->ln, dp->ln, d2c->ln, dc->ln, dp->ln, ror->ln, rop->ln, oz->ln};
-  double2 *pff[NF];
-  for (int q = 0; q < NF; q++) pff[q] = t[q]->e;
-  RET(launch_rtran_bwd_n(c, NF, in, ln, pff));
+  RET(launch_band3(c, 1, psi->e, lnv, ang, lx));
+  if (q.lean) RET(values(0, nfff));
   // VALENE = -PRODCT(DELSQH(psi, 2 LN), psi) + PRODCT(DELSQH(chi), DEL2(chi)),
   // VALHEL = 2 PRODCT(DELSQH(psi), DEL2(chi))
-  const size_t na = (size_t)G.ntchop * G.nxchopdim;
-  RET(launch_energy_terms(c, pff[0], pff[1], 0, c->d.red));
-  RET(launch_energy_terms(c, pff[3], pff[2], 0, c->d.red + na));
-  RET(launch_energy_terms(c, pff[4], pff[2], 0, c->d.red + 2 * na));
+  RET(launch_set_ln(c, l2, psi->ln, 2.0, 0.0));
+  RET(launch_delsqh(c, psi->e, l2, a, la));
+  q.field(a, la, p[0]);
+  q.field(psi->e, lnv, p[1]);
+  q.term(p[0], p[1], 0, c->d.red);
+  RET(q.group());
+  RET(launch_check_top_m1(c, chi->e));
+  RET(launch_del2(c, chi->e, chi->ln, d2c, ld2));
+  q.field(d2c, ld2, p[2]);
+  q.field(dc, ldc, p[3]);
+  q.field(dp, ldp, p[4]);
+  q.term(p[3], p[2], 0, c->d.red + na);
+  q.term(p[4], p[2], 0, c->d.red + 2 * na);
+  RET(q.group());
+  // the vorticity: ROR, ROP of PC2VOR; OZH (1-x)^2 = OZ, but for its sign,
+  // which ABSVEC2 squares
+  RET(launch_pc2vor(c, psi->e, psi->ln, chi->e, chi->ln, ror, rop, oz, lr, lp, lx));
+  RET(launch_band3(c, 0, dp, ldp, m1, lx));
+  RET(launch_band3(c, 0, m1, lx, oz, lo));
+  q.field(ror, lr, p[5]);
+  q.field(rop, lp, p[6]);
+  q.field(oz, lo, p[7]);
+  RET(q.flush());
   // CALCXY: the vorticity to physical space
-  const double2 *vin[3] = {pff[5], pff[6], pff[7]};
-  double2 *vor[3] = {ror->e, rop->e, oz->e};
+  const double2 *vin[3] = {p[5], p[6], p[7]};
   RET(launch_verfft_bwd_n(c, 3, vin, vor));
   RET(launch_horfft_bwd_n(c, 3, vor, 1.0, 1.0, nullptr));
-  KGrid g = kgrid(c);
-  hipLaunchKernelGGL(k_absvec2_sum, dim3((g.nr + 63) / 64, g.nth), dim3(256), 0, c->stream, g, ror->e, rop->e, oz->e, c->d.r,
-                     c->d.x, t[0]->e);
+  hipLaunchKernelGGL(k_absvec2_sum, dim3((G.nr + 63) / 64, G.nth), dim3(256), 0, c->stream, kgrid(c), vor[0], vor[1], vor[2],
+                     c->d.r, c->d.x, sum);
   MLG_CHECK_HIP(hipGetLastError());
-  const int nxd = G.nxchopdim, nval = IT1_AT1 + 2 * nxd;
-  It1 v;
-  v.dp = dp->e, v.dc = dc->e, v.ang = ang->e;
-  v.f[0] = psi->e, v.f[1] = chi->e;
-  v.at1 = c->d.at1, v.x = c->d.x, v.w = c->d.w, v.r2 = c->d.r, v.terms = c->d.red;
-  v.abs = t[0]->e;
-  v.p00 = G.pf[0];
-  v.na = (int)na, v.nn = G.nrchop;
-  v.minc = G.p.minc;
-  double *res = reinterpret_cast<double *>(t[1]->e);  // nval doubles: far fewer than a field's
-  hipLaunchKernelGGL(k_it1_values, dim3(nval), dim3(1024), 0, c->stream, g, v, res);
-  MLG_CHECK_HIP(hipGetLastError());
+  RET(values(q.lean ? nfff : 0, nval));
   std::vector<double> h(nval);
-  MLG_CHECK_HIP(hipMemcpyAsync(h.data(), res, sizeof(double) * nval, hipMemcpyDeviceToHost, c->stream));
+  MLG_CHECK_HIP(hipMemcpyAsync(h.data(), c->d.it1, sizeof(double) * nval, hipMemcpyDeviceToHost, c->stream));
   MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
   // INTEG (src/mod_scalar3.f90:312-353): 4 pi ZLEN ELL^2 Re(f(0,0,0)) NORM(0, m=0)
   const double fi = 4.0 * pi * G.zlen * G.ell2;
@@ -190,7 +218,7 @@ static int diagnost_it1(const mlg_field *psi, const mlg_field *chi, double *out)
   out[4] = -(2.0 * pi * G.zlen * G.ell2 * h[2]);
   // psi and chi at r = infinity (CALCAT1, src/mod_scalar3.f90:286-310)
   for (int q = 0; q < 2; q++) {
-    const double *at = h.data() + IT1_AT1 + q * nxd;
+    const double *at = h.data() + IT1_FIXED + q * nxd;
     out[5 + 2 * q] = at[0];
     out[6 + 2 * q] = *std::max_element(at, at + nxd) - *std::min_element(at, at + nxd);
   }

@@ -53,6 +53,7 @@ struct FusedAny {
   long lds = 0;  // bytes a block
 };
 
+constexpr int LNV = 16, IT1_FIXED = 10;
 // Device copies of the tables and scratch.
 struct DevTables {
   double *pf = nullptr;       // [mm][n][i]  (i fastest), npf rows
@@ -65,7 +66,9 @@ struct DevTables {
   double2 *tw_t = nullptr;    // e^{-2 pi i j / NTH}, j < NTH
   double2 *tw_h = nullptr;    // e^{-2 pi i j / (2 NTH)}, j <= NTH
   double *hv = nullptr;       // [hv_r | hv_t | hv_x | hd_r | hd_t | hd_x]
-  double *red = nullptr;      // reduction scratch
+  double *red = nullptr;      // reduction scratch: 4 values per (m, k), then
+  double *lnv = nullptr;      // LNV log-term coefficients of diagnostics' fields (lnv[0] stays 0), then
+  double *it1 = nullptr;      // IT1_FIXED + 2 NXCHOPDIM results of the every-IT1 section
   double *vproj = nullptr;    // VEL2PLN projections [NRCHOPDIM]
   double *cvdt = nullptr;     // PROJECT tables composed with RTRAN (built on first use)
   // Split hi/lo FP32 forms of the Legendre tables (built when the split
@@ -569,6 +572,69 @@ struct Temps {
   ~Temps() {
     for (auto *f : v) pool_give(c, f);
   }
+};
+
+// Arrays of one call in as few pooled buffers as they fit, at most `cap`: a
+// buffer holds the largest space's field, several of FFF or PFF.  The first
+// `lo` buffers are taken at once; arrays that are `live` do not go there.
+// ok is false once an array had no room.
+struct Pack {
+  Temps &T;
+  const int cap, lo;
+  bool ok = true;
+  std::vector<double2 *> e;  // the buffers
+  std::vector<long> used;
+  Pack(Temps &t, int cap_, int lo_ = 0) : T(t), cap(cap_), lo(lo_) { grow(lo); }
+  void grow(int n) {
+    while ((int)e.size() < n) {
+      mlg_field *f = T.buffer();
+      e.push_back(f ? f->e : nullptr);
+      used.push_back(0);
+    }
+  }
+  double2 *take(long n, bool live = false) {
+    n = (n + 7) / 8 * 8;  // whole cache lines
+    for (size_t i = live ? lo : 0;; i++) {
+      if (i == e.size()) {
+        if ((int)i >= cap || n > T.c->n_max) {
+          ok = false;
+          return nullptr;
+        }
+        grow((int)i + 1);
+      }
+      if (!e[i]) return nullptr;  // T.ready() reports it
+      if (used[i] + n > T.c->n_max) continue;
+      used[i] += n;
+      return e[i] + (used[i] - n);
+    }
+  }
+};
+
+// Fields of a diagnostic on their way to PFF and the per-(m, k) products of
+// the results.  All of them in one backward launch, or, `lean`, a group at a
+// time so that a group's buffers serve the next one: the diagnostics choose
+// that where their fields would not fit the buffers that it takes.
+struct PffProducts {
+  mlg_ctx *c;
+  bool lean;
+  int n = 0, nt = 0;
+  const double2 *in[MAX_TRANSFORM_JOBS];
+  const double *ln[MAX_TRANSFORM_JOBS];
+  double2 *out[MAX_TRANSFORM_JOBS];
+  struct Term {
+    const double2 *a, *b;
+    int l2;
+    double *sums;
+  } t[4];
+  void field(const double2 *i, const double *l, double2 *o) { in[n] = i, ln[n] = l, out[n++] = o; }
+  void term(const double2 *a, const double2 *b, int l2, double *sums) { t[nt++] = Term{a, b, l2, sums}; }
+  int flush() {
+    int rc = n ? launch_rtran_bwd_n(c, n, in, ln, out) : 0;
+    for (int i = 0; i < nt && !rc; i++) rc = launch_energy_terms(c, t[i].a, t[i].b, t[i].l2, t[i].sums);
+    n = nt = 0;
+    return rc;
+  }
+  int group() { return lean ? flush() : 0; }
 };
 
 }  // namespace mlg

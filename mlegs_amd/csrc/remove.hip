@@ -250,25 +250,36 @@ static int enemon(const mlg_field *psi, const mlg_field *chi, double *em, double
   mlg_ctx *c = psi->ctx;
   const Grid &G = c->g;
   const int nt = G.ntchop, nxc = G.nxchop;
-  // DELSQH(psi, 2 LN), psi with LN = 0, DEL2(chi) and DELSQH(chi) share one
-  // backward launch, and the two products one copy to the host
-  constexpr int NF = 4;
-  Temps T(c);
-  mlg_field *zero = T.get(), *ln2 = T.buffer(), *a = T.buffer(), *d2 = T.buffer(), *dh = T.buffer(), *t[NF];
-  for (auto &q : t) q = T.buffer();
-  RET(T.ready());
-  RET(launch_set_ln(c, ln2->ln, psi->ln, 2.0, 0.0));  // W1%LN = 2 PSI%LN
-  RET(launch_delsqh(c, psi->e, ln2->ln, a->e, a->ln));
-  RET(mlg_del2(chi, d2));
-  RET(mlg_delsqh(chi, dh));
-  const double2 *in[NF] = {a->e, psi->e, d2->e, dh->e};
-  const double *ln[NF] = {a->ln, zero->ln, d2->ln, dh->ln};
-  double2 *pff[NF];
-  for (int q = 0; q < NF; q++) pff[q] = t[q]->e;
-  RET(launch_rtran_bwd_n(c, NF, in, ln, pff));
   const size_t na = (size_t)nt * G.nxchopdim;
-  RET(launch_energy_terms(c, pff[0], pff[1], 0, c->d.red));
-  RET(launch_energy_terms(c, pff[3], pff[2], 0, c->d.red + na));
+  double *lnv = c->d.lnv;  // [zero, 2 LN, the fields' own]
+  // DELSQH(psi, 2 LN), psi with LN = 0, DEL2(chi) and DELSQH(chi) to PFF, in
+  // three buffers
+  Temps T(c);
+  Pack P(T, 3);
+  double2 *p[4], *a, *d2, *dh;
+  for (auto &q : p) q = P.take(c->n_pff);
+  a = P.take(c->n_fff), d2 = P.take(c->n_fff), dh = P.take(c->n_fff);
+  PffProducts q{c, !P.ok};
+  if (q.lean) {
+    P.grow(3);
+    a = d2 = dh = P.e[0];
+    p[0] = p[2] = P.e[1], p[1] = p[3] = P.e[2];
+  }
+  RET(T.ready());
+  RET(launch_set_ln(c, lnv + 1, psi->ln, 2.0, 0.0));  // W1%LN = 2 PSI%LN
+  RET(launch_delsqh(c, psi->e, lnv + 1, a, lnv + 2));
+  q.field(a, lnv + 2, p[0]);
+  q.field(psi->e, lnv, p[1]);
+  q.term(p[0], p[1], 0, c->d.red);
+  RET(q.group());
+  RET(launch_check_top_m1(c, chi->e));
+  RET(launch_del2(c, chi->e, chi->ln, d2, lnv + 3));
+  q.field(d2, lnv + 3, p[2]);
+  RET(q.group());
+  RET(launch_delsqh(c, chi->e, chi->ln, dh, lnv + 4));
+  q.field(dh, lnv + 4, p[3]);
+  q.term(p[3], p[2], 0, c->d.red + na);
+  RET(q.flush());
   std::vector<double> h(2 * na), mk, am(nt), ak(nxc);
   MLG_CHECK_HIP(hipMemcpyAsync(h.data(), c->d.red, sizeof(double) * 2 * na, hipMemcpyDeviceToHost, c->stream));
   MLG_CHECK_HIP(hipStreamSynchronize(c->stream));
