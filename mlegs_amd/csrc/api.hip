@@ -870,58 +870,62 @@ extern "C" int mlg_project(mlg_field *rur, mlg_field *rup, mlg_field *uz, mlg_fi
 }
 
 // ------------------------------------------------------------------ Boussinesq terms
-// The seven FFF fields fs to PFP (TOFP without the theta transform) with one
-// RTRAN backward launch and one VERFFT backward launch, the FFF storage and
-// LN of the first three moving to keep[], together with GRAD's i m b and i k b in PFP (rbp, bz), which come
-// from one backward Legendre transform of b (b stays in FFF): the
-// z-transform multiplies by i m or i k as it loads.  The same linear maps as
-// GRAD then RTRAN, VERFFT, in another order.
-static int to_pfp_b(mlg_ctx *c, mlg_field *const *fs, const mlg_field *b, mlg_field *rbp, mlg_field *bz,
-                    mlg_field *const *keep) {
-  constexpr int n = 7;
-  for (int i = 0; i < n; i++)
-    if (fs[i]->space != MLG_FFF) return 2;
-  Temps T(c);
-  mlg_field *t[n + 1];
-  for (int i = 0; i <= n; i++) t[i] = T.buffer();
-  RET(T.ready());
+// Backward transforms of a right-hand side's fields, FFF to PFP (TOFP without
+// the theta transform): Legendre job j takes in[j], ln[j] at NRCHOP + dn[j]
+// through PFF, the z-transform puts it to out[j].  The job `twice` has two
+// results: i m times it in out[twice], i k times it in out[twice + 1]; later
+// jobs' results follow.  The PFF arrays share pooled buffers, at most five
+// (PFF is about a quarter of the largest space at the usual truncations: nine
+// jobs take three buffers), and the jobs go in as few batches as that allows,
+// two at the most for nine jobs.
+constexpr int PFF_BUFFERS = 5;
+struct ToPfp {
+  int n = 0, twice = -1;
   const double2 *in[MAX_TRANSFORM_JOBS];
   const double *ln[MAX_TRANSFORM_JOBS];
+  int dn[MAX_TRANSFORM_JOBS];
   double2 *out[MAX_TRANSFORM_JOBS];
-  for (int i = 0; i < n; i++) {
-    in[i] = fs[i]->e;
-    ln[i] = fs[i]->ln;
-    out[i] = t[i]->e;
-  }
-  in[n] = b->e;
-  ln[n] = b->ln;
-  out[n] = t[n]->e;
-  RET(launch_rtran_bwd_n(c, n + 1, in, ln, out));  // padding rows included
-  double *lns[n];
-  for (int i = 0; i < n; i++) {
-    swap_storage(fs[i], t[i]);
-    if (keep && i < 3) {  // the FFF storage and its LN move to keep[i]
-      std::swap(keep[i]->e, t[i]->e);
-      std::swap(keep[i]->ln, fs[i]->ln);
-      keep[i]->space = MLG_FFF;
+  double *zl[MAX_TRANSFORM_JOBS];  // LN coefficients cleared with the last results
+  int nzl = 0;
+  int run(mlg_ctx *c, std::initializer_list<mlg_field *> spare = {}) const {  // spare: buffers of the caller's to use first
+    Temps T(c);
+    Pack P(T, std::min(PFF_BUFFERS, n));
+    for (mlg_field *q : spare) P.give(q->e);
+    double2 *pff[MAX_TRANSFORM_JOBS];
+    int cap = 0;
+    while (cap < n && P.ok) {
+      pff[cap] = P.take(c->n_pff);
+      if (P.ok) cap++;
     }
-    fs[i]->space = MLG_PFF;
-    lns[i] = fs[i]->ln;
-    in[i] = fs[i]->e;
-    out[i] = t[i]->e;
+    if (cap == 0) {  // the rounding of Pack's arrays: one a buffer
+      P.grow(std::min(PFF_BUFFERS, n));
+      for (; cap < (int)P.e.size(); cap++) pff[cap] = P.e[cap];
+    }
+    RET(T.ready());
+    for (int j0 = 0; j0 < n; j0 += cap) {
+      const int nj = std::min(cap, n - j0);
+      RET(launch_rtran_bwd_n(c, nj, in + j0, ln + j0, pff, dn + j0));  // padding rows included
+      const double2 *zi[MAX_TRANSFORM_JOBS];
+      double2 *zo[MAX_TRANSFORM_JOBS];
+      int nz = 0;
+      unsigned dz = 0, dm = 0;
+      for (int j = j0; j < j0 + nj; j++) {
+        zi[nz] = pff[j - j0];
+        zo[nz] = out[twice >= 0 && j > twice ? j + 1 : j];
+        if (j == twice) {
+          dm = 1u << nz++;
+          zi[nz] = pff[j - j0];
+          zo[nz] = out[j + 1];
+          dz = 1u << nz;
+        }
+        nz++;
+      }
+      const bool last = j0 + nj == n;
+      RET(launch_verfft_bwd_n(c, nz, zi, zo, dz, dm, zl, last ? nzl : 0));
+    }
+    return 0;
   }
-  in[n] = t[n]->e;  // b in PFF, transformed twice: times i m and times i k
-  out[n] = rbp->e;
-  in[n + 1] = t[n]->e;
-  out[n + 1] = bz->e;
-  RET(launch_verfft_bwd_n(c, n + 2, in, out, 1u << (n + 1), 1u << n, lns, n));  // the PFF fields' LN = 0
-  for (int i = 0; i < n; i++) {
-    swap_storage(fs[i], t[i]);
-    fs[i]->space = MLG_PFP;
-  }
-  rbp->space = bz->space = MLG_PFP;
-  return 0;
-}
+};
 
 // CALC_BOUSSI_FORCE where the products are fused with the theta transforms.
 // W = TOFP(B) at NRCHOP and GRAD's i m b and i k b at NRCHOP+3 are Legendre
@@ -933,16 +937,19 @@ static int to_pfp_b(mlg_ctx *c, mlg_field *const *fs, const mlg_field *b, mlg_fi
 // With the AB2 step and VISC2's right-hand sides in one launch (visc_cn) a
 // step is twelve launches instead of twenty-seven: 178 -> 102 us at 64x32x32,
 // 225 -> 159 at 128x64x64.
+// Memory: the ten PFP fields lie in the three results and seven temporaries,
+// which hold the FFF fields before and the PFF ones after; with the PFF
+// buffers of the transforms that is twelve temporaries at most, as many as
+// the routines called one by one take.
 static int force_fused(const mlg_field *psi, const mlg_field *chi, const mlg_field *b, mlg_field *psin, mlg_field *chin,
                        mlg_field *bn) {
   mlg_ctx *c = psi->ctx;
   if (psi->space != MLG_FFF || chi->space != MLG_FFF || b->space != MLG_FFF) return 3;
   Temps T(c);
-  constexpr int NL = 9, NZ = 10;
-  mlg_field *f[NZ], *t[NL];  // rur rup uz ror rop oz rbr rbp bz w
-  for (auto &q : f) q = T.buffer();
-  for (auto &q : t) q = T.buffer();
-  mlg_field *w2 = T.buffer();
+  mlg_field *f[10] = {psin, chin};  // rur rup uz ror rop oz rbr rbp bz w
+  f[8] = bn;
+  for (auto &q : f)  // a result that is also an input is written at the end only
+    if (!q || q == psi || q == chi || q == b) q = T.buffer();
   RET(T.ready());
   VelVorOut vo;
   for (int i = 0; i < 7; i++) vo.e[i] = f[i]->e, vo.ln[i] = f[i]->ln;
@@ -950,38 +957,37 @@ static int force_fused(const mlg_field *psi, const mlg_field *chi, const mlg_fie
   vo.ln_b = b->ln;
   RET(mlg_chopset(c, 3));
   int rc = launch_pc2velvor(c, psi->e, psi->ln, chi->e, chi->ln, vo);  // with PC2VOR's DEL2 check
-  const double2 *in[NZ];
-  const double *ln[NL];
-  double2 *out[NZ];
-  const int dn[NL] = {0, 0, 0, 0, 0, 0, 0, 0, -3};
-  for (int i = 0; i < NL; i++) {
-    in[i] = i < 7 ? f[i]->e : b->e;
-    ln[i] = i < 7 ? f[i]->ln : b->ln;
-    out[i] = t[i]->e;
+  ToPfp tp;
+  tp.n = 9;
+  tp.twice = 7;
+  for (int i = 0; i < 9; i++) {
+    tp.in[i] = i < 7 ? f[i]->e : b->e;
+    tp.ln[i] = i < 7 ? f[i]->ln : b->ln;
+    tp.dn[i] = i == 8 ? -3 : 0;
   }
-  if (!rc) rc = launch_rtran_bwd_n(c, NL, in, ln, out, dn);
+  for (int i = 0; i < 10; i++) tp.out[i] = f[i]->e;
+  if (!rc) rc = tp.run(c);
   mlg_chopset(c, -3);
   RET(rc);
-  for (int i = 0; i < NZ; i++) {  // b's transform is read twice
-    in[i] = t[i < 8 ? i : i - 1]->e;
-    out[i] = f[i]->e;
-  }
-  RET(launch_verfft_bwd_n(c, NZ, in, out, 1u << 8, 1u << 7));
   {
     const double2 *pi[10];
     for (int i = 0; i < 10; i++) pi[i] = f[i]->e;
-    double2 *po[4] = {f[3]->e, f[4]->e, f[5]->e, bn->e};
+    double2 *po[4] = {f[3]->e, f[4]->e, f[5]->e, f[8]->e};
     RET(launch_fused_products(c, pi, po, 2 * c->g.p.omega, std::pow(c->g.p.bv0, 2.0), 1, bn->ln));  // and N_b's LN = 0
   }
-  bn->space = f[3]->space = f[4]->space = f[5]->space = MLG_PFP;
-  mlg_field *const pf4[4] = {f[3], f[4], f[5], bn};
-  RET(to_pff_n(c, 4, pf4));
-  RET(project_impl(f[3], f[4], f[5], psin, w2, 1, 0.0, nullptr, true));
+  // r N_r, r N_theta, N_z, N_b to PFF in the room of uz, rbr, rbp and w
+  mlg_field *const n[4] = {f[2], f[6], f[7], f[9]}, *const w2 = f[3];
+  {
+    const double2 *zi[4] = {f[3]->e, f[4]->e, f[5]->e, f[8]->e};
+    double2 *zo[4];
+    for (int i = 0; i < 4; i++) zo[i] = n[i]->e, n[i]->space = MLG_PFF;
+    RET(launch_verfft_fwd_n(c, 4, zi, zo));
+  }
+  RET(project_impl(n[0], n[1], n[2], psin, w2, 1, 0.0, nullptr, true));
   RET(solve_op(w2, chin, 1, 0.0, 0, 0.0, false));  // IDEL2LN
   double2 *const fix[2] = {psin->e, chin->e};
   // N_b to FFF; CHOPDO, and the fixes at infinity of PROJECT and IDEL2LN
-  RET(launch_rtran_fwd_fix(c, bn->e, w2->e, bn->ln, fix));
-  swap_storage(bn, w2);
+  RET(launch_rtran_fwd_fix(c, n[3]->e, bn->e, bn->ln, fix));
   bn->space = MLG_FFF;
   return 0;
 }
@@ -1040,44 +1046,79 @@ static int nonlin_impl(const mlg_field *b, mlg_field *rur, mlg_field *rup, mlg_f
   // path only their E is used), VEL2PLN psi's, IDEL2 chi's; W's (and chi's,
   // before IDEL2) are cleared by the first launch
   Temps T(c);
-  mlg_field *rbr = T.buffer(), *rbp = T.buffer(), *bz = T.buffer(), *psi = T.buffer(), *chi = T.buffer(), *w = T.buffer();
-  RET(T.ready());
   int rc;
   if (fused_products_supported(c)) {
     // GRAD's r d/dr b is formed in FFF; its i m b and i k b components come
-    // from b's own transform (to_pfp_b)
+    // from b's own transform.  With i k b in bn's room, the PFF fields in those
+    // of psi, chi and w first, and PROJECT's inputs in those of rbr and rbp,
+    // seven temporaries at most, as many as the routines called one by one take
+    mlg_field *rbr = T.buffer(), *rbp = T.buffer(), *psi = T.buffer(), *chi = T.buffer(), *w = T.buffer();
+    RET(T.ready());
     RET(mlg_chopset(c, 1));
     rc = launch_grad(c, b->e, b->ln, rbr->e, rbr->ln, nullptr, nullptr, nullptr, nullptr, w->ln, chi->ln);
     mlg_chopset(c, -1);
     RET(rc);
+    mlg_field *const fs7[7] = {rur, rup, uz, ror, rop, oz, rbr};
+    mlg_field *bz = bn;
+    if (bn == b) bz = T.buffer();
+    RET(T.ready());
     rbr->space = MLG_FFF;
-    mlg_field *fs7[7] = {rur, rup, uz, ror, rop, oz, rbr};
-    RET(to_pfp_b(c, fs7, b, rbp, bz, vel_fff));
+    ToPfp tp;
+    tp.n = 8;
+    tp.twice = 7;
+    for (int i = 0; i < 7; i++) {
+      if (fs7[i]->space != MLG_FFF) return 2;
+      // velocities that are kept stay where they are, in vel_fff[] afterwards
+      mlg_field *const to = vel_fff && i < 3 ? vel_fff[i] : fs7[i];
+      tp.in[i] = fs7[i]->e, tp.ln[i] = fs7[i]->ln, tp.dn[i] = 0, tp.out[i] = to->e;
+      tp.zl[tp.nzl++] = to->ln;  // the PFP fields' LN = 0
+    }
+    tp.in[7] = b->e, tp.ln[7] = b->ln, tp.dn[7] = 0, tp.out[7] = rbp->e, tp.out[8] = bz->e;
+    RET(tp.run(c, {psi, chi, w}));
+    for (int i = 0; i < 7; i++) {
+      if (vel_fff && i < 3) {
+        std::swap(vel_fff[i]->e, fs7[i]->e);
+        std::swap(vel_fff[i]->ln, fs7[i]->ln);
+        vel_fff[i]->space = MLG_FFF;
+      }
+      fs7[i]->space = MLG_PFP;
+    }
     const double2 *in[10] = {rur->e, rup->e, uz->e, ror->e, rop->e, oz->e, rbr->e, rbp->e, bz->e, nullptr};
-    double2 *out[4] = {ror->e, rop->e, oz->e, bn->e};
+    double2 *out[4] = {ror->e, rop->e, oz->e, bz->e};
     RET(launch_fused_products(c, in, out, 0.0, 0.0, 0, bn->ln));  // and N_b's LN = 0
-    bn->space = ror->space = rop->space = oz->space = MLG_PFP;
     if (!keep_velocity) {
       RET(mlg_horfft(rur, 1));
       RET(mlg_horfft(rup, 1));
       RET(mlg_horfft(uz, 1));
     }
-    {  // the z-transforms of PROJECT's inputs and of N_b (TOFF's first part) in one launch
-      mlg_field *const pf4[4] = {ror, rop, oz, bn};
-      RET(to_pff_n(c, 4, pf4));
-    }
-    // psi and chi are read by PC2VEL only: PROJECT's fix-up at infinity of
-    // psi, and IDEL2's CHOPDO and fix-up of chi, are made there, on the
-    // columns it stages
     const int nrchop0 = c->g.nrchop;
-    RET(project_impl(ror, rop, oz, psi, w, 1, 0.0, nullptr, true));
+    mlg_field *const nb = T.buffer();
+    {
+      // the z-transforms of PROJECT's inputs and of N_b (TOFF's first part) in one launch
+      Temps T2(c);
+      mlg_field *const n[4] = {rbr, rbp, T2.buffer(), nb};
+      RET(T.ready());
+      RET(T2.ready());
+      const double2 *zi[4] = {ror->e, rop->e, oz->e, bz->e};
+      double2 *zo[4];
+      for (int i = 0; i < 4; i++) zo[i] = n[i]->e, n[i]->space = MLG_PFF;
+      RET(launch_verfft_fwd_n(c, 4, zi, zo));
+      // psi and chi are read by PC2VEL only: PROJECT's fix-up at infinity of
+      // psi, and IDEL2's CHOPDO and fix-up of chi, are made there, on the
+      // columns it stages
+      RET(project_impl(n[0], n[1], n[2], psi, w, 1, 0.0, nullptr, true));
+    }
     RET(solve_op(w, chi, 0, 0.0, 0, 0.0, false));  // IDEL2
     RET(mlg_chopset(c, 3));
     rc = pc2vel_impl(psi, chi, ror, rop, oz, nrchop0);
     mlg_chopset(c, -3);
     RET(rc);
-    return mlg_toff(bn);
+    RET(launch_rtran_fwd(c, nb->e, bn->e, bn->ln));
+    bn->space = MLG_FFF;
+    return 0;
   }
+  mlg_field *rbr = T.buffer(), *rbp = T.buffer(), *bz = T.buffer(), *psi = T.buffer(), *chi = T.buffer(), *w = T.buffer();
+  RET(T.ready());
   {
     double *lz[3] = {psi->ln, chi->ln, w->ln};
     RET(launch_zero_lns(c, lz, 3));

@@ -585,6 +585,10 @@ struct Pack {
   std::vector<double2 *> e;  // the buffers
   std::vector<long> used;
   Pack(Temps &t, int cap_, int lo_ = 0) : T(t), cap(cap_), lo(lo_) { grow(lo); }
+  void give(double2 *buffer) {  // one of the caller's
+    e.push_back(buffer);
+    used.push_back(0);
+  }
   void grow(int n) {
     while ((int)e.size() < n) {
       mlg_field *f = T.buffer();

@@ -3,7 +3,8 @@ of the largest space), and the diagnostics against the oracle where their
 fields are taken to PFF a group at a time for it.
 
 The bounds are what the routines need one after the other: ENERGY two
-spectral and two PFF fields, ENEMON three, DIAGNOST seven.  The half field
+spectral and two PFF fields, ENEMON three, DIAGNOST seven, the right-hand
+sides twelve (FORCE) and seven (NONLIN).  The half field
 above a bound is for LN coefficients, tables and the allocator's granularity
 (a field is 34 MB here)."""
 import numpy as np
@@ -25,11 +26,13 @@ GRIDS = {
 }
 
 
-def grown(cfg, call, nfields):
+def grown(cfg, call, nfields, before=None):
     import torch
 
     g = H.Grid(dict(CFG1, **cfg))
     f = [g.scalar(H.FFF, np.zeros(g.shape(H.FFF), dtype=complex)) for _ in range(nfields)]
+    if before:  # its band factors; it leaves one field with the pool
+        before(f[0], f[1])
     g.synchronize()
     free = torch.cuda.mem_get_info()[0]
     call(*f)
@@ -46,6 +49,37 @@ def test_buffers_of_the_diagnostics(grid):
     assert grown(cfg, H.calc_boussi_energy, 3) <= 4.5
     assert grown(cfg, H.enemon, 2) <= 3.5
     assert grown(cfg, H.diagnost_it1, 2) <= 7.5
+
+
+@pytest.mark.parametrize("grid", list(GRIDS))
+def test_buffers_of_the_right_hand_sides(grid):
+    cfg = GRIDS[grid]
+    assert grown(cfg, H.calc_boussi_force, 6, H.idel2ln) <= 11.5
+    assert grown(cfg, H.calc_boussi_nonlin, 8, H.idel2) <= 6.5
+
+
+def test_right_hand_side_in_two_batches_and_in_place():
+    """Truncations whose PFF fields take a buffer each, so that nine jobs go
+    in two batches; results that are inputs give what separate ones do."""
+    p = Pair(dict(SMALL, nr=24, nth=8, nx=8, nrchop=18, ntchop=8, nxchop=4))
+    try:
+        st = state(p)
+        o, on = [p.o.field(O.FFF, a, ln) for a, ln in st], [p.o.field(O.FFF) for _ in range(3)]
+        p.o.call("force", *o, *on)
+        apart = None
+        for same in ({}, {2: 2}, {0: 0, 1: 1, 2: 2}, {0: 1, 1: 2, 2: 0}):  # result -> the input that it is
+            g = [p.g.scalar(O.FFF, a, ln) for a, ln in st]
+            gn = [g[same[i]] if i in same else p.g.scalar(O.FFF) for i in range(3)]
+            H.calc_boussi_force(*g, *gn)
+            got = [x.download() for x in gn]
+            if not same:
+                apart = got
+                for i in range(3):
+                    p.check(gn[i], on[i], what=f"FORCE[{i}]")
+            for x, y in zip(got, apart):
+                assert np.array_equal(x[0], y[0]) and x[1:] == y[1:], same
+    finally:
+        p.close()
 
 
 @pytest.mark.parametrize("cfg", [dict(SMALL, nr=24, nth=8, nx=8, nrchop=18, ntchop=8, nxchop=4),
