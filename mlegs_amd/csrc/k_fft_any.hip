@@ -22,8 +22,6 @@
 //   HORFFT backward  6.5 -> 0.65 ms, forward  7.4 -> 0.44 (2.1, 3.1 TB/s)
 // and at NTH = 512, NX = 384 (NR = 192): 1.84 -> 0.14, 3.13 -> 0.13, 0.76 ->
 // 0.40 and 0.73 -> 0.30 ms.
-#include <mutex>
-
 #include "fft_radix.h"
 #include "mlegs_internal.h"
 #include "xcd.h"
@@ -295,25 +293,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 }
 
 // Pencils per block (log2): as many of 1..32 as fit 80 KB of LDS (two blocks
-// per CU), `copies` buffers of the line.  Runs of 8 nodes (128 B) or more up
-// to N = 640.
+// per CU), `copies` buffers of the line; one pencil of 4096 points with a
+// second buffer takes 128 KB.  Runs of 8 nodes (128 B) or more up to N = 640.
+// (Dynamic LDS up to the device's 160 KB needs no function attribute.)
 static int any_lgp(int n, int copies) {
   int lg = 5;
   while (lg > 0 && ((size_t)n << lg) * sizeof(double2) * copies > 80 * 1024) lg--;
   return lg;
-}
-
-// dynamic LDS above the default limit, once per process
-static int any_lds_limit() {
-  static std::once_flag once;
-  static int rc = 0;
-  std::call_once(once, [] {
-    const void *fn[] = {(const void *)k_verfft_fwd_any, (const void *)k_verfft_bwd_any, (const void *)k_horfft_fwd_any,
-                        (const void *)k_horfft_bwd_any};
-    for (const void *k : fn)
-      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024) != hipSuccess) rc = MLG_E_HIP;
-  });
-  return rc;
 }
 
 int fft_any_setup(int n, FftAny *f) {
@@ -332,7 +318,7 @@ int fft_any_setup(int n, FftAny *f) {
   f->ns = ff.ns;
   f->direct = ff.direct;
   for (int i = 0; i < ff.ns; i++) f->rad[i] = ff.rad[i];
-  return any_lds_limit();
+  return 0;
 }
 
 int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd) {

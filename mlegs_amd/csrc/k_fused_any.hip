@@ -15,8 +15,6 @@
 // transforms (k_fft_any.hip): 1.39 ms against 1.94 at NTH = 204, NR = 408, NX =
 // 128.  PFP traffic (nine or ten fields in, four out) is 0.16 ms of it; the
 // rest is the stages' LDS passes and barriers at two waves a SIMD.
-#include <mutex>
-
 #include "fft_radix.h"
 #include "fused_io.h"
 #include "mlegs_internal.h"
@@ -286,25 +284,10 @@ k_fused_any(KGrid g, FusedAny f, const double *__restrict__ rsq, const double2 *
   forward(A, 3);
 }
 
-template <int R>
-static int lds_limit() {
-  const void *fn[] = {(const void *)k_fused_any<R, true>, (const void *)k_fused_any<R, false>};
-  for (const void *k : fn)
-    if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) return MLG_E_HIP;
-  return 0;
-}
-
 int fused_any_setup(int nth, FusedAny *f) {
   FusedPlan q;
   *f = FusedAny{};
   if (!fused_plan(nth, q)) return 0;
-  static std::once_flag once;
-  static int rc = 0;
-  std::call_once(once, [] {
-    for (int r : {lds_limit<2>(), lds_limit<3>(), lds_limit<4>(), lds_limit<5>(), lds_limit<6>()})
-      if (r) rc = r;
-  });
-  if (rc) return rc;
   f->n = q.n, f->R = q.R, f->D = q.D, f->nmid = q.nmid, f->P = q.P, f->T = q.T;
   // i / M = umulhi(i, ceil(2^32 / M)) exactly for i, M < 2^16; M >= 2 in every stage before the last
   auto magic = [](int m) { return (unsigned)(((1ull << 32) + m - 1) / m); };

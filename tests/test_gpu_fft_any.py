@@ -5,7 +5,7 @@ radial counts that leave part of a block's pencils empty.
 
 Tolerance: an FFT of length N rounds within a few eps log2 N of the largest
 value; the direct stage and the odd primes sum up to D terms (eps D / 2 at
-most, D <= 607 here, on values of unit size)."""
+most, D <= 4093 here, on values of unit size)."""
 import numpy as np
 import pytest
 
@@ -84,3 +84,10 @@ def test_horfft(n, full):
         assert not got[36:].any() and not got[:, n].any()
     finally:
         g.close()
+
+
+# two line buffers of 128 KB (a prime), one of 64 KB
+@pytest.mark.parametrize("n", [4093, 4096])
+def test_largest_lines(n):
+    test_verfft(n, False)
+    test_horfft(n, False)
