@@ -292,6 +292,159 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   if (inr && threadIdx.x < P) a[(size_t)g.ndimr * N] = make_double2(0.0, 0.0);
 }
 
+// -------------------------------------------------------------------------
+// Short lengths (fft_short): each thread sums one result directly from the
+// block's staged lines.  On small grids a launch is a chain of latencies, and
+// the kernels above add the look-up of their plan to it; on large ones their
+// one butterfly a thread leaves most lanes of a block idle.  us, backward and
+// forward together, against the kernels above (NR x lines):
+//                16x4         128x32       200x64       400x256
+//   VERFFT 12    5.4   10.4    8.2  12.7    8.4  12.8   11.9  19.6
+//          17    7.3   12.9   10.7  15.1   10.7  15.6   15.5  24.5
+//          20    7.9    8.8   11.5  11.1   11.3  11.2   19.2  24.6
+//          24    8.8    8.9   15.3  11.1   12.3  11.4   25.2  25.4
+//   HORFFT 12    5.7    8.9    7.9   9.8    8.8  10.1   18.9  39.3
+//          20    7.3    9.8    9.5  10.8   11.3  12.5   28.3  56.4
+//          24    8.1   10.0   10.3  10.9   12.0  13.0   37.2  60.6
+// s: [position][pencil]; w: the roots.
+constexpr int SHORT_MAX = FFT_SHORT_THETA, SHORT_P = 32;
+
+__global__ void __launch_bounds__(256) k_verfft_fwd_short(KGrid g, int N, const double2 *__restrict__ tw, TransformJobs jobs) {
+  __shared__ double2 s[SHORT_MAX * SHORT_P], w[SHORT_MAX];
+  const int p = threadIdx.x % SHORT_P, i0 = threadIdx.x / SHORT_P, rr = blockIdx.x * SHORT_P + p, mm = blockIdx.y;
+  const bool live = rr < g.nr;
+  const double2 *__restrict__ in = jobs.in[blockIdx.z] + rr + (size_t)g.ndimr * mm;
+  double2 *__restrict__ out = jobs.out[blockIdx.z] + rr + (size_t)g.ndimr * mm;
+  if ((int)threadIdx.x < N) w[threadIdx.x] = tw[threadIdx.x];
+  for (int z = i0; z < N; z += 256 / SHORT_P)
+    s[z * SHORT_P + p] = live ? in[(size_t)g.ndimr * g.ndimth * z] : make_double2(0.0, 0.0);
+  __syncthreads();
+  if (rr >= g.ndimr) return;
+  for (int kk = i0; kk < g.nxchopdim; kk += 256 / SHORT_P) {
+    const int k = kk < g.nxchop ? kk : N - (g.nxchopdim - kk);
+    double2 a = make_double2(0.0, 0.0);
+    int ph = 0;
+    for (int z = 0; z < N; z++) {
+      a = cadd(a, cmul(s[z * SHORT_P + p], w[ph]));
+      ph += k;
+      if (ph >= N) ph -= N;
+    }
+    out[(size_t)g.ndimr * g.ntchopdim * kk] = make_double2(a.x / N, a.y / N);
+  }
+}
+
+__global__ void __launch_bounds__(256) k_verfft_bwd_short(KGrid g, int N, const double2 *__restrict__ tw, TransformJobs jobs,
+                                                          const double *__restrict__ ak) {
+  __shared__ double2 s[SHORT_MAX * SHORT_P], w[SHORT_MAX];
+  const int p = threadIdx.x % SHORT_P, i0 = threadIdx.x / SHORT_P, rr = blockIdx.x * SHORT_P + p, mm = blockIdx.y;
+  const int fj = blockIdx.z, K = g.nxchopdim;
+  if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && (int)threadIdx.x < jobs.nzl) jobs.zl[threadIdx.x][0] = 0.0;
+  const bool live = rr < g.nr, dz = (jobs.dz >> fj) & 1u, dm = (jobs.dm >> fj) & 1u;
+  const double2 *__restrict__ in = jobs.in[fj] + rr + (size_t)g.ndimr * mm;
+  double2 *__restrict__ out = jobs.out[fj] + rr + (size_t)g.ndimr * mm;
+  if ((int)threadIdx.x < N) w[threadIdx.x] = tw[threadIdx.x];
+  for (int kk = i0; kk < K; kk += 256 / SHORT_P) {
+    double2 v = live ? in[(size_t)g.ndimr * g.ntchopdim * kk] : make_double2(0.0, 0.0);
+    if (dz) {
+      const double kv = ak[mm + (size_t)g.ntchopdim * kk];
+      v = make_double2(-kv * v.y, kv * v.x);
+    }
+    if (dm) {
+      const double mv = (double)(mm * g.minc);
+      v = make_double2(-mv * v.y, mv * v.x);
+    }
+    s[kk * SHORT_P + p] = v;
+  }
+  __syncthreads();
+  if (rr >= g.ndimr) return;
+  for (int z = i0; z < N; z += 256 / SHORT_P) {
+    double2 a = make_double2(0.0, 0.0);
+    int ph = 0;  // k z mod N, k = kk for kk < NXCHOP, then N - (K - kk)
+    for (int kk = 0; kk < K; kk++) {
+      if (kk == g.nxchop) ph = (N - (K - kk)) * z % N;
+      a = cadd(a, rmul<true>(s[kk * SHORT_P + p], w[ph]));
+      ph += z;
+      if (ph >= N) ph -= N;
+    }
+    out[(size_t)g.ndimr * g.ndimth * z] = a;
+  }
+}
+
+// HORFFT: the 2 N real samples of a line (slot j: 2j, 2j + 1) and its modes
+// m < NTCHOPDIM, with the roots of order 2 N, in place
+__device__ __forceinline__ void short_roots(double2 *w, int N, const double2 *__restrict__ twh) {
+  if ((int)threadIdx.x < 2 * N) {
+    const int j = threadIdx.x;
+    const double2 t = twh[j <= N ? j : j - N];
+    w[j] = j <= N ? t : make_double2(-t.x, -t.y);
+  }
+}
+__global__ void __launch_bounds__(256) k_horfft_fwd_short(KGrid g, int N, const double2 *__restrict__ twh, HorJobs jobs) {
+  __shared__ double s[2 * SHORT_MAX * SHORT_P];
+  __shared__ double2 w[2 * SHORT_MAX];
+  const int p = threadIdx.x % SHORT_P, i0 = threadIdx.x / SHORT_P, rr = blockIdx.x * SHORT_P + p;
+  const bool live = rr < g.nr;
+  double2 *a = jobs.a[blockIdx.z] + rr + (size_t)g.ndimr * g.ndimth * blockIdx.y;
+  short_roots(w, N, twh);
+  for (int j = i0; j < N; j += 256 / SHORT_P) {
+    const double2 v = live ? a[(size_t)g.ndimr * j] : make_double2(0.0, 0.0);
+    s[2 * j * SHORT_P + p] = v.x;
+    s[(2 * j + 1) * SHORT_P + p] = v.y;
+  }
+  __syncthreads();
+  if (rr >= g.ndimr) return;
+  for (int mm = i0; mm < g.ntchopdim; mm += 256 / SHORT_P) {
+    double2 x = make_double2(0.0, 0.0);
+    if (mm < g.ntchop && live) {
+      int ph = 0;
+      for (int t = 0; t < 2 * N; t++) {
+        const double v = s[t * SHORT_P + p];
+        x = make_double2(x.x + v * w[ph].x, x.y + v * w[ph].y);
+        ph += mm;
+        if (ph >= 2 * N) ph -= 2 * N;
+      }
+      const double sm = (mm == 0 ? jobs.s0 : jobs.s1) / (2 * N);
+      x = make_double2(x.x * sm, mm == 0 ? 0.0 : x.y * sm);
+    }
+    a[(size_t)g.ndimr * mm] = x;
+  }
+}
+__global__ void __launch_bounds__(256) k_horfft_bwd_short(KGrid g, int N, const double2 *__restrict__ twh, HorJobs jobs) {
+  __shared__ double2 s[SHORT_MAX * SHORT_P], w[2 * SHORT_MAX];
+  const int p = threadIdx.x % SHORT_P, i0 = threadIdx.x / SHORT_P, rr = blockIdx.x * SHORT_P + p, M = g.ntchopdim;
+  const bool live = rr < g.nr;
+  double2 *a = jobs.a[blockIdx.z] + rr + (size_t)g.ndimr * g.ndimth * blockIdx.y;
+  const double wr = jobs.wr && live ? jobs.wr[rr < g.nr - 1 - rr ? rr : g.nr - 1 - rr] : 1.0;
+  short_roots(w, N, twh);
+  for (int mm = i0; mm < M; mm += 256 / SHORT_P) {
+    double2 v = make_double2(0.0, 0.0);
+    if (live && mm < g.ntchop) {
+      const double sm = (mm == 0 ? jobs.s0 : 2.0 * jobs.s1) * wr;  // m >= 1 twice, as m and -m
+      v = a[(size_t)g.ndimr * mm];
+      v = make_double2(v.x * sm, mm == 0 ? 0.0 : v.y * sm);
+    }
+    s[mm * SHORT_P + p] = v;
+  }
+  __syncthreads();
+  if (rr >= g.ndimr) return;
+  for (int j = i0; j <= N; j += 256 / SHORT_P) {
+    double2 x = make_double2(0.0, 0.0);
+    if (j < N) {
+      int pe = 0, po = 0;  // m 2j and m (2j + 1) mod 2 N
+      for (int mm = 0; mm < M; mm++) {
+        const double2 c = s[mm * SHORT_P + p];
+        x.x += c.x * w[pe].x + c.y * w[pe].y;
+        x.y += c.x * w[po].x + c.y * w[po].y;
+        pe += 2 * j;
+        if (pe >= 2 * N) pe -= 2 * N;
+        po += 2 * j + 1;
+        if (po >= 2 * N) po -= 2 * N;
+      }
+    }
+    a[(size_t)g.ndimr * j] = x;
+  }
+}
+
 // Pencils per block (log2): as many of 1..32 as fit 80 KB of LDS (two blocks
 // per CU), `copies` buffers of the line; one pencil of 4096 points with a
 // second buffer takes 128 KB.  Runs of 8 nodes (128 B) or more up to N = 640.
@@ -302,9 +455,11 @@ static int any_lgp(int n, int copies) {
   return lg;
 }
 
-int fft_any_setup(int n, FftAny *f) {
+int fft_any_setup(int n, bool theta, FftAny *f) {
   FftFactors ff;
   *f = FftAny{};
+  f->n = n;
+  if (fft_short(n, theta)) return 0;
   if (!fft_factor(n, ff)) return MLG_E_ARG;
   std::vector<int> freq, pos;
   fft_order(ff, freq, pos);
@@ -314,7 +469,6 @@ int fft_any_setup(int n, FftAny *f) {
   f->freq = d;
   f->pos = d + (freq.size() - pos.size());
   MLG_CHECK_HIP(hipMemcpy(d, freq.data(), sizeof(int) * freq.size(), hipMemcpyHostToDevice));
-  f->n = n;
   f->ns = ff.ns;
   f->direct = ff.direct;
   for (int i = 0; i < ff.ns; i++) f->rad[i] = ff.rad[i];
@@ -324,10 +478,17 @@ int fft_any_setup(int n, FftAny *f) {
 int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd) {
   KGrid g = kgrid(c);
   const FftAny &f = c->fz;
+  KScope ks(c, fwd ? K_VERFFT_FWD : K_VERFFT_BWD, n * 16.0 * g.nr * g.ntchopdim * (double)(g.nx + g.nxchopdim));
+  if (fft_short(f.n, false)) {
+    const dim3 grid((g.ndimr + SHORT_P - 1) / SHORT_P, g.ntchopdim, n);
+    if (fwd) hipLaunchKernelGGL(k_verfft_fwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_z, jobs);
+    else hipLaunchKernelGGL(k_verfft_bwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_z, jobs, c->d.ak);
+    MLG_CHECK_HIP(hipGetLastError());
+    return 0;
+  }
   const int lg = any_lgp(f.n, 1), P = 1 << lg;
   const dim3 grid(xcd_grid((g.ndimr + P - 1) / P * g.ntchopdim * n));
   const size_t lds = sizeof(double2) * ((size_t)f.n << lg);
-  KScope ks(c, fwd ? K_VERFFT_FWD : K_VERFFT_BWD, n * 16.0 * g.nr * g.ntchopdim * (double)(g.nx + g.nxchopdim));
   if (fwd)
     hipLaunchKernelGGL(k_verfft_fwd_any, grid, dim3(256), lds, c->stream, g, f, lg, c->d.tw_z, jobs, n);
   else
@@ -339,6 +500,13 @@ int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd) {
 int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd) {
   KGrid g = kgrid(c);
   const FftAny &f = c->ft;
+  if (fft_short(f.n, true)) {
+    const dim3 grid((g.ndimr + SHORT_P - 1) / SHORT_P, g.ndimx, jobs.n);
+    if (fwd) hipLaunchKernelGGL(k_horfft_fwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_h, jobs);
+    else hipLaunchKernelGGL(k_horfft_bwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_h, jobs);
+    MLG_CHECK_HIP(hipGetLastError());
+    return 0;
+  }
   const int copies = fwd && f.direct ? 2 : 1;
   const int lg = any_lgp(f.n, copies), P = 1 << lg;
   const dim3 grid(xcd_grid((g.ndimr + P - 1) / P * g.ndimx * jobs.n));

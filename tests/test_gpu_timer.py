@@ -15,7 +15,7 @@ def grid(**k):
 
 
 # the four-step kernels, the theta lines, the short, mixed-radix and direct lengths
-@pytest.mark.parametrize("n", [8, 64, 512, 12, 24, 46, 1024])
+@pytest.mark.parametrize("n", [8, 64, 512, 12, 30, 46, 1024])
 def test_one_record_per_transform(n):
     g = grid(nth=n)
     f = g.scalar(H.PPP, np.ones(g.shape(H.PPP), dtype=complex))
