@@ -247,8 +247,8 @@ extern "C" int mlg_init(const mlg_params *p, mlg_ctx **out) {
     for (int j = 0; j <= G.nth; j++) v[j] = make_double2(re[j], im[j]);
     RET(upload(&d.tw_h, v));
   }
-  if (!fft4_length(G.nx)) RET(fft_any_setup(G.nx, false, &c->fz));
-  if (!fft4_length(G.nth)) RET(fft_any_setup(G.nth, true, &c->ft));
+  if (!fft4_length(G.nx)) RET(fft_any_setup(G.nx, &c->fz));
+  if (!fft4_length(G.nth)) RET(fft_any_setup(G.nth, &c->ft));
   if (!fused_line_length(G.nth)) RET(fused_any_setup(G.nth, &c->fp));
   if (!G.hv_r.empty()) {
     std::vector<double> hv;

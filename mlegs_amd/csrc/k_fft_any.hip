@@ -16,7 +16,7 @@
 // times.  A prime factor above 19 is summed directly in the last stage.
 //
 // Direct O(N^2) sums, and radix-2 stages in LDS for powers of two above 256,
-// took these lengths before.  Per field at NTH = 204, NX = 608 (NR = 408, 136
+// took these lengths before (up to 24 points direct sums still do).  Per field at NTH = 204, NX = 608 (NR = 408, 136
 // modes, 607 wavenumbers; 1.09 GB a z-transform, 1.36 GB a theta transform):
 //   VERFFT backward 11.0 -> 0.36 ms, forward 13.5 -> 0.37 (3.0 TB/s)
 //   HORFFT backward  6.5 -> 0.65 ms, forward  7.4 -> 0.44 (2.1, 3.1 TB/s)
@@ -293,21 +293,30 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 }
 
 // -------------------------------------------------------------------------
-// Short lengths (fft_short): each thread sums one result directly from the
-// block's staged lines.  On small grids a launch is a chain of latencies, and
-// the kernels above add the look-up of their plan to it; on large ones their
-// one butterfly a thread leaves most lanes of a block idle.  us, backward and
-// forward together, against the kernels above (NR x lines):
+// Short lengths (fft_short, N <= 24): each thread sums one result directly from
+// the block's staged lines, terms paired by symmetry.  On small grids a launch
+// is a chain of latencies, and the kernels above add the look-up of their plan
+// to it; on large ones their one butterfly a thread leaves most lanes of a
+// block idle.  us, backward and forward together, against the kernels above
+// (NR x lines); the line is where the sums' work has eaten the difference:
 //                16x4         128x32       200x64       400x256
-//   VERFFT 12    5.4   10.4    8.2  12.7    8.4  12.8   11.9  19.6
-//          17    7.3   12.9   10.7  15.1   10.7  15.6   15.5  24.5
-//          20    7.9    8.8   11.5  11.1   11.3  11.2   19.2  24.6
-//          24    8.8    8.9   15.3  11.1   12.3  11.4   25.2  25.4
-//   HORFFT 12    5.7    8.9    7.9   9.8    8.8  10.1   18.9  39.3
-//          20    7.3    9.8    9.5  10.8   11.3  12.5   28.3  56.4
-//          24    8.1   10.0   10.3  10.9   12.0  13.0   37.2  60.6
+//   VERFFT 12    4.9   10.1    7.5  12.8    7.7  13.0   10.3  19.8
+//          20    6.3    8.8    9.5  11.3    9.6  11.3   15.0  24.5
+//          24    6.9    9.0   11.4  11.4   10.5  11.6   17.5  25.9
+//   HORFFT 12    5.9    8.9    7.4  10.3    8.2  10.5   17.4  39.3
+//          20    7.2   10.0    9.0  11.0   10.2  12.7   26.4  56.1
+//          24    7.4   10.1    9.1  11.2   11.1  13.0   33.1  60.1
 // s: [position][pencil]; w: the roots.
-constexpr int SHORT_MAX = FFT_SHORT_THETA, SHORT_P = 32;
+constexpr int SHORT_MAX = FFT_SHORT, SHORT_P = 32;
+
+// Terms j and N - j of a sum, u w^j + v w^-j: A + i B gathers (u + v) Re w^j and
+// (u - v) Im w^j, half the products and the smaller rounding
+__device__ __forceinline__ void short_pair(double2 u, double2 v, double2 t, double2 &A, double2 &B) {
+  A.x += (u.x + v.x) * t.x;
+  A.y += (u.y + v.y) * t.x;
+  B.x += (u.x - v.x) * t.y;
+  B.y += (u.y - v.y) * t.y;
+}
 
 __global__ void __launch_bounds__(256) k_verfft_fwd_short(KGrid g, int N, const double2 *__restrict__ tw, TransformJobs jobs) {
   __shared__ double2 s[SHORT_MAX * SHORT_P], w[SHORT_MAX];
@@ -322,14 +331,19 @@ __global__ void __launch_bounds__(256) k_verfft_fwd_short(KGrid g, int N, const 
   if (rr >= g.ndimr) return;
   for (int kk = i0; kk < g.nxchopdim; kk += 256 / SHORT_P) {
     const int k = kk < g.nxchop ? kk : N - (g.nxchopdim - kk);
-    double2 a = make_double2(0.0, 0.0);
+    double2 A = s[p], B = make_double2(0.0, 0.0);
     int ph = 0;
-    for (int z = 0; z < N; z++) {
-      a = cadd(a, cmul(s[z * SHORT_P + p], w[ph]));
+    for (int z = 1; 2 * z < N; z++) {
+      const double2 u = s[z * SHORT_P + p], v = s[(N - z) * SHORT_P + p];
       ph += k;
       if (ph >= N) ph -= N;
+      short_pair(u, v, w[ph], A, B);
     }
-    out[(size_t)g.ndimr * g.ntchopdim * kk] = make_double2(a.x / N, a.y / N);
+    if (N % 2 == 0) {
+      const double2 u = s[N / 2 * SHORT_P + p];
+      A = k % 2 ? csub(A, u) : cadd(A, u);
+    }
+    out[(size_t)g.ndimr * g.ntchopdim * kk] = make_double2((A.x - B.y) / N, (A.y + B.x) / N);
   }
 }
 
@@ -358,15 +372,14 @@ __global__ void __launch_bounds__(256) k_verfft_bwd_short(KGrid g, int N, const 
   __syncthreads();
   if (rr >= g.ndimr) return;
   for (int z = i0; z < N; z += 256 / SHORT_P) {
-    double2 a = make_double2(0.0, 0.0);
-    int ph = 0;  // k z mod N, k = kk for kk < NXCHOP, then N - (K - kk)
-    for (int kk = 0; kk < K; kk++) {
-      if (kk == g.nxchop) ph = (N - (K - kk)) * z % N;
-      a = cadd(a, rmul<true>(s[kk * SHORT_P + p], w[ph]));
+    double2 A = s[p], B = make_double2(0.0, 0.0);
+    int ph = 0;
+    for (int k = 1; k < g.nxchop; k++) {  // k and -k
       ph += z;
       if (ph >= N) ph -= N;
+      short_pair(s[k * SHORT_P + p], s[(K - k) * SHORT_P + p], w[ph], A, B);
     }
-    out[(size_t)g.ndimr * g.ndimth * z] = a;
+    out[(size_t)g.ndimr * g.ndimth * z] = make_double2(A.x + B.y, A.y - B.x);
   }
 }
 
@@ -396,12 +409,22 @@ __global__ void __launch_bounds__(256) k_horfft_fwd_short(KGrid g, int N, const 
   for (int mm = i0; mm < g.ntchopdim; mm += 256 / SHORT_P) {
     double2 x = make_double2(0.0, 0.0);
     if (mm < g.ntchop && live) {
+      // samples t, 2 N - t, N - t and N + t together
+      const double sg = mm % 2 ? -1.0 : 1.0;
+      auto S = [&](int t) { return s[t * SHORT_P + p]; };
+      x.x = S(0) + sg * S(N);
       int ph = 0;
-      for (int t = 0; t < 2 * N; t++) {
-        const double v = s[t * SHORT_P + p];
-        x = make_double2(x.x + v * w[ph].x, x.y + v * w[ph].y);
+      for (int t = 1; 2 * t < N; t++) {
         ph += mm;
         if (ph >= 2 * N) ph -= 2 * N;
+        const double a = S(t), b = S(2 * N - t), c = S(N - t), d = S(N + t);
+        x = make_double2(x.x + ((a + b) + sg * (c + d)) * w[ph].x, x.y + ((a - b) - sg * (c - d)) * w[ph].y);
+      }
+      if (N % 2 == 0) {
+        const double a = S(N / 2), b = S(N + N / 2);
+        ph += mm;
+        if (ph >= 2 * N) ph -= 2 * N;
+        x = make_double2(x.x + (a + b) * w[ph].x, x.y + (a - b) * w[ph].y);
       }
       const double sm = (mm == 0 ? jobs.s0 : jobs.s1) / (2 * N);
       x = make_double2(x.x * sm, mm == 0 ? 0.0 : x.y * sm);
@@ -455,11 +478,11 @@ static int any_lgp(int n, int copies) {
   return lg;
 }
 
-int fft_any_setup(int n, bool theta, FftAny *f) {
+int fft_any_setup(int n, FftAny *f) {
   FftFactors ff;
   *f = FftAny{};
   f->n = n;
-  if (fft_short(n, theta)) return 0;
+  if (fft_short(n)) return 0;
   if (!fft_factor(n, ff)) return MLG_E_ARG;
   std::vector<int> freq, pos;
   fft_order(ff, freq, pos);
@@ -479,7 +502,7 @@ int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd) {
   KGrid g = kgrid(c);
   const FftAny &f = c->fz;
   KScope ks(c, fwd ? K_VERFFT_FWD : K_VERFFT_BWD, n * 16.0 * g.nr * g.ntchopdim * (double)(g.nx + g.nxchopdim));
-  if (fft_short(f.n, false)) {
+  if (fft_short(f.n)) {
     const dim3 grid((g.ndimr + SHORT_P - 1) / SHORT_P, g.ntchopdim, n);
     if (fwd) hipLaunchKernelGGL(k_verfft_fwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_z, jobs);
     else hipLaunchKernelGGL(k_verfft_bwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_z, jobs, c->d.ak);
@@ -500,7 +523,7 @@ int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd) {
 int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd) {
   KGrid g = kgrid(c);
   const FftAny &f = c->ft;
-  if (fft_short(f.n, true)) {
+  if (fft_short(f.n)) {
     const dim3 grid((g.ndimr + SHORT_P - 1) / SHORT_P, g.ndimx, jobs.n);
     if (fwd) hipLaunchKernelGGL(k_horfft_fwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_h, jobs);
     else hipLaunchKernelGGL(k_horfft_bwd_short, grid, dim3(256), 0, c->stream, g, f.n, c->d.tw_h, jobs);

@@ -323,9 +323,9 @@ int launch_horfft_bwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double 
 // lengths of the four-step register kernels
 static inline bool fft4_length(int n) { return n >= 2 && n <= 256 && (n & (n - 1)) == 0; }
 // lengths, not powers of two, that are summed directly (k_fft_any.hip has both sides' times)
-constexpr int FFT_SHORT_Z = 20, FFT_SHORT_THETA = 24;
-static inline bool fft_short(int n, bool theta) { return n <= (theta ? FFT_SHORT_THETA : FFT_SHORT_Z); }
-int fft_any_setup(int n, bool theta, FftAny *f);  // allocates f's device tables
+constexpr int FFT_SHORT = 24;
+static inline bool fft_short(int n) { return n <= FFT_SHORT; }
+int fft_any_setup(int n, FftAny *f);  // allocates f's device tables
 int launch_verfft_any(mlg_ctx *c, int n, const TransformJobs &jobs, bool fwd);
 int launch_horfft_any(mlg_ctx *c, const HorJobs &jobs, bool fwd);  // inside the caller's KScope
 // NTH = 16, 32, .. 512 without scale factors, on the lines of the fused products (k_fused.hip); inside the caller's KScope
