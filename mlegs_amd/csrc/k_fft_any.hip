@@ -119,13 +119,7 @@ __device__ __forceinline__ void fft_any(const FftAny &f, const double2 *__restri
   auto out = [&](int pos, int b, int k, double2 v) { st(pos, f.freq[b] + outstep * k, v); };
   int L = n, q = 0;
   if (!STAGED) {
-    if (last == 0 && !f.direct) {
-#define C_ONE(R_) stage<R_, INV>(n, n, i0, istep, tw, ld, out)
-      FFT_ANY_RADIX(f.rad[0], C_ONE)
-#undef C_ONE
-      return;
-    }
-    if (last == 0) {  // direct only: stage the line as it lies
+    if (last == 0) {  // direct only (lengths of one butterfly are summed, fft_short): stage the line as it lies
       for (int i = i0; i < n; i += istep) s[(i << lgp) + p] = ld(i);
     } else {
 #define C_FIRST(R_) stage<R_, INV>(n, n, i0, istep, tw, ld, lds_st)
