@@ -1316,8 +1316,8 @@ static int richardson(mlg_field *y, const mlg_field *x1, bool ln) {
 // IHELM of n independent fields, A_i = IHELM(B_i, ALP_i), with one band-solve
 // launch for all of them (each field as solve_op does it for op 2).
 // bil: the right-hand sides b are row-interleaved (launch_visc2_rhs_il);
-// chop false: the rows past the truncation of a are zero already
-static int ihelm_n(int n, mlg_field *const *b, mlg_field *const *a, const double *alp, int bil = 0, bool chop = true) {
+// ab2: they formed the AB2 step, and the rows of a past the truncation are zero already
+static int ihelm_n(int n, mlg_field *const *b, mlg_field *const *a, const double *alp, int bil = 0, bool ab2 = false) {
   mlg_ctx *c = b[0]->ctx;
   const double2 *be[3];
   double2 *ae[3];
@@ -1338,8 +1338,8 @@ static int ihelm_n(int n, mlg_field *const *b, mlg_field *const *a, const double
   RET(T.ready());
   double2 *te[3] = {nullptr, nullptr, nullptr};
   for (int i = 0; i < n; i++) te[i] = tf[i]->e;
-  RET(launch_band_solve_n(c, 2, n, be, ae, aln, bln, alp, 0, 0.0, te, bil));
-  return chop ? launch_chopdo_fff_n(c, n, ae, false) : 0;
+  RET(launch_band_solve_n(c, 2, n, be, ae, aln, bln, alp, 0, 0.0, te, bil, ab2));
+  return ab2 ? 0 : launch_chopdo_fff_n(c, n, ae, false);
 }
 
 // VISC1 (mod_march.f90:1529-1576): backward Euler diffusion; the right-hand
@@ -1404,10 +1404,11 @@ static int visc_cn(mlg_ctx *c, mlg_field *const *f, const mlg_field *const *fa, 
   }
   jobs.dt = c->g.p.dt;
   // WK row-interleaved for the one-thread-per-system solve, in columns for the partitioned one
-  const int il = band_lanes(kgrid(c)) == 0;
+  const bool ab2 = x != nullptr;
+  const int il = band_lanes(kgrid(c), ab2) == 0;
   RET(launch_visc2_rhs_il(c, n, jobs, il));
   mlg_field *out[3] = {f[0], f[1], f[2]};
-  return ihelm_n(n, wk, out, alp, il, x == nullptr);  // with x the outputs are chopped with the right-hand sides
+  return ihelm_n(n, wk, out, alp, il, ab2);  // with x the outputs are chopped with the right-hand sides
 }
 static int visc_cn(mlg_ctx *c, mlg_field *psi, mlg_field *chi, mlg_field *b, const mlg_field *psio, const mlg_field *chio,
                    const mlg_field *bo) {
@@ -1496,7 +1497,7 @@ static int step_ab_cn(mlg_solver *s, mlg_field *psi, mlg_field *chi, mlg_field *
   mlg_field *y[3] = {psi, chi, b}, *h[3] = {s->n_psi, s->n_chi, s->n_b}, *x[3] = {psin, chin, bn};
   bool fff = true;
   for (int i = 0; i < 3; i++) fff = fff && y[i]->space == MLG_FFF && x[i]->space == MLG_FFF;
-  if (fff && c->g.p.visc_sw == 1 && c->g.p.kappa != 0.0 && band_lanes(kgrid(c)) != 0) {
+  if (fff && c->g.p.visc_sw == 1 && c->g.p.kappa != 0.0 && band_lanes(kgrid(c), true) != 0) {
     // the AB2 step, the history copies and VISC2's right-hand sides of the
     // three fields in one launch (right-hand sides in columns)
     RET(visc_cn(c, y, y, y, x, h));

@@ -1786,17 +1786,7 @@ __device__ void apply_penta_part(const KGrid &g, int op, int has_ln, const BandJ
   const int nlast = max(nd - 1, 0);
   // right-hand sides into LDS: system jp's row n at slot (jp P + n / LS), row n % LS
   const size_t fstride = (size_t)64 * SLOT;
-  if (jobs.bil) {
-    // row n of system s at b[n nsys + s]: lanes over W consecutive systems
-    int m2, k2;
-    const int jp = lane % W;
-    const int ndp = penta_rows(g, op, sys0 + jp, m2, k2);
-    for (int n = lane / W; n < ndp; n += P) {
-      const int sl = (jp * P + n / LS) * SLOT + n % LS;
-#pragma unroll
-      for (int jj = 0; jj < NJ; jj++) lds[jj * fstride + sl] = jobs.j[jobs.gjob[grp][jj]].b[(size_t)n * nsys + sys0 + jp];
-    }
-  } else if (P < 16) {
+  if (P < 16) {
     part_rows_each(g, op, sys0, P, [&](int sl, size_t i) {
 #pragma unroll
       for (int jj = 0; jj < NJ; jj++) lds[jj * fstride + sl] = jobs.j[jobs.gjob[grp][jj]].b[i];
@@ -1967,9 +1957,9 @@ __global__ void __launch_bounds__(64) k_band_apply(KGrid g, const double *bxm, i
 // IHELM's.
 __device__ void apply_m0_part(const KGrid &g, const double *bxm, int op, double alp, int has_ln, double lnval,
                               const double2 *b, double2 *a, double *ln_a, const double *ln_b, const double *__restrict__ F,
-                              int k, double2 *lds, int bil) {
+                              int k, double2 *lds) {
   if (solve_kind(op, 0, k) == 1) {
-    apply_m0(g, bxm, op, alp, has_ln, lnval, b, a, ln_a, ln_b, F, k, reinterpret_cast<double *>(lds), bil);
+    apply_m0(g, bxm, op, alp, has_ln, lnval, b, a, ln_a, ln_b, F, k, reinterpret_cast<double *>(lds), 0);
     return;
   }
   constexpr int LS = PART_LS, SLOT = PART_LS + 1;
@@ -1983,13 +1973,12 @@ __device__ void apply_m0_part(const KGrid &g, const double *bxm, int op, double 
   if (nn < 1 || g.ntchop < 1 || kind == 0) return;  // the whole block
   const int kabs = k < g.nxchop ? k : g.nxchopdim - k;
   const long cls = (long)g.ntchopdim * kabs;
-  const size_t bstride = bil ? (size_t)g.ntchopdim * g.nxchopdim : 1;
-  const double2 *xb = bil ? b + (size_t)g.ntchopdim * k : b + (size_t)g.nrchopdim * ((size_t)g.ntchopdim * k);
+  const double2 *xb = b + (size_t)g.nrchopdim * ((size_t)g.ntchopdim * k);
   double2 *xg = a + (size_t)g.nrchopdim * ((size_t)g.ntchopdim * k);
   auto slot = [&](int n) { return (n / LS) * SLOT + n % LS; };
   const double lnA = k == 0 ? -ln_b[0] / alp : 0.0;
   for (int n = lane; n < nn; n += 64) {
-    double2 v = xb[n * bstride];
+    double2 v = xb[n];
     if (k == 0) {
       if (n == 0) v.x = v.x - lnA * (4.0 / 3 / g.ell2) / g.norm0;
       if (n == 1) v.x = v.x - lnA * (-2 / g.norm1 / g.ell2);
@@ -2045,7 +2034,7 @@ __global__ void __launch_bounds__(64, 3) k_band_apply_part(KGrid g, const double
   if ((int)blockIdx.x < nm0 * jobs.n) {
     const BandJob &J = jobs.j[blockIdx.x / nm0];
     apply_m0_part(g, bxm, op, J.alp, has_ln, lnval, J.b, J.a, J.ln_a, J.ln_b, J.F, blockIdx.x % nm0,
-                  reinterpret_cast<double2 *>(m0s), jobs.bil);
+                  reinterpret_cast<double2 *>(m0s));
     return;
   }
   // the penta-diagonal blocks from the next multiple of 8 on, XCD-aware: the
@@ -2064,13 +2053,15 @@ __global__ void __launch_bounds__(64, 3) k_band_apply_part(KGrid g, const double
 
 // Lanes per penta-diagonal system of the partitioned solve: the smallest
 // power of two, at least 2, whose segments of PART_LS rows cover NRCHOP.
-// 0: one thread per system (NRCHOP above 64 PART_LS); that path is
-// LUBKSBB's arithmetic, bitwise.  A solve (mean of IDEL2LN's and the three
-// fields' IHELM) takes 15.3 us on 8 lanes at NRCHOP 48 against 25.9 on one
-// thread per system; at 22 it takes 14.5 against 12.5, but its right-hand
-// sides in columns form the AB2 step on the way, two launches less.
-int band_lanes(const KGrid &g) {
-  if (g.nrchop > 64 * PART_LS) return 0;
+// 0: one thread per system (NRCHOP above 64 PART_LS, or below 20); that path
+// is LUBKSBB's arithmetic, bitwise.  Short systems: IDEL2LN takes 9.3 us on one
+// thread per system against 13.0 at NRCHOP 14, 12.4 against 13.4 at 22 and
+// 16.2 against 13.6 at 36 (16x16), 10.8 against 13.2, 13.5 against 13.4 and
+// 17.4 against 15.6 at 128x128; IHELM 10.2 against 12.3 at 14 and 14.0 against
+// 12.6 at 22.  ab2: right-hand sides in columns that form the AB2 step on the
+// way, which saves two launches, take the lanes at any length.
+int band_lanes(const KGrid &g, bool ab2) {
+  if (g.nrchop > 64 * PART_LS || (g.nrchop < 20 && !ab2)) return 0;
   int p = 2;
   while (p * PART_LS < g.nrchop) p *= 2;
   return p;
@@ -2117,7 +2108,8 @@ static double *factor_set(mlg_ctx *c, int op, double alp, const double *const *k
 }
 
 int launch_band_solve_n(mlg_ctx *c, int op, int n, const double2 *const *b, double2 *const *a, double *const *ln_a,
-                        const double *const *ln_b, const double *alp, int has_ln, double ln, double2 *const *t, int bil) {
+                        const double *const *ln_b, const double *alp, int has_ln, double ln, double2 *const *t, int bil,
+                        bool ab2) {
   if (n < 1 || n > MAX_BAND_JOBS) return MLG_E_ARG;
   KGrid g = kgrid(c);
   long nsys = (long)g.ntchopdim * g.nxchopdim;
@@ -2141,7 +2133,8 @@ int launch_band_solve_n(mlg_ctx *c, int op, int n, const double2 *const *b, doub
     jobs.gjob[gi][jobs.gcount[gi]++] = i;
   }
   KScope ks(c, K_BAND_SOLVE, n * 2.0 * 16.0 * fff_count(g));  // the coefficients read and written once
-  const int lanes = band_lanes(g);
+  const int lanes = band_lanes(g, ab2);
+  if (lanes && bil) return MLG_E_ARG;  // the lanes read columns
   const int nm0 = (op != 1) ? g.nxchopdim : 0;
   size_t lds = nm0 ? m0_lds_bytes(g) : 0;
   if (lanes) {
@@ -2487,7 +2480,7 @@ int launch_band_solve_t_n(mlg_ctx *c, int op, int n, const BandTJob *in) {
   }
   const long nsys = (long)g.ntchopdim * g.nxchopdim;
   KScope ks(c, K_BAND_SOLVE, n * 2.0 * 16.0 * fff_count(g));
-  const int lanes = band_lanes(g);
+  const int lanes = band_lanes(g, false);
   if (lanes) {
     const int nm0 = op == 2 ? g.nxchopdim : 0;
     const long npart = (nsys + 64 / lanes - 1) / (64 / lanes);

@@ -407,7 +407,7 @@ struct Visc2Jobs {
 int launch_visc2_rhs_il(mlg_ctx *c, int n, const Visc2Jobs &jobs, int il);
 // lanes per penta-diagonal system of the band substitution (0: one thread
 // per system, which reads row-interleaved right-hand sides coalesced)
-int band_lanes(const KGrid &g);
+int band_lanes(const KGrid &g, bool ab2);  // ab2: right-hand sides that form the AB2 step
 int launch_set_ln(mlg_ctx *c, double *dst, const double *src, double scale, double add);
 int launch_zero_lns(mlg_ctx *c, double *const *ptrs, int n);  // LN = 0 for n fields, one launch per 32
 int launch_delsqh(mlg_ctx *c, const double2 *a, const double *ln_a, double2 *b, double *ln_b);
@@ -462,7 +462,7 @@ int launch_band_solve(mlg_ctx *c, int op, const double2 *b, double2 *a, double *
 // written by launch_visc2_rhs_il
 int launch_band_solve_n(mlg_ctx *c, int op, int n, const double2 *const *b, double2 *const *a, double *const *ln_a,
                         const double *const *ln_b, const double *alp, int has_ln, double ln, double2 *const *t,
-                        int bil = 0);
+                        int bil = 0, bool ab2 = false);
 // Adjoint of n (<= 3) op 1 (IDEL2LN) or op 2 (IHELM) solves in one launch:
 // job i reads the solution's adjoint from in (FFF, chopped on the way in)
 // and writes the right-hand side's adjoint to out (may equal in; CHOPDO
