@@ -386,19 +386,15 @@ int launch_verfft_bwd(mlg_ctx *c, const double2 *in, double2 *out) { return laun
 // 384x128x128, 55 -> 16 at 384x32x256, 8.1 -> 6.3 at 128x64x64.  Forward,
 // their reads are runs of 32 bytes, which costs fields that exceed the caches
 // (174 us against 156 at 384x256x256, 44 against 40 at 384x128x128, 102 MB)
-// what it gains smaller ones (28 -> 20 at 200x256x64, 53 MB; 27 -> 15 at
-// NTH = 32, where the runs are longer); NTH = 512 has no other kernel of that
-// kind and the mixed-radix one takes as long (106 us at 192x512x128) or
-// longer (12.8 against 7.8 at 64x512x16).  Forward at NTH = 16 keeps its
-// rounding: the lines' error is the smaller one (1.39e-16 rms against 1.48e-16)
-// and their time too (7.9 us against 19.7 at 384x16x256), but the check of
-// PROJECT's transpose at 32x16x16 compares sums that cancel by six digits, and
-// which of two such roundings meets its bar is chance.
+// what it gains smaller ones (28 -> 20 at 200x256x64, 53 MB); at NTH = 16 and
+// 32 the runs are longer (19.7 -> 7.9 us at 384x16x256, 27 -> 15 at NTH = 32);
+// NTH = 512 has no other kernel of that kind and the mixed-radix one takes as
+// long (106 us at 192x512x128) or longer (12.8 against 7.8 at 64x512x16).
 static bool horfft_on_lines(const KGrid &g, const HorJobs &j, bool fwd) {
   const int n = g.nth;
   if (n < 16 || n > 512 || (n & (n - 1)) || j.s0 != 1.0 || j.s1 != 1.0 || j.wr) return false;
   const double bytes = 16.0 * g.ndimr * g.ndimth * (double)g.ndimx * j.n;
-  return !fwd || n == 32 || n == 512 || (n > 16 && bytes <= 64e6);
+  return !fwd || n <= 32 || n == 512 || bytes <= 64e6;
 }
 int launch_horfft_fwd_n(mlg_ctx *c, int n, double2 *const *a, double s0, double s1) {
   if (n < 1 || n > MAX_HOR_JOBS) return MLG_E_ARG;
