@@ -14,8 +14,8 @@
 //     fields of a line in one wave (k_fused_products_256, k_fused_products_reg)
 //     or one wave a field (k_fused_products_wide); launch_line has the rule
 //   every other length: k_fused_any.hip
-// Every value goes through the operations of the separate HORFFT and
-// product kernels, in the same order.
+// The products are the separate kernels' operations, in the same order; the
+// transforms may factor their length in another way than the separate HORFFT.
 #include "fused_io.h"
 #include "mlegs_internal.h"
 #include "xcd.h"
@@ -1185,7 +1185,7 @@ struct Line512 {
 // lines), NTH = 32 (Line32: 4 lanes, 64 lines) or NTH = 16 (Line16: 2 lanes,
 // 128 lines); a block takes adjacent
 // radial nodes of one z plane.
-template <class L, bool LINEAR>
+template <class L, bool LINEAR, bool FULL = false>
 __global__ void __launch_bounds__(L::THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw, const double2 *twh, FusedIO io,
                      double two_omega, double n2) {
@@ -1221,25 +1221,25 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
   const double r2 = live ? rsq[rr] : 1.0;
 
   double2 A[8], B[8], C[8], U[8], V[8], T[8];
-  L::template inverse<false>(x, g, in(0), lo, live, A);  // rur
-  L::template inverse<false>(x, g, in(1), lo, live, B);  // rup
-  L::template inverse<false>(x, g, in(2), lo, live, C);  // uz
+  L::template inverse<FULL>(x, g, in(0), lo, live, A);  // rur
+  L::template inverse<FULL>(x, g, in(1), lo, live, B);  // rup
+  L::template inverse<FULL>(x, g, in(2), lo, live, C);  // uz
   // oz: U = rup oz, V = rur oz
-  L::template inverse<false>(x, g, in(5), lo, live, T);
+  L::template inverse<FULL>(x, g, in(5), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     U[i] = make_double2(B[i].x * T[i].x, B[i].y * T[i].y);
     V[i] = make_double2(A[i].x * T[i].x, A[i].y * T[i].y);
   }
   // ror: Y = uz ror - rur oz (to LDS); V = rup ror
-  L::template inverse<false>(x, g, in(3), lo, live, T);
+  L::template inverse<FULL>(x, g, in(3), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     ys[LANES * i] = make_double2(C[i].x * T[i].x - V[i].x, C[i].y * T[i].y - V[i].y);
     V[i] = make_double2(B[i].x * T[i].x, B[i].y * T[i].y);
   }
   // rop: X = rup oz - uz rop in U; Z = (rur rop - rup ror) / r^2 in V
-  L::template inverse<false>(x, g, in(4), lo, live, T);
+  L::template inverse<FULL>(x, g, in(4), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     U[i] = make_double2(U[i].x - C[i].x * T[i].x, U[i].y - C[i].y * T[i].y);
@@ -1250,29 +1250,29 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
 #pragma unroll
     for (int i = 0; i < 8; i++) U[i] = make_double2(U[i].x + two_omega * B[i].x, U[i].y + two_omega * B[i].y);
   }
-  L::template forward<false>(x, g, U, out(0), lo, inr, live);
+  L::template forward<FULL>(x, g, U, out(0), lo, inr, live);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     T[i] = ys[LANES * i];
     if (LINEAR) T[i] = make_double2(T[i].x - two_omega * A[i].x, T[i].y - two_omega * A[i].y);
   }
-  L::template forward<false>(x, g, T, out(1), lo, inr, live);
+  L::template forward<FULL>(x, g, T, out(1), lo, inr, live);
   if (LINEAR) {
     // W: N_z = Z - W
-    L::template inverse<false>(x, g, in(9), lo, live, T);
+    L::template inverse<FULL>(x, g, in(9), lo, live, T);
 #pragma unroll
     for (int i = 0; i < 8; i++) V[i] = make_double2(V[i].x - T[i].x, V[i].y - T[i].y);
   }
-  L::template forward<false>(x, g, V, out(2), lo, inr, live);
+  L::template forward<FULL>(x, g, V, out(2), lo, inr, live);
   // rbr, rbp: A = rur rbr + rup rbp
-  L::template inverse<false>(x, g, in(6), lo, live, T);
+  L::template inverse<FULL>(x, g, in(6), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) A[i] = make_double2(A[i].x * T[i].x, A[i].y * T[i].y);
-  L::template inverse<false>(x, g, in(7), lo, live, T);
+  L::template inverse<FULL>(x, g, in(7), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) A[i] = make_double2(A[i].x + B[i].x * T[i].x, A[i].y + B[i].y * T[i].y);
   // bz: N_b = -(T / r^2 + uz bz) (+ Nbar^2 uz)
-  L::template inverse<false>(x, g, in(8), lo, live, T);
+  L::template inverse<FULL>(x, g, in(8), lo, live, T);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     const double vr = A[i].x / r2 + C[i].x * T[i].x, vi = A[i].y / r2 + C[i].y * T[i].y;
@@ -1280,7 +1280,7 @@ k_fused_products_reg(KGrid g, const double *__restrict__ rsq, const double2 *tw,
     if (LINEAR) nb = make_double2(nb.x + n2 * C[i].x, nb.y + n2 * C[i].y);
     A[i] = nb;
   }
-  L::template forward<false>(x, g, A, out(3), lo, inr, live);
+  L::template forward<FULL>(x, g, A, out(3), lo, inr, live);
 }
 
 struct Line256 {
@@ -1463,33 +1463,47 @@ bool fused_products_supported(const mlg_ctx *c) {
 
 // One wave a field or a line's fields in one wave.  Truncations past 3/8 of
 // NTH (FULL: both terms in the merge) spill in the kernels that hold all
-// fields, so they always go a wave a field: at 256 x NTH x 256, NTH = 32, 64,
-// 128 163, 335, 777 us against 295, 541, 884; 128 x 512 x 128 1019 against
-// 898.  Others do while the blocks fill the chip at most three times (one
-// block a CU): at NR = 64, NX = 32 8.1 us against 20.3 (NTH = 32, 160 blocks),
-// 14.3 against 20.4 (64, 288) and 25.2 against 28.8 (128, 544), but 33.6
-// against 28.5 at 128 x 64 x 64 (1088) and 234 against 150 at 256 x 64 x 256.
+// fields, so they go a wave a field: at 256 x NTH x 256, NTH = 32, 64, 128 163,
+// 335, 777 us against 295, 541, 884.  At NTH = 512, where a wave a field is one
+// line a block, only up to sixteen blocks a CU: 64 x 512 x 32 (2080 blocks) 129
+// us against 147, 128 x 512 x 32 (4128) 265 against 253, 128 x 512 x 64 525
+// against 468, 192 x 512 x 384 4.46 ms against 3.75.  Others do while the
+// blocks fill the chip at most three times (one block a CU): at NR = 64, NX =
+// 32 8.1 us against 20.3 (NTH = 32, 160 blocks), 14.3 against 20.4 (64, 288)
+// and 25.2 against 28.8 (128, 544), but 33.6 against 28.5 at 128 x 64 x 64
+// (1088) and 234 against 150 at 256 x 64 x 256.
 template <class L, bool LINEAR>
 static int launch_line(mlg_ctx *c, const FusedIO &io, double two_omega, double n2) {
   KGrid g = kgrid(c);
   constexpr int wl = 64 / L::LANES;
   const int wide = (g.ndimr + wl - 1) / wl * g.ndimx;
-  const bool full = g.ntchopdim > L::MMAX;
-  if (full) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_wide<L, LINEAR, true>), dim3(xcd_grid(wide)),
-                       dim3(LINEAR ? 640 : 576), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
+#define L_WIDE(FULL_)                                                                                    \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_wide<L, LINEAR, FULL_>), dim3(xcd_grid(wide)),     \
+                     dim3(LINEAR ? 640 : 576), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2)
+#define L_REG(FULL_)                                                                                     \
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_reg<L, LINEAR, FULL_>),                            \
+                     dim3(xcd_grid((g.ndimr + L::THREADS / L::LANES - 1) / (L::THREADS / L::LANES) * g.ndimx)), \
+                     dim3(L::THREADS), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2)
+  if constexpr (L::N == 512) {
+    if (g.ntchopdim > L::MMAX && wide > 16 * 256) {
+      L_REG(true);
+      MLG_CHECK_HIP(hipGetLastError());
+      return 0;
+    }
+  }
+  if (g.ntchopdim > L::MMAX) {
+    L_WIDE(true);
   } else if constexpr (L::MMAX > 0) {
     if (wide <= 3 * 256)
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_wide<L, LINEAR, false>), dim3(xcd_grid(wide)),
-                         dim3(LINEAR ? 640 : 576), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
+      L_WIDE(false);
     else if constexpr (L::N == 256)
       hipLaunchKernelGGL(k_fused_products_256<LINEAR>, dim3(xcd_grid((g.ndimr + 7) / 8 * g.ndimx)), dim3(256), 0,
                          c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
     else
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_fused_products_reg<L, LINEAR>),
-                         dim3(xcd_grid((g.ndimr + L::THREADS / L::LANES - 1) / (L::THREADS / L::LANES) * g.ndimx)),
-                         dim3(L::THREADS), 0, c->stream, g, c->d.r, c->d.tw_t, c->d.tw_h, io, two_omega, n2);
+      L_REG(false);
   }
+#undef L_WIDE
+#undef L_REG
   MLG_CHECK_HIP(hipGetLastError());
   return 0;
 }

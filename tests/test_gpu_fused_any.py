@@ -27,8 +27,9 @@ def test_right_hand_sides(nth, full):
     compare(dict(CFG1, nr=nr, nth=nth, nx=6, nrchop=nrchop, ntchop=ntc, nxchop=3))
 
 
-# more than 768 blocks of a wave a field (64, 32, .. 1 of the 15 lines of a plane each)
-@pytest.mark.parametrize("nth,nx", [(8, 800), (16, 800), (32, 800), (64, 400), (128, 200), (256, 100), (512, 54)])
+# more than 768 blocks of a wave a field (64, 32, .. 1 of the 15 lines of a plane each), more than 4096 at 512
+@pytest.mark.parametrize("nth,nx", [(8, 800), (16, 800), (32, 800), (64, 400), (128, 200), (256, 100), (512, 54),
+                                    (512, 280)])
 @pytest.mark.parametrize("full", [False, True], ids=["third", "twothirds"])
 def test_right_hand_sides_on_large_grids(nth, nx, full):
     ntc = 2 * nth // 3 if full else nth // 3
