@@ -897,10 +897,6 @@ struct ToPfp {
       pff[cap] = P.take(c->n_pff);
       if (P.ok) cap++;
     }
-    if (cap == 0) {  // the rounding of Pack's arrays: one a buffer
-      P.grow(std::min(PFF_BUFFERS, n));
-      for (; cap < (int)P.e.size(); cap++) pff[cap] = P.e[cap];
-    }
     RET(T.ready());
     for (int j0 = 0; j0 < n; j0 += cap) {
       const int nj = std::min(cap, n - j0);

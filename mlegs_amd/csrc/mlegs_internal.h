@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <unordered_set>
 #include <vector>
@@ -599,11 +600,11 @@ struct Pack {
       used.push_back(0);
     }
   }
-  double2 *take(long n, bool live = false) {
-    n = (n + 7) / 8 * 8;  // whole cache lines
+  double2 *take(long n, bool live = false) {  // n <= n_max
+    n = std::min((n + 7) / 8 * 8, T.c->n_max);  // whole cache lines
     for (size_t i = live ? lo : 0;; i++) {
       if (i == e.size()) {
-        if ((int)i >= cap || n > T.c->n_max) {
+        if ((int)i >= cap) {
           ok = false;
           return nullptr;
         }

@@ -469,8 +469,13 @@ static int sweep_build(mlg_sweep *w) {
           rc = MLG_E_HIP;
     }
   } else if (!rc) {
-    // one graph: each run's segments in order, a grouped launch after the
-    // segments before it of every run it serves
+    // one graph: each run's segments in order, and every grouped launch after
+    // the segments before it and before those after it of all runs, whether it
+    // serves them or not.  A grouped kernel node that waits for the segments of
+    // some runs only ran ahead of them on replays, unless they were the first
+    // run's: sweeps of runs with unequal numbers of products a step (two
+    // batches in the right-hand side, theta lengths without fused products)
+    // gave wrong results (also by_grid, see mlg_sweep_create)
     hipGraph_t G = nullptr;
     if (hipGraphCreate(&G, 0) != hipSuccess) rc = MLG_E_HIP;
     std::vector<hipGraphNode_t> last(w->nruns, nullptr);
@@ -491,8 +496,8 @@ static int sweep_build(mlg_sweep *w) {
       for (int l : at_pos[p]) {
         mlg_sweep::Grouped &q = w->gl[l];
         std::vector<hipGraphNode_t> deps;
-        for (int r : q.served)
-          if (last[r]) deps.push_back(last[r]);
+        for (hipGraphNode_t n : last)
+          if (n && std::find(deps.begin(), deps.end(), n) == deps.end()) deps.push_back(n);
         void *args[4] = {(void *)&q.dj, (void *)&q.db0, (void *)&q.njobs, (void *)&q.total};
         hipKernelNodeParams kp;
         std::memset(&kp, 0, sizeof(kp));
@@ -504,7 +509,7 @@ static int sweep_build(mlg_sweep *w) {
         kp.extra = nullptr;
         hipGraphNode_t node = nullptr;
         if (hipGraphAddKernelNode(&node, G, deps.data(), deps.size(), &kp) != hipSuccess) rc = MLG_E_HIP;
-        for (int r : q.served) last[r] = node;
+        std::fill(last.begin(), last.end(), node);
         nodes++;
         if (rc) break;
       }

@@ -104,6 +104,18 @@ def test_sweep_equals_runs_alone(kw):
         assert info["grouped_positions"] == 0 and info["grouped_jobs"] == 0
 
 
+@pytest.mark.parametrize("kw", [dict(grouped=True, shape=0), dict(grouped=True, shape=0, streams=True)],
+                         ids=["grouped", "grouped_streams"])
+def test_runs_with_unequal_numbers_of_products(kw):
+    """A step has one backward product, two where the truncation leaves no room
+    for one batch, and ten at theta lengths without fused products."""
+    wide = dict(CFG1, nr=24, nth=8, nx=8, nrchop=18, ntchop=8, nxchop=4)
+    apart = dict(CFG1, nr=24, nth=67, nx=8, nrchop=16, ntchop=6, nxchop=3)
+    for runs, npos in (([SMALL_RUNS[0], wide, SMALL_RUNS[1]], 2), ([wide, wide], 2), ([apart, SMALL_RUNS[0], wide], 10)):
+        info = check_sweep(runs, [4, 3], **kw)
+        assert info["grouped_positions"] == npos
+
+
 def test_sweep_rerecords_after_buffer_swap():
     """A transform of a run's field between calls moves its buffers: the next
     call records the sweep again and still matches the run stepped alone."""
