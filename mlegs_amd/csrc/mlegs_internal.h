@@ -583,32 +583,33 @@ struct Temps {
 // `lo` buffers are taken at once; arrays that are `live` do not go there.
 // ok is false once an array had no room.
 struct Pack {
+  static constexpr int MAX = 8;
   Temps &T;
   const int cap, lo;
   bool ok = true;
-  std::vector<double2 *> e;  // the buffers
-  std::vector<long> used;
-  Pack(Temps &t, int cap_, int lo_ = 0) : T(t), cap(cap_), lo(lo_) { grow(lo); }
+  int n_e = 0;
+  double2 *e[MAX];  // the buffers
+  long used[MAX];
+  Pack(Temps &t, int cap_, int lo_ = 0) : T(t), cap(cap_ < MAX ? cap_ : MAX), lo(lo_) { grow(lo); }
   void give(double2 *buffer) {  // one of the caller's
-    e.push_back(buffer);
-    used.push_back(0);
+    e[n_e] = buffer;
+    used[n_e++] = 0;
   }
   void grow(int n) {
-    while ((int)e.size() < n) {
+    while (n_e < n) {
       mlg_field *f = T.buffer();
-      e.push_back(f ? f->e : nullptr);
-      used.push_back(0);
+      give(f ? f->e : nullptr);
     }
   }
   double2 *take(long n, bool live = false) {  // n <= n_max
     n = std::min((n + 7) / 8 * 8, T.c->n_max);  // whole cache lines
-    for (size_t i = live ? lo : 0;; i++) {
-      if (i == e.size()) {
-        if ((int)i >= cap) {
+    for (int i = live ? lo : 0;; i++) {
+      if (i == n_e) {
+        if (i >= cap) {
           ok = false;
           return nullptr;
         }
-        grow((int)i + 1);
+        grow(i + 1);
       }
       if (!e[i]) return nullptr;  // T.ready() reports it
       if (used[i] + n > T.c->n_max) continue;
